@@ -115,6 +115,10 @@ struct llfem_ctx {
   void* h_stage[2] = {nullptr, nullptr};
   size_t stage_bytes = 0;
   hipEvent_t stage_ev[2] = {nullptr, nullptr};
+  // pinned word a running solve sets when it is done, and the events of its
+  // two queued batches
+  double* h_poll = nullptr;
+  hipEvent_t poll_ev[2] = {nullptr, nullptr};
 };
 
 struct llfem_mesh {

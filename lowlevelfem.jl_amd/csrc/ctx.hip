@@ -202,6 +202,12 @@ int llfem_ctx_create(int device, size_t hbm_budget_bytes, llfem_ctx** out) {
     llfem_ctx_destroy(c);
     return fail(LLFEM_EHIP, "hipEventCreate failed");
   }
+  if (hipHostMalloc((void**)&c->h_poll, 64, hipHostMallocDefault) != hipSuccess ||
+      hipEventCreateWithFlags(&c->poll_ev[0], hipEventDisableTiming) != hipSuccess ||
+      hipEventCreateWithFlags(&c->poll_ev[1], hipEventDisableTiming) != hipSuccess) {
+    llfem_ctx_destroy(c);
+    return fail(LLFEM_EHIP, "llfem_ctx_create: pinned memory or events failed");
+  }
   *out = c;
   return LLFEM_OK;
 }
@@ -224,6 +230,9 @@ int llfem_ctx_destroy(llfem_ctx* ctx) {
     if (ctx->join_ev[k]) (void)hipEventDestroy(ctx->join_ev[k]);
   }
   if (ctx->fork_ev) (void)hipEventDestroy(ctx->fork_ev);
+  if (ctx->h_poll) (void)hipHostFree(ctx->h_poll);
+  for (auto& e : ctx->poll_ev)
+    if (e) (void)hipEventDestroy(e);
   for (int b = 0; b < 2; ++b) {
     if (ctx->h_stage[b]) (void)hipHostFree(ctx->h_stage[b]);
     if (ctx->stage_ev[b]) (void)hipEventDestroy(ctx->stage_ev[b]);

@@ -26,73 +26,185 @@ namespace llfem {
 namespace {
 
 constexpr int kBS = 256;
-constexpr int kG = 8;   // lanes per node row in the SpMV
+constexpr int kWaves = kBS / 64;
+constexpr int kG = 8;   // lanes per row the workspace's partial count is sized for (solve_ws_bytes)
+// Partials a kernel sums by itself in every block: up to this many cost each
+// block about a microsecond out of L2, less than a reduction launch of its
+// own.  More of them (large systems) go through k_fold first.
+constexpr int64_t kFoldMax = 2048;
+constexpr unsigned kFoldBlocks = 64;
+constexpr int64_t kMaxPasses = 8;
+constexpr int64_t kFuseMax = 30000;   // DoFs up to which pcg forms the direction inside the SpMV
 
-enum { S_RHO = 0, S_ALPHA, S_BETA, S_RR, S_PQ, S_TOL2, S_DONE, S_ITER, S_NS };
+// S_RHO0 / S_RHO1: r.z of even / odd iterations (the p-update reads one and
+// writes the other, so no block sees the new value in place of the old).
+enum { S_RHO0 = 0, S_RHO1, S_RR, S_TOL2, S_DONE, S_ITER, S_NS = 8 };
 
+// Sum over the block in a fixed order: a butterfly per wavefront, then the
+// wavefronts' sums in order.  One barrier before the result, one after it
+// (sh may be reused at once).
 __device__ __forceinline__ double block_sum(double v, double* sh) {
-  const int t = threadIdx.x;
-  sh[t] = v;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
   __syncthreads();
-  for (int o = blockDim.x / 2; o > 0; o >>= 1) {
-    if (t < o) sh[t] += sh[t + o];
-    __syncthreads();
-  }
   double r = sh[0];
+#pragma unroll
+  for (int w = 1; w < kWaves; ++w) r += sh[w];
   __syncthreads();
   return r;
 }
 
-// y = mask(K x); optional partial of dot(x, y).  Node row j uses kG lanes.
-template <typename MT, typename VT>
-__global__ __launch_bounds__(kBS) void k_spmv(int64_t N, const int64_t* __restrict__ adj_ptr,
-                                             const int32_t* __restrict__ adj, const MT* __restrict__ val,
-                                             const VT* __restrict__ x, const uint8_t* __restrict__ fixed,
-                                             VT* __restrict__ y, double* __restrict__ part,
-                                             const double* __restrict__ scal) {
-  __shared__ double sh[kBS];
-  if (scal && scal[S_DONE] != 0.0) return;
-  const int64_t gt = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t j = gt / kG;
-  const int l = (int)(gt % kG);
-  VT a0 = 0, a1 = 0, a2 = 0;
-  if (j < N) {
-    const int64_t p0 = adj_ptr[j];
-    const int R = (int)(adj_ptr[j + 1] - p0);
-    const MT* P = val + 9 * p0;
-    for (int s = l; s < R; s += kG) {
-      const int64_t i = adj[p0 + s];
-      const VT x0 = x[3 * i], x1 = x[3 * i + 1], x2 = x[3 * i + 2];
-      a0 += (VT)P[3 * s] * x0 + (VT)P[3 * s + 1] * x1 + (VT)P[3 * s + 2] * x2;
-      a1 += (VT)P[3 * R + 3 * s] * x0 + (VT)P[3 * R + 3 * s + 1] * x1 + (VT)P[3 * R + 3 * s + 2] * x2;
-      a2 += (VT)P[6 * R + 3 * s] * x0 + (VT)P[6 * R + 3 * s + 1] * x1 + (VT)P[6 * R + 3 * s + 2] * x2;
+__device__ __forceinline__ double2 block_sum2(double a, double b, double* sh) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    a += __shfl_xor(a, o, 64);
+    b += __shfl_xor(b, o, 64);
+  }
+  if ((threadIdx.x & 63) == 0) {
+    sh[threadIdx.x >> 6] = a;
+    sh[kWaves + (threadIdx.x >> 6)] = b;
+  }
+  __syncthreads();
+  double ra = sh[0], rb = sh[kWaves];
+#pragma unroll
+  for (int w = 1; w < kWaves; ++w) {
+    ra += sh[w];
+    rb += sh[kWaves + w];
+  }
+  __syncthreads();
+  return make_double2(ra, rb);
+}
+
+// Sum of n partials, or of n pairs of them; the same order in every block.
+__device__ __forceinline__ double sum_partials(int64_t n, const double* __restrict__ part, double* sh) {
+  double s = 0.0;
+  for (int64_t i = threadIdx.x; i < n; i += kBS) s += part[i];
+  return block_sum(s, sh);
+}
+__device__ __forceinline__ double2 sum_pairs(int64_t n, const double* __restrict__ part, double* sh) {
+  double a = 0.0, b = 0.0;
+  for (int64_t i = threadIdx.x; i < n; i += kBS) {
+    const double2 v = reinterpret_cast<const double2*>(part)[i];
+    a += v.x;
+    b += v.y;
+  }
+  return block_sum2(a, b, sh);
+}
+
+// Blocks are dealt round-robin to the 8 XCDs; neighbouring rows share most of
+// the x entries they read, so give each XCD a contiguous run of blocks (the
+// last gridDim % 8 blocks keep their place).  FP64 panels of 46,575 nodes:
+// 23.1 -> 20.8 us; at 2.1 M nodes the same.
+__device__ __forceinline__ int64_t xcd_block() {
+  const unsigned nb = gridDim.x & ~7u, b = blockIdx.x;
+  return b < nb ? (int64_t)(b & 7u) * (nb >> 3) + (b >> 3) : (int64_t)b;
+}
+
+// What an SpMV multiplies: a vector as it stands, ...
+template <typename VT>
+struct Plain {
+  const VT* __restrict__ x;
+  __device__ __forceinline__ bool begin(double*) { return true; }
+  __device__ __forceinline__ VT at(int64_t i) const { return x[i]; }
+  __device__ __forceinline__ void keep(int64_t, VT) const {}
+};
+
+// ... or the CG direction p = z + beta p_old, formed while it is gathered: the
+// launch that would write it first, and its pass over z and p, are not needed.
+// Every block sums the previous update's partials (r.r, r.z) itself; block 0
+// keeps the scalars, tests convergence and tells the host.  Each row's owner
+// writes its part of p to a second array (neighbours still read p_old).
+template <typename VT>
+struct Direction {
+  const VT* __restrict__ z;
+  const VT* __restrict__ pold;
+  VT* __restrict__ pnew;
+  double* scal;
+  const double* part;   // np pairs (r.r, r.z) of the update before
+  int64_t np, it, maxiter;
+  volatile double* done_host;
+  VT beta;
+  __device__ __forceinline__ bool begin(double* sh) {
+    beta = 0;
+    if (it == 0) return true;   // p = z, rho from k_init_scal
+    const double2 s = sum_pairs(np, part, sh);
+    beta = (VT)(s.y / scal[S_RHO0 + (int)((it - 1) & 1)]);
+    const bool done = s.x <= scal[S_TOL2] || it >= maxiter;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      scal[S_RHO0 + (int)(it & 1)] = s.y;
+      scal[S_RR] = s.x;
+      scal[S_ITER] = (double)it;
+      if (done) {
+        scal[S_DONE] = 1.0;
+        *done_host = 1.0;
+      }
     }
+    return !done;
   }
-#pragma unroll
-  for (int o = kG / 2; o > 0; o >>= 1) {
-    a0 += __shfl_xor(a0, o, kG);
-    a1 += __shfl_xor(a1, o, kG);
-    a2 += __shfl_xor(a2, o, kG);
-  }
+  __device__ __forceinline__ VT at(int64_t i) const { return it == 0 ? z[i] : z[i] + beta * pold[i]; }
+  __device__ __forceinline__ void keep(int64_t i, VT v) const { pnew[i] = v; }
+};
+
+// y = mask(K x); optional partial of dot(x, y).  Node row j uses G lanes, one
+// 3x3 block per lane and step.  Bound: HBM for large K, a chain of dependent
+// loads (row pointer -> column -> x) for small ones; with G covering a whole
+// row the chain is walked once.  FP64, tet10 panels (28 blocks a row): G = 8
+// 1013 us, 32 912 us at 2.1 M nodes (4.5 -> 5.0 TB/s of 76 bytes a block);
+// 23.0 -> 17.5 us at 46,575 nodes.  A block walks `passes` row groups, so
+// that the systems of up to a few 100,000 DoFs leave no more partials than
+// the next kernel's blocks sum by themselves.
+template <typename MT, typename VT, int G, typename X>
+__global__ __launch_bounds__(kBS) void k_spmv(int64_t N, int passes, const int64_t* __restrict__ adj_ptr,
+                                             const int32_t* __restrict__ adj, const MT* __restrict__ val, X xs,
+                                             const uint8_t* __restrict__ fixed, VT* __restrict__ y,
+                                             double* __restrict__ part, const double* __restrict__ scal) {
+  __shared__ double sh[2 * kWaves];
+  if (scal && scal[S_DONE] != 0.0) return;
+  if (!xs.begin(sh)) return;
+  const int64_t lb = xcd_block();
+  const int l = (int)(threadIdx.x % G);
   double d = 0.0;
-  if (j < N && l == 0) {
-    const VT r[3] = {a0, a1, a2};
+  for (int ps = 0; ps < passes; ++ps) {
+    const int64_t j = (lb * passes + ps) * (kBS / G) + threadIdx.x / G;
+    VT a0 = 0, a1 = 0, a2 = 0;
+    if (j < N) {
+      const int64_t p0 = adj_ptr[j];
+      const int R = (int)(adj_ptr[j + 1] - p0);
+      const MT* P = val + 9 * p0;
+      for (int s = l; s < R; s += G) {
+        const int64_t i = adj[p0 + s];
+        const VT x0 = xs.at(3 * i), x1 = xs.at(3 * i + 1), x2 = xs.at(3 * i + 2);
+        a0 += (VT)P[3 * s] * x0 + (VT)P[3 * s + 1] * x1 + (VT)P[3 * s + 2] * x2;
+        a1 += (VT)P[3 * R + 3 * s] * x0 + (VT)P[3 * R + 3 * s + 1] * x1 + (VT)P[3 * R + 3 * s + 2] * x2;
+        a2 += (VT)P[6 * R + 3 * s] * x0 + (VT)P[6 * R + 3 * s + 1] * x1 + (VT)P[6 * R + 3 * s + 2] * x2;
+      }
+    }
 #pragma unroll
-    for (int c = 0; c < 3; ++c) {
-      const VT v = (fixed && fixed[3 * j + c]) ? (VT)0 : r[c];
-      y[3 * j + c] = v;
-      d += (double)x[3 * j + c] * (double)v;
+    for (int o = G / 2; o > 0; o >>= 1) {
+      a0 += __shfl_xor(a0, o, G);
+      a1 += __shfl_xor(a1, o, G);
+      a2 += __shfl_xor(a2, o, G);
+    }
+    if (j < N && l < 3) {   // lane c writes component c
+      const VT r = l == 0 ? a0 : l == 1 ? a1 : a2;
+      const int64_t i = 3 * j + l;
+      const VT v = (fixed && fixed[i]) ? (VT)0 : r;
+      const VT xv = xs.at(i);
+      y[i] = v;
+      xs.keep(i, xv);
+      d += (double)xv * (double)v;
     }
   }
   if (part) {
     const double s = block_sum(d, sh);
-    if (threadIdx.x == 0) part[blockIdx.x] = s;
+    if (threadIdx.x == 0) part[lb] = s;
   }
 }
 
 // Fixed-order final reduction of `n` partial rows of width w into out[0..w).
 __global__ void k_reduce(int64_t n, int w, const double* __restrict__ part, double* __restrict__ out) {
-  __shared__ double sh[kBS];
+  __shared__ double sh[kWaves];
   for (int c = 0; c < w; ++c) {
     double s = 0.0;
     for (int64_t i = threadIdx.x; i < n; i += blockDim.x) s += part[i * w + c];
@@ -101,23 +213,31 @@ __global__ void k_reduce(int64_t n, int w, const double* __restrict__ part, doub
   }
 }
 
-// alpha = rho / (p.q)
-__global__ void k_alpha(double* scal, const double* red) {
+// n partials -> gridDim.x partials, each the sum of one contiguous run.
+__global__ __launch_bounds__(kBS) void k_fold(int64_t n, const double* __restrict__ part, double* __restrict__ out,
+                                             const double* __restrict__ scal) {
+  __shared__ double sh[kWaves];
   if (scal[S_DONE] != 0.0) return;
-  scal[S_PQ] = red[0];
-  scal[S_ALPHA] = scal[S_RHO] / red[0];
+  const int64_t per = (n + gridDim.x - 1) / gridDim.x, i0 = blockIdx.x * per, i1 = min(n, i0 + per);
+  double s = 0.0;
+  for (int64_t i = i0 + threadIdx.x; i < i1; i += kBS) s += part[i];
+  s = block_sum(s, sh);
+  if (threadIdx.x == 0) out[blockIdx.x] = s;
 }
 
-// x += alpha p; r -= alpha q; z = dinv r; partials (r.r, r.z)
+// alpha = rho / p.q, then x += alpha p; r -= alpha q; z = dinv r; partials
+// (r.r, r.z).  Every block sums the np partials of p.q itself (same order,
+// same alpha), which takes the reduction and scalar launches between the
+// SpMV and this kernel out of the iteration.
 template <typename VT>
-__global__ __launch_bounds__(kBS) void k_update(int64_t n, const double* __restrict__ scal,
-                                               VT* __restrict__ x, VT* __restrict__ r,
-                                               const VT* __restrict__ p, const VT* __restrict__ q,
-                                               const VT* __restrict__ dinv, VT* __restrict__ z,
-                                               double* __restrict__ part) {
-  __shared__ double sh[kBS];
+__global__ __launch_bounds__(kBS) void k_update(int64_t n, const double* __restrict__ scal, int par, int64_t np,
+                                               const double* __restrict__ pq, VT* __restrict__ x,
+                                               VT* __restrict__ r, const VT* __restrict__ p,
+                                               const VT* __restrict__ q, const VT* __restrict__ dinv,
+                                               VT* __restrict__ z, double* __restrict__ part) {
+  __shared__ double sh[2 * kWaves];
   if (scal[S_DONE] != 0.0) return;
-  const VT alpha = (VT)scal[S_ALPHA];
+  const VT alpha = (VT)(scal[S_RHO0 + par] / sum_partials(np, pq, sh));
   double rr = 0.0, rz = 0.0;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * blockDim.x) {
@@ -129,64 +249,74 @@ __global__ __launch_bounds__(kBS) void k_update(int64_t n, const double* __restr
     rr += (double)ri * (double)ri;
     rz += (double)ri * (double)zi;
   }
-  rr = block_sum(rr, sh);
-  rz = block_sum(rz, sh);
-  if (threadIdx.x == 0) {
-    part[2 * blockIdx.x] = rr;
-    part[2 * blockIdx.x + 1] = rz;
-  }
+  const double2 s = block_sum2(rr, rz, sh);
+  if (threadIdx.x == 0) reinterpret_cast<double2*>(part)[blockIdx.x] = s;
 }
 
-// beta = rz / rho; rho = rz; convergence test on ||r||
-__global__ void k_beta(double* scal, const double* red, int64_t maxiter) {
-  if (scal[S_DONE] != 0.0) return;
-  scal[S_RR] = red[0];
-  scal[S_BETA] = red[1] / scal[S_RHO];
-  scal[S_RHO] = red[1];
-  scal[S_ITER] += 1.0;
-  if (red[0] <= scal[S_TOL2] || scal[S_ITER] >= (double)maxiter) scal[S_DONE] = 1.0;
-}
-
+// beta = rz / rho, p = z + beta p; block 0 keeps the scalars, tests
+// convergence on ||r|| and tells the host (done_host: pinned memory).  A block
+// that starts after block 0 set S_DONE leaves its part of p as it was: no
+// kernel of this solve reads p any more then.
 template <typename VT>
-__global__ void k_pupd(int64_t n, const double* __restrict__ scal, const VT* __restrict__ z,
-                       VT* __restrict__ p) {
+__global__ __launch_bounds__(kBS) void k_pupd(int64_t n, double* __restrict__ scal, int64_t it, int64_t np,
+                                             const double* __restrict__ part, int64_t maxiter,
+                                             const VT* __restrict__ z, VT* __restrict__ p,
+                                             volatile double* done_host) {
+  __shared__ double sh[2 * kWaves];
   if (scal[S_DONE] != 0.0) return;
-  const VT beta = (VT)scal[S_BETA];
+  const double2 s = sum_pairs(np, part, sh);   // r.r, r.z
+  const double rho = scal[S_RHO0 + (int)(it & 1)];
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    scal[S_RHO0 + (int)(~it & 1)] = s.y;
+    scal[S_RR] = s.x;
+    scal[S_ITER] = (double)(it + 1);
+    if (s.x <= scal[S_TOL2] || it + 1 >= maxiter) {
+      scal[S_DONE] = 1.0;
+      *done_host = 1.0;
+    }
+  }
+  const VT beta = (VT)(s.y / rho);
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * blockDim.x)
     p[i] = z[i] + beta * p[i];
 }
 
-// init: x = 0; z = dinv r; p = z; partials (r.r, r.z)
+// init: x = 0; r = b; z = dinv r; p = z; partials (r.r, r.z)
 template <typename VT>
-__global__ __launch_bounds__(kBS) void k_init(int64_t n, VT* __restrict__ x, const VT* __restrict__ r,
-                                             const VT* __restrict__ dinv, VT* __restrict__ z,
+__global__ __launch_bounds__(kBS) void k_init(int64_t n, VT* __restrict__ x, const VT* __restrict__ b,
+                                             VT* __restrict__ r, const VT* __restrict__ dinv, VT* __restrict__ z,
                                              VT* __restrict__ p, double* __restrict__ part) {
-  __shared__ double sh[kBS];
+  __shared__ double sh[2 * kWaves];
   double rr = 0.0, rz = 0.0;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * blockDim.x) {
     x[i] = 0;
-    const VT zi = dinv[i] * r[i];
+    const VT ri = b[i];
+    r[i] = ri;
+    const VT zi = dinv[i] * ri;
     z[i] = zi;
     p[i] = zi;
-    rr += (double)r[i] * (double)r[i];
-    rz += (double)r[i] * (double)zi;
+    rr += (double)ri * (double)ri;
+    rz += (double)ri * (double)zi;
   }
-  rr = block_sum(rr, sh);
-  rz = block_sum(rz, sh);
-  if (threadIdx.x == 0) {
-    part[2 * blockIdx.x] = rr;
-    part[2 * blockIdx.x + 1] = rz;
-  }
+  const double2 s = block_sum2(rr, rz, sh);
+  if (threadIdx.x == 0) reinterpret_cast<double2*>(part)[blockIdx.x] = s;
 }
 
-__global__ void k_init_scal(double* scal, const double* red, double rtol) {
-  scal[S_RR] = red[0];
-  scal[S_RHO] = red[1];
-  scal[S_TOL2] = rtol * rtol * red[0];
+// scalars of the first iteration from the np partials of k_init (one block)
+__global__ __launch_bounds__(kBS) void k_init_scal(int64_t np, const double* __restrict__ part, double* scal,
+                                                   double rtol, volatile double* done_host) {
+  __shared__ double sh[2 * kWaves];
+  const double2 s = sum_pairs(np, part, sh);
+  if (threadIdx.x != 0) return;
+  const double rr = s.x;
+  scal[S_RR] = rr;
+  scal[S_RHO0] = s.y;
+  scal[S_TOL2] = rtol * rtol * rr;
   scal[S_ITER] = 0.0;
-  scal[S_DONE] = (red[0] <= scal[S_TOL2] || red[0] == 0.0) ? 1.0 : 0.0;
+  const double done = (rr <= scal[S_TOL2] || rr == 0.0) ? 1.0 : 0.0;
+  scal[S_DONE] = done;
+  *done_host = done;
 }
 
 // diag / Jacobi inverse from the panels; 0 on fixed DoFs
@@ -205,16 +335,16 @@ __global__ void k_dinv(int64_t N, const int64_t* __restrict__ adj_ptr, const int
   }
 }
 
-// r = mask(f - y); for the FP64 residual of the refinement loop
+// r = mask(f - y) (y NULL: mask(f); r NULL: only the norm); partial of r.r
 __global__ void k_resid(int64_t n, const double* __restrict__ f, const double* __restrict__ y,
                         const uint8_t* __restrict__ fixed, double* __restrict__ r,
                         double* __restrict__ part) {
-  __shared__ double sh[kBS];
+  __shared__ double sh[kWaves];
   double rr = 0.0;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * blockDim.x) {
-    const double v = fixed[i] ? 0.0 : f[i] - y[i];
-    r[i] = v;
+    const double v = fixed[i] ? 0.0 : (y ? f[i] - y[i] : f[i]);
+    if (r) r[i] = v;
     rr += v * v;
   }
   rr = block_sum(rr, sh);
@@ -252,60 +382,89 @@ __global__ void k_axpy(int64_t n, double s, const double* __restrict__ d, double
     x[i] += s * d[i];
 }
 
-// Scalar CSC operator (caller-supplied symmetric matrix, used as CSR of K^T).
-template <typename MT, typename VT>
-__global__ __launch_bounds__(kBS) void k_spmv_csc(int64_t n, const int64_t* __restrict__ colptr,
+// Scalar CSC operator (caller-supplied symmetric matrix, used as CSR of K^T),
+// G lanes per row.  A hexahedral or tetrahedral K has 60-90 entries a row:
+// 32 lanes walk it in three steps and give a small system (5,400 rows: 675
+// blocks instead of 169) a block on every CU.
+template <typename MT, typename VT, int G, typename X>
+__global__ __launch_bounds__(kBS) void k_spmv_csc(int64_t n, int passes, const int64_t* __restrict__ colptr,
                                                  const int32_t* __restrict__ rowval,
-                                                 const MT* __restrict__ val, const VT* __restrict__ x,
+                                                 const MT* __restrict__ val, X xs,
                                                  const uint8_t* __restrict__ fixed, VT* __restrict__ y,
                                                  double* __restrict__ part,
                                                  const double* __restrict__ scal) {
-  __shared__ double sh[kBS];
+  __shared__ double sh[2 * kWaves];
   if (scal && scal[S_DONE] != 0.0) return;
-  const int64_t gt = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t j = gt / kG;
-  const int l = (int)(gt % kG);
-  VT acc = 0;
-  if (j < n)
-    for (int64_t p = colptr[j] + l; p < colptr[j + 1]; p += kG) acc += (VT)val[p] * x[rowval[p]];
-#pragma unroll
-  for (int o = kG / 2; o > 0; o >>= 1) acc += __shfl_xor(acc, o, kG);
+  if (!xs.begin(sh)) return;
+  const int64_t lb = xcd_block();
+  const int l = (int)(threadIdx.x % G);
   double d = 0.0;
-  if (j < n && l == 0) {
-    const VT v = (fixed && fixed[j]) ? (VT)0 : acc;
-    y[j] = v;
-    d = (double)x[j] * (double)v;
+  for (int ps = 0; ps < passes; ++ps) {
+    const int64_t j = (lb * passes + ps) * (kBS / G) + threadIdx.x / G;
+    VT acc = 0;
+    if (j < n) {
+      const int64_t p1 = colptr[j + 1];
+#pragma unroll 4
+      for (int64_t p = colptr[j] + l; p < p1; p += G) acc += (VT)val[p] * xs.at(rowval[p]);
+    }
+#pragma unroll
+    for (int o = G / 2; o > 0; o >>= 1) acc += __shfl_xor(acc, o, G);
+    if (j < n && l == 0) {
+      const VT v = (fixed && fixed[j]) ? (VT)0 : acc;
+      const VT xv = xs.at(j);
+      y[j] = v;
+      xs.keep(j, xv);
+      d += (double)xv * (double)v;
+    }
   }
   if (part) {
     const double s = block_sum(d, sh);
-    if (threadIdx.x == 0) part[blockIdx.x] = s;
+    if (threadIdx.x == 0) part[lb] = s;
   }
 }
 
+// Jacobi inverse of a CSC operator, kG lanes per column; of several stored
+// diagonal entries the last one counts.
 template <typename VT>
-__global__ void k_dinv_csc(int64_t n, const int64_t* __restrict__ colptr, const int32_t* __restrict__ rowval,
-                           const double* __restrict__ val, const uint8_t* __restrict__ fixed,
-                           VT* __restrict__ dinv) {
-  int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+__global__ __launch_bounds__(kBS) void k_dinv_csc(int64_t n, const int64_t* __restrict__ colptr,
+                                                  const int32_t* __restrict__ rowval, const double* __restrict__ val,
+                                                  const uint8_t* __restrict__ fixed, VT* __restrict__ dinv) {
+  const int64_t j = ((int64_t)blockIdx.x * kBS + threadIdx.x) / kG;
   if (j >= n) return;
-  double dv = 0.0;
-  for (int64_t p = colptr[j]; p < colptr[j + 1]; ++p)
-    if (rowval[p] == j) dv = val[p];
+  const int64_t p1 = colptr[j + 1];
+  int64_t at = -1;
+  for (int64_t p = colptr[j] + threadIdx.x % kG; p < p1; p += kG)
+    if (rowval[p] == j) at = p;
+#pragma unroll
+  for (int o = kG / 2; o > 0; o >>= 1) at = max(at, (int64_t)__shfl_xor((long long)at, o, kG));
+  if (threadIdx.x % kG != 0) return;
+  const double dv = at >= 0 ? val[at] : 0.0;
   dinv[j] = (fixed[j] || dv == 0.0) ? (VT)0 : (VT)(1.0 / dv);
 }
 
-// Operator views.
+// Operator views.  Lanes per row by the average row: 32 from 20 blocks (48
+// entries) on, 16 from 9 blocks (16 entries), else kG.
+inline unsigned row_blocks(int64_t rows, int lanes) { return (unsigned)((rows * lanes + kBS - 1) / kBS); }
+inline int panel_lanes(int64_t N, int64_t nadj) { return nadj >= 20 * N ? 32 : nadj >= 9 * N ? 16 : kG; }
+inline int csc_lanes(int64_t n, int64_t nnz) { return nnz >= 48 * n ? 32 : nnz >= 16 * n ? 16 : kG; }
+
 struct PanelOp {
   int64_t N;
   const int64_t* adj_ptr;
   const int32_t* adj;
   const int32_t* dslot;
+  int lanes;
   int64_t ndof() const { return 3 * N; }
-  unsigned grid() const { return (unsigned)((N * kG + kBS - 1) / kBS); }
-  template <typename MT, typename VT>
-  void spmv(hipStream_t st, const MT* val, const VT* x, const uint8_t* fixed, VT* y, double* part,
-            const double* scal) const {
-    k_spmv<MT, VT><<<grid(), kBS, 0, st>>>(N, adj_ptr, adj, val, x, fixed, y, part, scal);
+  int64_t rows() const { return N; }
+  template <typename MT, typename VT, typename X>
+  void spmv(hipStream_t st, unsigned grid, int passes, const MT* val, const X& x, const uint8_t* fixed, VT* y,
+            double* part, const double* scal) const {
+    if (lanes == 32)
+      k_spmv<MT, VT, 32, X><<<grid, kBS, 0, st>>>(N, passes, adj_ptr, adj, val, x, fixed, y, part, scal);
+    else if (lanes == 16)
+      k_spmv<MT, VT, 16, X><<<grid, kBS, 0, st>>>(N, passes, adj_ptr, adj, val, x, fixed, y, part, scal);
+    else
+      k_spmv<MT, VT, kG, X><<<grid, kBS, 0, st>>>(N, passes, adj_ptr, adj, val, x, fixed, y, part, scal);
   }
   template <typename VT>
   void dinv(hipStream_t st, const double* val, const uint8_t* fixed, VT* d) const {
@@ -317,18 +476,31 @@ struct CscOp {
   int64_t n;
   const int64_t* colptr;
   const int32_t* rowval;
+  int lanes;
   int64_t ndof() const { return n; }
-  unsigned grid() const { return (unsigned)((n * kG + kBS - 1) / kBS); }
-  template <typename MT, typename VT>
-  void spmv(hipStream_t st, const MT* val, const VT* x, const uint8_t* fixed, VT* y, double* part,
-            const double* scal) const {
-    k_spmv_csc<MT, VT><<<grid(), kBS, 0, st>>>(n, colptr, rowval, val, x, fixed, y, part, scal);
+  int64_t rows() const { return n; }
+  template <typename MT, typename VT, typename X>
+  void spmv(hipStream_t st, unsigned grid, int passes, const MT* val, const X& x, const uint8_t* fixed, VT* y,
+            double* part, const double* scal) const {
+    if (lanes == 32)
+      k_spmv_csc<MT, VT, 32, X><<<grid, kBS, 0, st>>>(n, passes, colptr, rowval, val, x, fixed, y, part, scal);
+    else if (lanes == 16)
+      k_spmv_csc<MT, VT, 16, X><<<grid, kBS, 0, st>>>(n, passes, colptr, rowval, val, x, fixed, y, part, scal);
+    else
+      k_spmv_csc<MT, VT, kG, X><<<grid, kBS, 0, st>>>(n, passes, colptr, rowval, val, x, fixed, y, part, scal);
   }
   template <typename VT>
   void dinv(hipStream_t st, const double* val, const uint8_t* fixed, VT* d) const {
-    k_dinv_csc<VT><<<(unsigned)((n + 255) / 256), 256, 0, st>>>(n, colptr, rowval, val, fixed, d);
+    k_dinv_csc<VT><<<row_blocks(n, kG), kBS, 0, st>>>(n, colptr, rowval, val, fixed, d);
   }
 };
+
+// y = mask(K x) outside the iteration
+template <typename Op>
+void apply(hipStream_t st, const Op& K, const double* val, const double* x, const uint8_t* fixed, double* y) {
+  K.template spmv<double, double>(st, row_blocks(K.rows(), K.lanes), 1, val, Plain<double>{x}, fixed, y, nullptr,
+                                  nullptr);
+}
 
 inline unsigned vgrid(int64_t n, llfem_ctx* ctx) {
   int64_t g = (n + kBS - 1) / kBS;
@@ -336,50 +508,93 @@ inline unsigned vgrid(int64_t n, llfem_ctx* ctx) {
   return (unsigned)std::max<int64_t>(1, std::min<int64_t>(g, cap));
 }
 
+// What the host needs after a solve, in one go: the recursion's iterations,
+// r.r and tolerance, and up to two sums of n partials (NULL: 0).
+__global__ __launch_bounds__(kBS) void k_report(int64_t n, const double* __restrict__ part1,
+                                                const double* __restrict__ part2, const double* __restrict__ scal,
+                                                double* out) {
+  __shared__ double sh[kWaves];
+  const double s1 = part1 ? sum_partials(n, part1, sh) : 0.0;
+  const double s2 = part2 ? sum_partials(n, part2, sh) : 0.0;
+  if (threadIdx.x != 0) return;
+  out[0] = scal[S_ITER];
+  out[1] = scal[S_RR];
+  out[2] = scal[S_TOL2];
+  out[3] = s1;
+  out[4] = s2;
+}
+
 struct Scratch {   // partial sums + scalars
-  double* part;
+  double* part;    // of the vector kernels
+  double* spart;   // of the SpMV (ndof doubles: at most ndof / 8 blocks, then kFoldBlocks sums of them)
   double* red;
   double* scal;
 };
 
-// Jacobi-PCG (IterativeSolvers.cg semantics, x0 = 0) on vectors of type VT.
+// Jacobi-PCG (IterativeSolvers.cg semantics, x0 = 0) on vectors of type VT; b
+// is overwritten (it is the second direction array once r holds it).
+// The scalars stay on the device and each kernel sums the partials it needs,
+// so an iteration is two launches -- SpMV of the direction formed on the fly,
+// update -- up to kFuseMax DoFs, and three above, where gathering two vectors
+// costs the SpMV more than the p-update's own launch and pass.  Whole solves,
+// three / two launches: panels of 5,400 DoFs 2.18 / 1.85 ms, 28,611 4.50 /
+// 4.19, 139,725 33.3 / 38.1; CSC 5,400 2.10 / 1.85, 28,611 5.10 / 4.98, 35,547
+// 12.3 / 13.8.  With seven launches an iteration (separate reductions and
+// scalars, a host wait every 16) it was 50 ms at 139,725 DoFs (panels) and
+// 4.8 ms at 5,400 (CSC).
+// The host keeps two batches queued and looks at the flag after the older one,
+// so the device never waits for it.
 template <typename Op, typename MT, typename VT>
-int pcg(llfem_ctx* ctx, const Op& K, const MT* val, const uint8_t* fixed, const VT* dinv, const VT* b,
-        VT* x, VT* r, VT* z, VT* p, VT* q, const Scratch& S, double rtol, int64_t maxiter,
-        int64_t* iters, double* res_rel) {
+int pcg(llfem_ctx* ctx, const Op& K, const MT* val, const uint8_t* fixed, const VT* dinv, VT* b,
+        VT* x, VT* r, VT* z, VT* p, VT* q, const Scratch& S, double rtol, int64_t maxiter) {
   hipStream_t st = ctx->stream;
   const int64_t n = K.ndof();
   const unsigned gv = vgrid(n, ctx);
-  const unsigned gs = K.grid();
-  LLFEM_HIP(hipMemcpyAsync(r, b, sizeof(VT) * n, hipMemcpyDeviceToDevice, st));
-  k_init<VT><<<gv, kBS, 0, st>>>(n, x, r, dinv, z, p, S.part);
-  k_reduce<<<1, kBS, 0, st>>>(gv, 2, S.part, S.red);
-  k_init_scal<<<1, 1, 0, st>>>(S.scal, S.red, rtol);
-  double h[S_NS];
-  const int poll = 16;
-  for (int64_t it = 0; it < maxiter;) {
-    const int64_t batch = std::min<int64_t>(poll, maxiter - it);
-    for (int64_t k = 0; k < batch; ++k) {
-      K.template spmv<MT, VT>(st, val, p, fixed, q, S.part, S.scal);
-      k_reduce<<<1, kBS, 0, st>>>(gs, 1, S.part, S.red);
-      k_alpha<<<1, 1, 0, st>>>(S.scal, S.red);
-      k_update<VT><<<gv, kBS, 0, st>>>(n, S.scal, x, r, p, q, dinv, z, S.part);
-      k_reduce<<<1, kBS, 0, st>>>(gv, 2, S.part, S.red);
-      k_beta<<<1, 1, 0, st>>>(S.scal, S.red, maxiter);
-      k_pupd<VT><<<gv, kBS, 0, st>>>(n, S.scal, z, p);
+  const int64_t groups = row_blocks(K.rows(), K.lanes);
+  // up to kMaxPasses row groups a block keep the partials within kFoldMax
+  const int64_t need = (groups + kFoldMax - 1) / kFoldMax;
+  const int passes = need <= kMaxPasses ? (int)need : 1;
+  const unsigned gs = (unsigned)((groups + passes - 1) / passes);
+  const bool fold = (int64_t)gs > kFoldMax;
+  const bool fuse = n <= kFuseMax;
+  volatile double* flag = ctx->h_poll;
+  *flag = 0.0;
+  k_init<VT><<<gv, kBS, 0, st>>>(n, x, b, r, dinv, z, p, S.part);
+  k_init_scal<<<1, kBS, 0, st>>>(gv, S.part, S.scal, rtol, ctx->h_poll);
+  VT* dir[2] = {p, b};
+  auto direction = [&](int64_t it) {
+    return Direction<VT>{z, dir[(it + 1) & 1], dir[it & 1], S.scal, S.part, (int64_t)gv, it, maxiter, ctx->h_poll, 0};
+  };
+  const int batch = 8;
+  int64_t it = 0;
+  for (int64_t k = 0;; ++k) {
+    for (int i = 0; i < batch && it < maxiter; ++i, ++it) {
+      VT* d = fuse ? dir[it & 1] : p;
+      if (fuse) K.template spmv<MT, VT>(st, gs, passes, val, direction(it), fixed, q, S.spart, S.scal);
+      else K.template spmv<MT, VT>(st, gs, passes, val, Plain<VT>{p}, fixed, q, S.spart, S.scal);
+      if (fold) k_fold<<<kFoldBlocks, kBS, 0, st>>>(gs, S.spart, S.spart + gs, S.scal);
+      k_update<VT><<<gv, kBS, 0, st>>>(n, S.scal, (int)(it & 1), fold ? (int64_t)kFoldBlocks : (int64_t)gs,
+                                       fold ? S.spart + gs : S.spart, x, r, d, q, dinv, z, S.part);
+      if (!fuse) k_pupd<VT><<<gv, kBS, 0, st>>>(n, S.scal, it, gv, S.part, maxiter, z, p, ctx->h_poll);
     }
-    it += batch;
-    LLFEM_HIP(hipMemcpyAsync(h, S.scal, sizeof(h), hipMemcpyDeviceToHost, st));
-    LLFEM_HIP(hipStreamSynchronize(st));
-    if (h[S_DONE] != 0.0) break;
+    // the fused SpMV tests the update before it: one more when maxiter is reached
+    if (fuse && it >= maxiter && it > 0)
+      K.template spmv<MT, VT>(st, gs, passes, val, direction(it), fixed, q, S.spart, S.scal);
+    LLFEM_HIP(hipEventRecord(ctx->poll_ev[k & 1], st));
+    if (k > 0) LLFEM_HIP(hipEventSynchronize(ctx->poll_ev[(k - 1) & 1]));
+    if (*flag != 0.0 || it >= maxiter) break;
   }
-  LLFEM_HIP(hipMemcpyAsync(h, S.scal, sizeof(h), hipMemcpyDeviceToHost, st));
-  LLFEM_HIP(hipStreamSynchronize(st));
   LLFEM_HIP(hipGetLastError());
-  *iters = (int64_t)h[S_ITER];
-  const double b2 = rtol > 0 ? h[S_TOL2] / (rtol * rtol) : 0.0;
-  *res_rel = b2 > 0 ? std::sqrt(h[S_RR] / b2) : 0.0;
   return LLFEM_OK;
+}
+
+// Iterations and relative recursive residual of a finished pcg from the
+// words k_report left.
+void pcg_result(const llfem_ctx* ctx, double rtol, int64_t* iters, double* res_rel) {
+  const double* h = ctx->h_poll + 1;
+  *iters = (int64_t)h[0];
+  const double b2 = rtol > 0 ? h[2] / (rtol * rtol) : 0.0;
+  *res_rel = b2 > 0 ? std::sqrt(h[1] / b2) : 0.0;
 }
 
 __global__ void k_zero(int64_t n, double* __restrict__ a) {
@@ -393,7 +608,7 @@ __global__ void k_zero(int64_t n, double* __restrict__ a) {
 template <typename Op>
 size_t solve_ws_bytes(llfem_ctx* ctx, const Op& K, int method) {
   const int64_t n = K.ndof();
-  const int64_t nparts = std::max<int64_t>(K.grid(), 2 * (int64_t)vgrid(n, ctx)) + 2;
+  const int64_t nparts = std::max<int64_t>(row_blocks(K.rows(), kG), 2 * (int64_t)vgrid(n, ctx)) + 2;
   const size_t nf = method == LLFEM_PCG_MIXED_REFINE ? 7 : 0;
   return sizeof(double) * (8 * (size_t)n + (size_t)nparts + 8 + S_NS + 8) + sizeof(float) * (nf * (size_t)n + 8);
 }
@@ -409,7 +624,7 @@ int solve_device_ws(llfem_ctx* ctx, const Op& K, const double* val, const float*
   hipStream_t st = ctx->stream;
   const int64_t n = K.ndof();
   const unsigned gv = vgrid(n, ctx);
-  const int64_t nparts = std::max<int64_t>(K.grid(), 2 * (int64_t)gv) + 2;
+  const int64_t nparts = std::max<int64_t>(row_blocks(K.rows(), kG), 2 * (int64_t)gv) + 2;
   const bool mixed = (method == LLFEM_PCG_MIXED_REFINE);
   double* b = (double*)base;
   double* x = b + n;
@@ -419,7 +634,7 @@ int solve_device_ws(llfem_ctx* ctx, const Op& K, const double* val, const float*
   double* q = p + n;
   double* dinv = q + n;
   double* y = dinv + n;
-  Scratch S{y + n, y + n + nparts, y + n + nparts + 8};
+  Scratch S{y + n, y, y + n + nparts, y + n + nparts + 8};   // y is free while pcg runs
   float* f32 = (float*)(S.scal + S_NS + 8);
   float *b32 = f32, *x32 = b32 + n, *r32 = x32 + n, *z32 = r32 + n, *p32 = z32 + n, *q32 = p32 + n,
         *dinv32 = q32 + n;
@@ -428,24 +643,19 @@ int solve_device_ws(llfem_ctx* ctx, const Op& K, const double* val, const float*
   if (mixed) K.template dinv<float>(st, val, fixed, dinv32);
   // u = u_fixed on constrained DoFs; b = mask(f - K u)  (src/linear.jl:3730-3733)
   k_masked_set<<<gv, kBS, 0, st>>>(n, fixed, ufix, u);
-  K.template spmv<double, double>(st, val, u, (const uint8_t*)nullptr, y, nullptr, nullptr);
+  apply(st, K, val, u, nullptr, y);
   k_resid<<<gv, kBS, 0, st>>>(n, f, y, fixed, b, S.part);
-  k_reduce<<<1, kBS, 0, st>>>(gv, 1, S.part, S.red);
-  double bn2 = 0.0;
-  LLFEM_HIP(hipMemcpyAsync(&bn2, S.red, sizeof(double), hipMemcpyDeviceToHost, st));
-  LLFEM_HIP(hipStreamSynchronize(st));
-  const double bnorm = std::sqrt(bn2);
   int64_t total_it = 0, refinements = 0;
   bool converged = false;
   if (!mixed) {
-    int64_t it = 0;
-    double rr = 0.0;
-    LLFEM_TRY((pcg<Op, double, double>(ctx, K, val, fixed, dinv, b, x, r, z, p, q, S, reltol, maxiter,
-                                       &it, &rr)));
-    total_it = it;
-    converged = rr <= reltol;
+    LLFEM_TRY((pcg<Op, double, double>(ctx, K, val, fixed, dinv, b, x, r, z, p, q, S, reltol, maxiter)));
     k_axpy<<<gv, kBS, 0, st>>>(n, 1.0, x, u);
   } else {
+    double bn2 = 0.0;
+    k_reduce<<<1, kBS, 0, st>>>(gv, 1, S.part, S.red);
+    LLFEM_HIP(hipMemcpyAsync(&bn2, S.red, sizeof(double), hipMemcpyDeviceToHost, st));
+    LLFEM_HIP(hipStreamSynchronize(st));
+    const double bnorm = std::sqrt(bn2);
     // x accumulates the free-DoF correction in FP64; r is the FP64 residual
     k_zero<<<gv, kBS, 0, st>>>(n, x);
     LLFEM_HIP(hipMemcpyAsync(r, b, sizeof(double) * n, hipMemcpyDeviceToDevice, st));
@@ -460,17 +670,16 @@ int solve_device_ws(llfem_ctx* ctx, const Op& K, const double* val, const float*
       int64_t it = 0;
       double rr = 0.0;
       LLFEM_TRY((pcg<Op, float, float>(ctx, K, val32, fixed, dinv32, b32, x32, r32, z32, p32, q32, S,
-                                       rin, maxiter - total_it, &it, &rr)));
-      total_it += it;
+                                       rin, maxiter - total_it)));
       k_axpy_f32<<<gv, kBS, 0, st>>>(n, rnorm, x32, x);
       // FP64 residual r = mask(b - K x)
-      K.template spmv<double, double>(st, val, x, fixed, y, nullptr, nullptr);
+      apply(st, K, val, x, fixed, y);
       k_resid<<<gv, kBS, 0, st>>>(n, b, y, fixed, r, S.part);
-      k_reduce<<<1, kBS, 0, st>>>(gv, 1, S.part, S.red);
-      double r2 = 0.0;
-      LLFEM_HIP(hipMemcpyAsync(&r2, S.red, sizeof(double), hipMemcpyDeviceToHost, st));
+      k_report<<<1, kBS, 0, st>>>(gv, S.part, nullptr, S.scal, ctx->h_poll + 1);
       LLFEM_HIP(hipStreamSynchronize(st));
-      rnorm = std::sqrt(r2);
+      pcg_result(ctx, rin, &it, &rr);
+      total_it += it;
+      rnorm = std::sqrt(ctx->h_poll[4]);
       ++refinements;
       if (it == 0) break;
     }
@@ -478,20 +687,18 @@ int solve_device_ws(llfem_ctx* ctx, const Op& K, const double* val, const float*
     k_axpy<<<gv, kBS, 0, st>>>(n, 1.0, x, u);
   }
   // reported residual: ||(K u - f)_free|| / ||f_free|| (test/test_dsl.jl:106)
-  K.template spmv<double, double>(st, val, u, (const uint8_t*)nullptr, y, nullptr, nullptr);
-  k_resid<<<gv, kBS, 0, st>>>(n, f, y, fixed, r, S.part);
-  k_reduce<<<1, kBS, 0, st>>>(gv, 1, S.part, S.red);
-  double rr2 = 0.0;
-  LLFEM_HIP(hipMemcpyAsync(&rr2, S.red, sizeof(double), hipMemcpyDeviceToHost, st));
-  LLFEM_HIP(hipStreamSynchronize(st));
-  // ||f_free||
-  k_zero<<<gv, kBS, 0, st>>>(n, y);
-  k_resid<<<gv, kBS, 0, st>>>(n, f, y, fixed, z, S.part);
-  k_reduce<<<1, kBS, 0, st>>>(gv, 1, S.part, S.red);
-  double ff2 = 0.0;
-  LLFEM_HIP(hipMemcpyAsync(&ff2, S.red, sizeof(double), hipMemcpyDeviceToHost, st));
+  apply(st, K, val, u, nullptr, y);
+  k_resid<<<gv, kBS, 0, st>>>(n, f, y, fixed, nullptr, S.part);
+  k_resid<<<gv, kBS, 0, st>>>(n, f, nullptr, fixed, nullptr, S.part + gv);
+  k_report<<<1, kBS, 0, st>>>(gv, S.part, S.part + gv, S.scal, ctx->h_poll + 1);
   LLFEM_HIP(hipStreamSynchronize(st));
   LLFEM_HIP(hipGetLastError());
+  if (!mixed) {
+    double rr = 0.0;
+    pcg_result(ctx, reltol, &total_it, &rr);
+    converged = rr <= reltol;
+  }
+  const double rr2 = ctx->h_poll[4], ff2 = ctx->h_poll[5];
   const double relres = ff2 > 0 ? std::sqrt(rr2 / ff2) : std::sqrt(rr2);
   if (stats) {
     stats->iterations = total_it;
@@ -704,13 +911,27 @@ int ensure_k32(llfem_mesh* m) {
 }
 
 namespace {
+// err |= 4: colptr does not start at 0 or ends below it; 1: colptr falls;
+// 2: a row index out of range.  The row indices are only read while the ends
+// are in order.
 __global__ void k_check_csc(int64_t n, const int64_t* __restrict__ colptr, const int32_t* __restrict__ rowval,
-                            int64_t nnz, int* __restrict__ err) {
+                            int* __restrict__ err) {
+  const int64_t nnz = colptr[n];
+  if (colptr[0] != 0 || nnz < 0) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) atomicOr(err, 4);
+    return;
+  }
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   for (int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; j < n; j += stride)
     if (colptr[j + 1] < colptr[j]) atomicOr(err, 1);
   for (int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < nnz; k += stride)
     if (rowval[k] < 0 || (int64_t)rowval[k] >= n) atomicOr(err, 2);
+}
+
+__global__ void k_check_report(int64_t n, const int64_t* __restrict__ colptr, const int* __restrict__ err,
+                               double* out) {
+  out[0] = (double)*err;
+  out[1] = (double)colptr[n];
 }
 
 __global__ void k_zero_int(int* a) { *a = 0; }
@@ -748,7 +969,7 @@ int llfem_solve(llfem_mesh* m, const double* f, const int64_t* fixed, int64_t nf
                                u_fixed, u_out, stats, method == LLFEM_PCG_AMG_RELIABLE ? m : nullptr);
   }
   if (method == LLFEM_PCG_MIXED_REFINE) LLFEM_TRY(ensure_k32(m));
-  PanelOp K{m->N, m->d_adj_ptr, m->d_adj, m->d_diag_slot};
+  PanelOp K{m->N, m->d_adj_ptr, m->d_adj, m->d_diag_slot, panel_lanes(m->N, m->nadj)};
   return solve_host(m->ctx, K, m->d_valK, m->d_valK32, 3 * m->N, f, fixed, nfixed, one_based, u_fixed,
                     method, reltol, maxiter, u_out, stats);
 }
@@ -796,7 +1017,7 @@ int llfem_solve_csc(llfem_ctx* ctx, int64_t n, const int64_t* colptr, const int6
   k_i64_sub<<<vgrid(n + 1, ctx), kBS, 0, st>>>(n + 1, d_cp, base);
   k_i64_to_i32<<<vgrid(nnz, ctx), kBS, 0, st>>>(nnz, d_rv64, base, d_rv);
   if (method == LLFEM_PCG_MIXED_REFINE) k_cast_val<<<vgrid(nnz, ctx), kBS, 0, st>>>(nnz, d_val, d_val32);
-  CscOp K{n, d_cp, d_rv};
+  CscOp K{n, d_cp, d_rv, csc_lanes(n, nnz)};
   return solve_host(ctx, K, d_val, d_val32, n, f, fixed, nfixed, one_based, u_fixed, method, reltol,
                     maxiter, u_out, stats);
 }
@@ -809,7 +1030,7 @@ int llfem_solve_csc_noalloc(llfem_ctx* ctx, int64_t n, const int64_t* d_colptr, 
     return fail(LLFEM_EINVAL, "llfem_solve_csc_noalloc: NULL argument");
   if (n <= 0 || n >= ((int64_t)1 << 31)) return fail(LLFEM_EINVAL, "llfem_solve_csc_noalloc: bad size");
   if (!(reltol > 0)) return fail(LLFEM_EINVAL, "llfem_solve_csc_noalloc: reltol must be positive");
-  CscOp K{n, d_colptr, d_rowval};
+  CscOp K{n, d_colptr, d_rowval, kG};
   // the flag word of the index check sits after the solver's workspace
   const size_t ws = (solve_ws_bytes(ctx, K, LLFEM_PCG_JACOBI_FP64) + 255) & ~(size_t)255;
   if (ws + 256 > kNoAllocScratchBytes)
@@ -829,18 +1050,16 @@ int llfem_solve_csc_noalloc(llfem_ctx* ctx, int64_t n, const int64_t* d_colptr, 
   hipStream_t st = ctx->stream;
   auto t0 = std::chrono::steady_clock::now();
   // the same index checks as llfem_solve_csc, on the device
-  int64_t ends[2] = {0, 0};
-  LLFEM_HIP(hipMemcpyAsync(&ends[0], d_colptr, sizeof(int64_t), hipMemcpyDeviceToHost, st));
-  LLFEM_HIP(hipMemcpyAsync(&ends[1], d_colptr + n, sizeof(int64_t), hipMemcpyDeviceToHost, st));
-  LLFEM_HIP(hipStreamSynchronize(st));
-  if (ends[0] != 0 || ends[1] < 0) return fail(LLFEM_EINVAL, "llfem_solve_csc_noalloc: bad colptr");
   k_zero_int<<<1, 1, 0, st>>>(d_err);
-  k_check_csc<<<vgrid(std::max<int64_t>(n, ends[1]), ctx), kBS, 0, st>>>(n, d_colptr, d_rowval, ends[1], d_err);
-  int herr = 0;
-  LLFEM_HIP(hipMemcpyAsync(&herr, d_err, sizeof(int), hipMemcpyDeviceToHost, st));
+  k_check_csc<<<vgrid(8 * n, ctx), kBS, 0, st>>>(n, d_colptr, d_rowval, d_err);
+  k_check_report<<<1, 1, 0, st>>>(n, d_colptr, d_err, ctx->h_poll + 1);
   LLFEM_HIP(hipStreamSynchronize(st));
+  LLFEM_HIP(hipGetLastError());
+  const int herr = (int)ctx->h_poll[1];
+  if (herr & 4) return fail(LLFEM_EINVAL, "llfem_solve_csc_noalloc: bad colptr");
   if (herr & 1) return fail(LLFEM_EINVAL, "llfem_solve_csc_noalloc: colptr is not non-decreasing");
   if (herr & 2) return fail(LLFEM_EINVAL, "llfem_solve_csc_noalloc: row index out of range");
+  K.lanes = csc_lanes(n, (int64_t)ctx->h_poll[2]);
   const int s = solve_device_ws(ctx, K, d_nzval, nullptr, d_fixed, d_f, d_u_fixed, LLFEM_PCG_JACOBI_FP64,
                                 reltol, maxiter, d_u_out, stats, base);
   if (s != LLFEM_OK && s != LLFEM_ENOCONV) return s;
