@@ -110,6 +110,10 @@ struct llfem_ctx {
   std::map<uint64_t, llfem::DevTable> tables;      // by content hash
   void* d_scratch = nullptr;                       // batch descriptors + queue counter
   size_t scratch_bytes = 0;
+  // workspace kept between calls (WsGuard): at most kWsKeep bytes stay
+  void* ws = nullptr;
+  size_t ws_bytes = 0;
+  bool ws_busy = false;
   double* d_sink = nullptr;                        // 64 doubles: target of padding-lane panel stores
   // pinned staging for large device-to-host copies (copy_to_host)
   void* h_stage[2] = {nullptr, nullptr};
@@ -211,6 +215,33 @@ void drelease(llfem_ctx* ctx, T*& p, size_t count) {
   if (p) dfree(ctx, p, count * sizeof(T));
   p = nullptr;
 }
+
+// The context's workspace for one call: get() hands out `bytes` bytes that
+// hold anything, take() parts of them (256-byte aligned).  All work on it is
+// on the context's stream, so a later call's kernels run after this call's.
+// It is kept for the next call up to kWsKeep bytes (allocating and freeing the
+// few buffers of a load vector cost it 0.8 of 3.1 ms), counts as in use, and
+// is given back when an allocation would not fit otherwise.
+constexpr size_t kWsKeep = size_t(256) << 20;
+class WsGuard {
+ public:
+  explicit WsGuard(llfem_ctx* c) : c_(c) {}
+  ~WsGuard();
+  int get(size_t bytes);
+  template <typename T>
+  T* take(size_t count) {
+    T* p = reinterpret_cast<T*>(static_cast<char*>(c_->ws) + off_);
+    off_ += aligned(count * sizeof(T));
+    return p;
+  }
+  static size_t aligned(size_t bytes) { return (bytes + 255) & ~size_t(255); }
+
+ private:
+  llfem_ctx* c_;
+  size_t off_ = 0;
+  bool held_ = false;
+};
+void ws_release(llfem_ctx* ctx);   // frees an idle workspace
 
 int build_pattern(llfem_mesh* m);
 int rebuild_records(llfem_mesh* m);

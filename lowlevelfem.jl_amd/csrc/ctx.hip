@@ -17,11 +17,17 @@ void set_error(const std::string& msg) { g_error = msg; }
 int dmalloc(llfem_ctx* ctx, void** p, size_t bytes) {
   *p = nullptr;
   if (bytes == 0) return LLFEM_OK;
+  if (ctx->budget && ctx->in_use + bytes > ctx->budget) ws_release(ctx);
   if (ctx->budget && ctx->in_use + bytes > ctx->budget)
     return fail(LLFEM_ENOMEM, "HBM budget exceeded: need " + std::to_string(bytes) +
                                   " more bytes, " + std::to_string(ctx->in_use) + " of " +
                                   std::to_string(ctx->budget) + " in use");
   hipError_t e = hipMalloc(p, bytes);
+  if (e != hipSuccess && ctx->ws && !ctx->ws_busy) {
+    (void)hipGetLastError();
+    ws_release(ctx);
+    e = hipMalloc(p, bytes);
+  }
   if (e != hipSuccess) {
     *p = nullptr;
     (void)hipGetLastError();
@@ -36,6 +42,29 @@ void dfree(llfem_ctx* ctx, void* p, size_t bytes) {
   if (!p) return;
   (void)hipFree(p);
   ctx->in_use -= bytes;
+}
+
+void ws_release(llfem_ctx* ctx) {
+  if (!ctx->ws || ctx->ws_busy) return;
+  dfree(ctx, ctx->ws, ctx->ws_bytes);
+  ctx->ws = nullptr;
+  ctx->ws_bytes = 0;
+}
+
+int WsGuard::get(size_t bytes) {
+  if (c_->ws_bytes < bytes) {
+    ws_release(c_);
+    LLFEM_TRY(dmalloc(c_, &c_->ws, bytes));
+    c_->ws_bytes = bytes;
+  }
+  c_->ws_busy = held_ = true;
+  return LLFEM_OK;
+}
+
+WsGuard::~WsGuard() {
+  if (!held_) return;
+  c_->ws_busy = false;
+  if (c_->ws_bytes > kWsKeep) ws_release(c_);
 }
 
 // Large copies go through two pinned staging buffers: the DMA engine fills
@@ -221,6 +250,7 @@ int llfem_ctx_destroy(llfem_ctx* ctx) {
   for (auto& kv : ctx->tables) llfem::dfree(ctx, kv.second.ptr, kv.second.bytes);
   ctx->tables.clear();
   if (ctx->d_scratch) llfem::dfree(ctx, ctx->d_scratch, ctx->scratch_bytes);
+  llfem::ws_release(ctx);
   if (ctx->d_sink) llfem::dfree(ctx, ctx->d_sink, 64 * sizeof(double));
   for (int k = 0; k < 2; ++k) {
     if (ctx->side[k]) {
