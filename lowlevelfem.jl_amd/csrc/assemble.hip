@@ -330,23 +330,27 @@ int geometry_state(llfem_mesh* m, const llfem_op_desc* d, bool* affine_out) {
   return LLFEM_OK;
 }
 
-int run_geometry(llfem_mesh* m, const llfem_op_desc* d, bool affine, const double* d_scale, bool f32) {
-  llfem_ctx* ctx = m->ctx;
-  const int npe = m->npe, q = d->q;
-  const size_t geo_doubles = (size_t)kGeoStride * m->E * (affine ? 1 : q);
-  LLFEM_TRY(ensure_buf(ctx, &m->d_geo, &m->geo_bytes, sizeof(double) * geo_doubles));
+template <int MODE>
+void launch_geometry(llfem_mesh* m, int q, bool affine, const double* d_scale) {
+  const int npe = m->npe;
+  hipStream_t st = m->ctx->stream;
+  const double* w = m->d_tab + (size_t)q * npe * 3;
   const int64_t threads = affine ? m->E : m->E * q;
-  if (affine) {
-    const unsigned g = (unsigned)((m->E + 255) / 256);
-    const double* dN0 = m->d_tab;   // gradients at the first point
-#define LLFEM_GEO_AFFINE(n)                                                                        \
-  case n:                                                                                          \
-    if (f32)                                                                                       \
-      k_geometry_affine<n, true><<<g, 256, 0, ctx->stream>>>(m->E, m->d_xyz4, m->d_conn, dN0, m->d_geo, d_scale); \
-    else                                                                                           \
-      k_geometry_affine<n, false><<<g, 256, 0, ctx->stream>>>(m->E, m->d_xyz4, m->d_conn, dN0, m->d_geo, d_scale); \
-    return LLFEM_OK;
-    switch (npe) {
+  const unsigned g = (unsigned)((threads + 255) / 256);
+  double* dNT = m->d_tab + dnt_offset(npe, q);
+  if (!affine) {
+    const int64_t nt = (int64_t)q * npe * 3;
+    k_dn_transpose<<<(unsigned)((nt + 255) / 256), 256, 0, st>>>(npe, q, m->d_tab, dNT);
+  }
+#define LLFEM_GEO_AFFINE(n)                                                                                  \
+  case n:                                                                                                    \
+    k_geometry_affine<n, MODE><<<g, 256, 0, st>>>(m->E, m->d_xyz4, m->d_conn, m->d_tab, m->d_geo, d_scale); \
+    return;
+#define LLFEM_GEO_POINTS(n)                                                                                 \
+  case n:                                                                                                   \
+    k_geometry_points<n, MODE><<<g, 256, 0, st>>>(m->E, q, m->d_xyz4, m->d_conn, dNT, w, m->d_geo, d_scale); \
+    return;
+  if (affine) switch (npe) {   // gradients at the first point
       LLFEM_GEO_AFFINE(4)
       LLFEM_GEO_AFFINE(6)
       LLFEM_GEO_AFFINE(8)
@@ -355,21 +359,31 @@ int run_geometry(llfem_mesh* m, const llfem_op_desc* d, bool affine, const doubl
       LLFEM_GEO_AFFINE(27)
       default: break;
     }
-#undef LLFEM_GEO_AFFINE
-  }
-  if (!affine) {
-    double* dNT = m->d_tab + dnt_offset(npe, q);
-    const int64_t nt = (int64_t)q * npe * 3;
-    k_dn_transpose<<<(unsigned)((nt + 255) / 256), 256, 0, ctx->stream>>>(npe, q, m->d_tab, dNT);
-    if (npe <= kCurvedMaxNpe) {
-      k_geometry_curved<<<(unsigned)m->E, 128, 0, ctx->stream>>>(m->E, m->N, npe, q, m->d_xyz, m->d_conn, dNT,
-                                                                 m->d_tab + (size_t)q * npe * 3, m->d_geo, d_scale);
-      return LLFEM_OK;
+  else switch (npe) {
+      LLFEM_GEO_POINTS(4)
+      LLFEM_GEO_POINTS(6)
+      LLFEM_GEO_POINTS(8)
+      LLFEM_GEO_POINTS(10)
+      default: break;
     }
-  }
-  k_geometry<<<(unsigned)((threads + 255) / 256), 256, 0, ctx->stream>>>(
-      m->E, m->N, npe, q, affine ? 1 : 0, m->d_xyz, m->d_conn, m->d_tab,
-      m->d_tab + (size_t)q * npe * 3, m->d_geo, d_scale);
+#undef LLFEM_GEO_AFFINE
+#undef LLFEM_GEO_POINTS
+  if (!affine && npe <= kCurvedMaxNpe)
+    k_geometry_curved<MODE><<<(unsigned)m->E, 128, 0, st>>>(m->E, m->N, npe, q, m->d_xyz, m->d_conn, dNT, w, m->d_geo,
+                                                            d_scale);
+  else
+    k_geometry<MODE><<<g, 256, 0, st>>>(m->E, m->N, npe, q, affine ? 1 : 0, m->d_xyz, m->d_conn, m->d_tab, w,
+                                        m->d_geo, d_scale);
+}
+
+int run_geometry(llfem_mesh* m, const llfem_op_desc* d, bool affine, const double* d_scale, bool f32) {
+  const bool wd_only = d->op == LLFEM_OP_MASS;
+  const size_t recs = (size_t)m->E * (affine ? 1 : d->q);
+  LLFEM_TRY(ensure_buf(m->ctx, &m->d_geo, &m->geo_bytes, sizeof(double) * recs * (wd_only ? 1 : kGeoStride)));
+  if (wd_only) launch_geometry<kGeoWd>(m, d->q, affine, d_scale);
+  else if (f32) launch_geometry<kGeoF32>(m, d->q, affine, d_scale);
+  else launch_geometry<kGeoF64>(m, d->q, affine, d_scale);
+  LLFEM_HIP(hipGetLastError());
   return LLFEM_OK;
 }
 
@@ -470,6 +484,7 @@ int assemble_impl(llfem_mesh* m, const llfem_op_desc* d, double* nzval_out, llfe
   PanelParams P{};
   P.rec_bytes = m->rec_bytes;
   P.geo = m->d_geo;
+  P.geo_stride = 1;   // mass: packed wd
   P.E = m->E;
   P.q = q;
   P.tab = m->d_tab + off;
@@ -622,7 +637,9 @@ int assemble_impl(llfem_mesh* m, const llfem_op_desc* d, double* nzval_out, llfe
   }
   if (op == LLFEM_OP_MASS && d->lumped) {
     if (!m->d_lumped) LLFEM_TRY(dalloc(ctx, &m->d_lumped, 3 * m->N));
-    k_lump<<<(unsigned)((m->N + 255) / 256), 256, 0, st>>>(m->N, m->d_adj_ptr, m->d_valM, m->d_lumped);
+    k_lump<<<lump_blocks(m->N), 256, sizeof(double) * (affine ? npe : q), st>>>(
+        m->N, npe, q, affine ? 1 : 0, m->d_inc_ptr, m->d_inc_elem, m->d_inc_loc, m->d_geo, P.geo_stride, P.geo_ofs,
+        P.tab, d->rho, m->d_lumped);
   }
   LLFEM_HIP(hipEventRecord(ctx->ev[3], st));
   if (dev_out) {

@@ -361,6 +361,8 @@ extern "C" int llfem_assemble_batch(int32_t n, llfem_mesh* const* meshes, const 
       P.cnt = L.cnt;
       P.max_r = L.max_r;
       P.geo = m->d_geo;
+      P.geo_stride = kGeoStride;
+      P.geo_ofs = 9;
       P.E = m->E;
       P.q = d->q;
       P.tab = it.tab;
@@ -450,7 +452,9 @@ extern "C" int llfem_assemble_batch(int32_t n, llfem_mesh* const* meshes, const 
         m->have_lumped = it.d->lumped != 0;
         if (it.d->lumped) {
           if (!m->d_lumped) LLFEM_TRY(dalloc(ctx, &m->d_lumped, 3 * m->N));
-          k_lump<<<(unsigned)((m->N + 255) / 256), 256, 0, st>>>(m->N, m->d_adj_ptr, m->d_valM, m->d_lumped);
+          k_lump<<<lump_blocks(m->N), 256, sizeof(double) * (it.affine ? m->npe : it.d->q), st>>>(
+              m->N, m->npe, it.d->q, it.affine ? 1 : 0, m->d_inc_ptr, m->d_inc_elem, m->d_inc_loc, m->d_geo,
+              kGeoStride, 9, it.tab, it.d->rho, m->d_lumped);
         }
       }
     }

@@ -89,16 +89,29 @@ __global__ void k_geom_check(int64_t E, int64_t N, int npe, int q, const double*
 // (element, point), wd = |det J_p| w_p.
 constexpr int kGeoStride = 16;   // doubles
 
-// F32: also write the FP32 copy that the FP32-integration kernels read
-template <bool F32 = true>
-__device__ __forceinline__ void geometry_store(double* g, const double* Mi, double wd) {
+// What a geometry kernel writes: records without or with the FP32 copy that
+// the FP32-integration kernels read, or -- for the mass operators, which need
+// no inverse Jacobian -- only wd, packed.  A mass step gathers 8 bytes an
+// element (or q consecutive doubles, curved): out of the records that pulls a
+// 128-byte line for each, out of the packed array (12 MB on the 40x40x160
+// tet10 beam) it hits in L2, and the geometry kernel writes 8 bytes an element
+// instead of 80 (91 -> 38 us there).
+enum GeoMode { kGeoF64 = 0, kGeoF32 = 1, kGeoWd = 2 };
+
+template <int MODE = kGeoF32>
+__device__ __forceinline__ void geometry_store(double* geo, size_t i, const double* Mi, double wd) {
+  if constexpr (MODE == kGeoWd) {
+    geo[i] = wd;
+    return;
+  }
+  double* g = geo + i * kGeoStride;
   double2* g2 = reinterpret_cast<double2*>(g);
   g2[0] = make_double2(Mi[0], Mi[1]);
   g2[1] = make_double2(Mi[2], Mi[3]);
   g2[2] = make_double2(Mi[4], Mi[5]);
   g2[3] = make_double2(Mi[6], Mi[7]);
   g2[4] = make_double2(Mi[8], wd);
-  if constexpr (!F32) return;
+  if constexpr (MODE != kGeoF32) return;
   float4* f4 = reinterpret_cast<float4*>(g + 10);
   f4[0] = make_float4((float)Mi[0], (float)Mi[1], (float)Mi[2], (float)Mi[3]);
   f4[1] = make_float4((float)Mi[4], (float)Mi[5], (float)Mi[6], (float)Mi[7]);
@@ -120,7 +133,7 @@ __device__ __forceinline__ void geometry_one(int64_t E, int64_t N, int npe, int 
     jacobian(E, N, npe, e, xyz, conn, dN + (size_t)p * npe * 3, J);
     const double det = inv3(J, Mi);
     const double wd = (affine ? fabs(det) : fabs(det) * w[p]) * se;
-    geometry_store(geo + ((size_t)e * np + p) * kGeoStride, Mi, wd);
+    geometry_store(geo, (size_t)e * np + p, Mi, wd);
   }
 }
 
@@ -129,8 +142,8 @@ __device__ __forceinline__ void geometry_one(int64_t E, int64_t N, int npe, int 
 // before the first is used (the run-time loop waits for each node's gathers
 // in turn).  Coordinates come from the node-major copy (x, y, z, 0 per node:
 // two 16-byte loads from one line per node instead of three loads from three
-// arrays); F32 selects the FP32 copy in the record.
-template <int NPE, bool F32>
+// arrays).
+template <int NPE, int MODE>
 __global__ __launch_bounds__(256) void k_geometry_affine(int64_t E, const double4* __restrict__ xyz4,
                                                          const int32_t* __restrict__ conn,
                                                          const double* __restrict__ dN, double* __restrict__ geo,
@@ -160,7 +173,7 @@ __global__ __launch_bounds__(256) void k_geometry_affine(int64_t E, const double
     J[6] += dz * g0; J[7] += dz * g1; J[8] += dz * g2;
   }
   const double det = inv3(J, Mi);
-  geometry_store<F32>(geo + (size_t)e * kGeoStride, Mi, fabs(det) * (scale ? scale[e] : 1.0));
+  geometry_store<MODE>(geo, (size_t)e, Mi, fabs(det) * (scale ? scale[e] : 1.0));
 }
 
 // dNT[(a * q + p) * 3 + c] = dN[(p * npe + a) * 3 + c]: the gradient table
@@ -183,6 +196,7 @@ __global__ __launch_bounds__(256) void k_dn_transpose(int npe, int q, const doub
 // neighbouring points, load neighbouring doubles).
 constexpr int kCurvedMaxNpe = 128;
 
+template <int MODE>
 __global__ __launch_bounds__(128) void k_geometry_curved(int64_t E, int64_t N, int npe, int q,
                                                          const double* __restrict__ xyz,
                                                          const int32_t* __restrict__ conn,
@@ -213,29 +227,62 @@ __global__ __launch_bounds__(128) void k_geometry_curved(int64_t E, int64_t N, i
       J[6] += z * g0; J[7] += z * g1; J[8] += z * g2;
     }
     const double det = inv3(J, Mi);
-    geometry_store(geo + ((size_t)e * q + p) * kGeoStride, Mi, fabs(det) * w[p] * (scale ? scale[e] : 1.0));
+    geometry_store<MODE>(geo, (size_t)e * q + p, Mi, fabs(det) * w[p] * (scale ? scale[e] : 1.0));
   }
 }
 
-// Affine: thread per element.  Curved: thread per (element, point), so
-// high-order elements with many points keep the device busy.
+// Curved elements of few nodes: thread per (element, point), every gather
+// issued before the first is used; the lanes of an element's points read the
+// same addresses.  (A 128-thread block per element leaves 120 of them idle on
+// hex8 with 8 points: 66 us against 29 us for 63,360 elements.)
+template <int NPE, int MODE>
+__global__ __launch_bounds__(256) void k_geometry_points(int64_t E, int q, const double4* __restrict__ xyz4,
+                                                         const int32_t* __restrict__ conn,
+                                                         const double* __restrict__ dNT,
+                                                         const double* __restrict__ w, double* __restrict__ geo,
+                                                         const double* __restrict__ scale) {
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= E * q) return;
+  const int64_t e = t / q;
+  const int p = (int)(t - e * q);
+  int32_t v[NPE];
+#pragma unroll
+  for (int a = 0; a < NPE; ++a) v[a] = conn[(int64_t)a * E + e];
+  double4 x[NPE];
+#pragma unroll
+  for (int a = 0; a < NPE; ++a) x[a] = xyz4[v[a]];
+  double J[9], Mi[9];
+#pragma unroll
+  for (int k = 0; k < 9; ++k) J[k] = 0.0;
+#pragma unroll
+  for (int a = 1; a < NPE; ++a) {
+    const double dx = x[a].x - x[0].x, dy = x[a].y - x[0].y, dz = x[a].z - x[0].z;
+    const double* g = dNT + ((int64_t)a * q + p) * 3;
+    const double g0 = g[0], g1 = g[1], g2 = g[2];
+    J[0] += dx * g0; J[1] += dx * g1; J[2] += dx * g2;
+    J[3] += dy * g0; J[4] += dy * g1; J[5] += dy * g2;
+    J[6] += dz * g0; J[7] += dz * g1; J[8] += dz * g2;
+  }
+  const double det = inv3(J, Mi);
+  geometry_store<MODE>(geo, (size_t)t, Mi, fabs(det) * w[p] * (scale ? scale[e] : 1.0));
+}
+
+// Any node count.  Affine: thread per element.  Curved: thread per (element,
+// point).
+template <int MODE>
 __global__ void k_geometry(int64_t E, int64_t N, int npe, int q, int affine,
                            const double* __restrict__ xyz, const int32_t* __restrict__ conn,
                            const double* __restrict__ dN, const double* __restrict__ w,
                            double* __restrict__ geo, const double* __restrict__ scale) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (affine) {
-    if (t >= E) return;
-    geometry_one(E, N, npe, q, 1, xyz, conn, dN, w, geo, t, scale);
-    return;
-  }
-  if (t >= E * q) return;
-  const int64_t e = t / q;
-  const int p = (int)(t - e * q);
+  const int np = affine ? 1 : q;
+  if (t >= E * np) return;
+  const int64_t e = t / np;
+  const int p = (int)(t - e * np);
   double J[9], Mi[9];
   jacobian(E, N, npe, e, xyz, conn, dN + (size_t)p * npe * 3, J);
   const double det = inv3(J, Mi);
-  geometry_store(geo + (size_t)t * kGeoStride, Mi, fabs(det) * w[p] * (scale ? scale[e] : 1.0));
+  geometry_store<MODE>(geo, (size_t)t, Mi, (affine ? fabs(det) : fabs(det) * w[p]) * (scale ? scale[e] : 1.0));
 }
 
 // ---------------------------------------------------------------------------
@@ -248,6 +295,7 @@ struct PanelParams {
   int64_t waves;
   int rounds, cnt, max_r;
   const double* geo;
+  int geo_stride, geo_ofs;   // mass: wd of (element, point) i is geo[i * geo_stride + geo_ofs]
   int64_t E;
   int q;
   const double* tab;   // double table, see llfem_assemble
@@ -271,6 +319,20 @@ constexpr int kOpKM = 2;
 // instructions in order and a compiler barrier separates the steps.
 __device__ __forceinline__ void lds_add(double* p, double v) { *p += v; }
 
+// A finished mass panel (one value per row slot) to its three component
+// columns, and cleared: each slot is read once and stored three times, by the
+// same lane.  (A lane per stored value, which divides by R and reads every slot
+// three times, takes the same time: the launches are not bound by it.)
+__device__ __forceinline__ void store_mass_panel(double* pm, int R, double* o, int lane) {
+  for (int i = lane; i < R; i += 64) {
+    const double v = pm[i];
+    pm[i] = 0.0;
+    __builtin_nontemporal_store(v, o + i);
+    __builtin_nontemporal_store(v, o + R + i);
+    __builtin_nontemporal_store(v, o + 2 * R + i);
+  }
+}
+
 template <typename Real>
 struct Geo {
   Real Mi[9];
@@ -292,6 +354,18 @@ __device__ __forceinline__ Geo<Real> load_geo(const double* __restrict__ rec) {
     g.Mi[0] = v0.x; g.Mi[1] = v0.y; g.Mi[2] = v0.z; g.Mi[3] = v0.w; g.Mi[4] = v1.x;
     g.Mi[5] = v1.y; g.Mi[6] = v1.z; g.Mi[7] = v1.w; g.Mi[8] = v2.x; g.wd = v2.y;
   }
+  return g;
+}
+
+// The geometry a step of operator OP needs: the record (affine stiffness),
+// wd alone (affine mass), nothing (curved elements read their points' records
+// in the step).
+template <int OP, bool AFFINE, typename Real>
+__device__ __forceinline__ Geo<Real> load_step_geo(const PanelParams& P, const double* __restrict__ geo, int e) {
+  Geo<Real> g;
+  if constexpr (!AFFINE) return g;
+  else if constexpr (OP == LLFEM_OP_MASS) g.wd = (Real)geo[(size_t)e * P.geo_stride + P.geo_ofs];
+  else g = load_geo<Real>(geo + (size_t)e * kGeoStride);
   return g;
 }
 
@@ -503,7 +577,7 @@ __device__ __forceinline__ void contribute(const PanelParams& P, const double* g
     } else {
       mv = 0.0;
       for (int p = 0; p < P.q; ++p)
-        mv += geo[((size_t)e * P.q + p) * kGeoStride + 9] * tab[p * NPE + b] * tab[p * NPE + a];
+        mv += geo[((size_t)e * P.q + p) * P.geo_stride + P.geo_ofs] * tab[p * NPE + b] * tab[p * NPE + a];
       mv *= P.rho;
     }
     lds_add(wl + base + s, mv);
@@ -650,7 +724,7 @@ __device__ __forceinline__ void panel_wave(const PanelParams& P, int64_t w0, int
 #pragma unroll
   for (int v = 0; v < PF; ++v) {
     const int a = RG::a(rec[v]);
-    g[v] = load_geo<Real>(geo + (size_t)RG::e(rec[v]) * kGeoStride);
+    g[v] = load_step_geo<OP, AFFINE, Real>(P, geo, RG::e(rec[v]));
     tb[v] = load_tab<NPE, OP, AFFINE, Real>(tab, tabf, tab2, a < 0 ? 0 : a, b);
   }
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -707,34 +781,11 @@ __device__ __forceinline__ void panel_wave(const PanelParams& P, int64_t w0, int
                 __builtin_nontemporal_store(pm[i], o + i);
                 pm[i] = 0.0;
               }
-              if constexpr (OP == kOpKM) {
-                double* o2 = out2 + 3 * om;
-                const double* pmm = pm + mofs;
-                for (int i = lane; i < 3 * Rm; i += 64) {
-                  const int c = i / Rm;
-                  __builtin_nontemporal_store(pmm[i - c * Rm], o2 + i);
-                }
-              }
+              if constexpr (OP == kOpKM) store_mass_panel(pm + mofs, Rm, out2 + 3 * om, lane);
             } else {
-              double* o = out + 3 * om;
-              for (int i = lane; i < 3 * Rm; i += 64) {
-                const int c = i / Rm;
-                __builtin_nontemporal_store(pm[i - c * Rm], o + i);
-              }
+              store_mass_panel(pm, Rm, out + 3 * om, lane);
             }
           }
-          }
-          if constexpr (OP == LLFEM_OP_MASS) {
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            for (int i = lane; i < NPW * P.max_r; i += 64) wl[i] = 0.0;
-          } else if constexpr (OP == kOpKM) {   // clear the mass panels once all three copies are out
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            for (int i = lane; i < NPW * P.max_r; i += 64) {
-              const int m = i / P.max_r;
-              wl[(size_t)m * P.max_r * BLK + mofs + (i - m * P.max_r)] = 0.0;
-            }
           }
           __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
           __builtin_amdgcn_wave_barrier();
@@ -749,7 +800,7 @@ __device__ __forceinline__ void panel_wave(const PanelParams& P, int64_t w0, int
       // ring refill: geometry/table for step s+PF, record for step s+2PF
       const typename RG::T& nx = rec[(u + PF) % (2 * PF)];
       const int na = RG::a(nx);
-      g[u % PF] = load_geo<Real>(geo + (size_t)RG::e(nx) * kGeoStride);
+      g[u % PF] = load_step_geo<OP, AFFINE, Real>(P, geo, RG::e(nx));
       tb[u % PF] = load_tab<NPE, OP, AFFINE, Real>(tab, tabf, tab2, na < 0 ? 0 : na, b);
       rec[u] = RG::load(recs, P.rec_bytes, min(rbase + (s + 2 * PF) * NPW + lane_rec, rlast), b);
       __builtin_amdgcn_sched_barrier(0);   // keep the step's loads in the step
@@ -932,19 +983,51 @@ __global__ __launch_bounds__(ISO ? 512 : 256) void k_panel(PanelParams P) {
   panel_wave<NPE, MapT, OP, AFFINE, ISO, Real, KS>(P, w, 1, lds + (size_t)wave * P.lds_per_wave);
 }
 
-// lumped mass: row sums of the consistent mass panels (src/linear.jl:1999-2001)
-__global__ void k_lump(int64_t N, const int64_t* __restrict__ adj_ptr, const double* __restrict__ M,
-                       double* __restrict__ out) {
-  int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= N) return;
-  const int64_t a0 = adj_ptr[j];
-  const int R = (int)(adj_ptr[j + 1] - a0);
-  for (int c = 0; c < 3; ++c) {
-    double s = 0.0;
-    for (int i = 0; i < R; ++i) s += M[3 * a0 + (int64_t)c * R + i];
-    out[3 * j + c] = s;
+// Lumped mass (src/linear.jl:1999-2001, the row sums of the consistent mass):
+// sum_b M_ab of an element needs no M,
+//   lump_j = rho sum over the node's incidences (e, a) of sum_p wd_ep N_a(p) sum_b N_b(p)
+// with the affine table's row sums in place of the points', kLumpLanes lanes
+// a node, in a fixed order.  tab: [b][a] integrals (affine, q = 1) or N
+// [q][npe].  Bound: the incidence lists and wd, 13 bytes an incidence plus 8
+// per further point.  Summing the rows of the stored M instead took 1,929 us
+// with a thread per node and 199 us coalesced (40x40x160 tet10 beam); this
+// takes 109 us.
+constexpr int kLumpLanes = 4;
+__global__ __launch_bounds__(256) void k_lump(int64_t N, int npe, int q, int affine,
+                                              const int32_t* __restrict__ inc_ptr,
+                                              const int32_t* __restrict__ inc_elem,
+                                              const uint8_t* __restrict__ inc_loc, const double* __restrict__ geo,
+                                              int geo_stride, int geo_ofs, const double* __restrict__ tab, double rho,
+                                              double* __restrict__ out) {
+  extern __shared__ double row[];   // affine: sum_b tab[b][a] per a; else sum_b N_b per point
+  const int nr = affine ? npe : q;
+  for (int i = threadIdx.x; i < nr; i += blockDim.x) {
+    double t = 0.0;
+    for (int b = 0; b < npe; ++b) t += affine ? tab[b * npe + i] : tab[i * npe + b];
+    row[i] = t;
   }
+  __syncthreads();
+  const int64_t j = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kLumpLanes;
+  const int l = threadIdx.x % kLumpLanes;
+  double s = 0.0;
+  if (j < N) {
+    const int32_t k1 = inc_ptr[j + 1];
+    for (int32_t k = inc_ptr[j] + l; k < k1; k += kLumpLanes) {
+      const int64_t e = inc_elem[k];
+      const int a = inc_loc[k];
+      if (affine) {
+        s += geo[(size_t)e * geo_stride + geo_ofs] * row[a];
+      } else {
+        for (int p = 0; p < q; ++p) s += geo[((size_t)e * q + p) * geo_stride + geo_ofs] * (tab[p * npe + a] * row[p]);
+      }
+    }
+  }
+#pragma unroll
+  for (int o = kLumpLanes / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, kLumpLanes);
+  if (j < N && l < 3) out[3 * j + l] = rho * s;
 }
+
+inline unsigned lump_blocks(int64_t N) { return (unsigned)((N * kLumpLanes + 255) / 256); }
 
 }  // namespace
 }  // namespace llfem
