@@ -85,6 +85,7 @@ struct Tune {
 };
 
 struct AmgHier;
+class CopyPool;   // ctx.hip
 
 // A device copy of a reference table, shared by every mesh of a context.
 struct DevTable {
@@ -115,10 +116,11 @@ struct llfem_ctx {
   size_t ws_bytes = 0;
   bool ws_busy = false;
   double* d_sink = nullptr;                        // 64 doubles: target of padding-lane panel stores
-  // pinned staging for large device-to-host copies (copy_to_host)
-  void* h_stage[2] = {nullptr, nullptr};
-  size_t stage_bytes = 0;
-  hipEvent_t stage_ev[2] = {nullptr, nullptr};
+  // pinned staging of device-to-host copies and the threads that empty it
+  // (copy_to_host), made on first use
+  void* h_stage[8] = {};
+  hipEvent_t stage_ev[8] = {};
+  llfem::CopyPool* pool = nullptr;
   // pinned word a running solve sets when it is done, and the events of its
   // two queued batches
   double* h_poll = nullptr;

@@ -4,8 +4,11 @@
 #include "common.h"
 
 #include <algorithm>
+#include <atomic>
+#include <condition_variable>
 #include <cstring>
 #include <thread>
+#include <utility>
 #include <vector>
 
 namespace llfem {
@@ -67,50 +70,173 @@ WsGuard::~WsGuard() {
   if (c_->ws_bytes > kWsKeep) ws_release(c_);
 }
 
-// Large copies go through two pinned staging buffers: the DMA engine fills
-// one while host threads copy the other out to the caller's pageable memory
-// (HIP's own pageable path stages serially through one buffer).
-int copy_to_host(llfem_ctx* ctx, double* dst, const double* src, size_t n) {
-  constexpr size_t kStage = size_t(64) << 20;   // bytes per staging buffer
+// Up to eight threads that empty staging slots into the caller's memory, each
+// its slice of every chunk.  They sleep between copies and belong to one
+// context (whose calls one host thread makes), which joins them.  While a copy
+// runs they spin for the next chunk: it is a few ten microseconds away.
+class CopyPool {
+ public:
+  static constexpr int kSlots = 8;
+  CopyPool() {
+    const unsigned want = std::max(1u, std::min(8u, std::thread::hardware_concurrency()));
+    try {
+      for (unsigned t = 0; t < want; ++t) {
+        th_[n_] = std::thread([this, t] { run((int)t); });
+        ++n_;
+      }
+    } catch (...) {   // fewer threads; none at all: the caller copies
+    }
+  }
+  ~CopyPool() {
+    {
+      std::lock_guard<std::mutex> lk(mu_);
+      quit_ = true;
+    }
+    cv_.notify_all();
+    for (int t = 0; t < n_; ++t) th_[t].join();
+  }
+  int threads() const { return n_; }
+  // A copy of `chunks` chunks, chunk i staged in slot i % kSlots; arrived()
+  // hands one over, wait_free() returns when slot s is empty again, finish()
+  // when every chunk given is copied (abandon: without the others).
+  void begin(size_t chunks) {
+    std::lock_guard<std::mutex> lk(mu_);
+    chunks_ = chunks;
+    ready_.store(0);
+    abandon_.store(false);
+    for (auto& d : left_) d.store(0);
+    active_.store(n_);
+    ++gen_;
+    cv_.notify_all();
+  }
+  void arrived(size_t i, char* dst, const char* src, size_t len) {
+    Part& p = part_[i % kSlots];
+    p.dst = dst;
+    p.src = src;
+    p.len = len;
+    left_[i % kSlots].store(n_);
+    ready_.store(i + 1, std::memory_order_release);
+  }
+  void wait_free(size_t s) {
+    while (left_[s].load(std::memory_order_acquire) > 0) std::this_thread::yield();
+  }
+  void finish(bool abandon) {
+    if (abandon) abandon_.store(true);
+    while (active_.load(std::memory_order_acquire) > 0) std::this_thread::yield();
+  }
+
+ private:
+  struct Part {
+    char* dst;
+    const char* src;
+    size_t len;
+  };
+  void run(int t) {
+    uint64_t seen = 0;
+    for (;;) {
+      {
+        std::unique_lock<std::mutex> lk(mu_);
+        cv_.wait(lk, [&] { return quit_ || gen_ != seen; });
+        if (quit_) return;
+        seen = gen_;
+      }
+      for (size_t i = 0; i < chunks_; ++i) {
+        int spin = 0;
+        while (ready_.load(std::memory_order_acquire) <= i && !abandon_.load(std::memory_order_relaxed))
+          if (++spin > 2000) std::this_thread::yield();
+        if (ready_.load(std::memory_order_acquire) <= i) break;
+        const Part p = part_[i % kSlots];
+        const size_t per = ((p.len + n_ - 1) / n_ + 63) / 64 * 64;
+        const size_t lo = std::min(p.len, t * per), hi = std::min(p.len, lo + per);
+        if (lo < hi) std::memcpy(p.dst + lo, p.src + lo, hi - lo);
+        left_[i % kSlots].fetch_sub(1, std::memory_order_release);
+      }
+      active_.fetch_sub(1, std::memory_order_release);
+    }
+  }
+  std::thread th_[8];
+  int n_ = 0;
+  std::mutex mu_;
+  std::condition_variable cv_;
+  uint64_t gen_ = 0;
+  bool quit_ = false;
+  size_t chunks_ = 0;
+  Part part_[kSlots] = {};
+  std::atomic<size_t> ready_{0};
+  std::atomic<int> left_[kSlots] = {};
+  std::atomic<int> active_{0};
+  std::atomic<bool> abandon_{false};
+};
+
+// Device memory to the caller's pageable memory through pinned staging.  Up
+// to kOneCopy bytes: one copy, emptied by this thread.  Above: chunks through
+// a ring of slots, the device filling some while the pool's threads empty
+// others; large chunks first (each costs the device about 15 us besides its
+// transfer), small ones last (what is left for the threads after the last has
+// arrived).  PCIe bound, 57 GB/s.  HIP's own pageable path takes 18 GB/s:
+//   64 KB 39 -> 11 us, 4 MB 236 -> 120, 50 MB 2.97 -> 1.06 ms, 124 MB 7.4 -> 2.5.
+int copy_to_host(llfem_ctx* ctx, double* dst_, const double* src_, size_t n) {
+  constexpr size_t kOneCopy = size_t(512) << 10, kSmall = size_t(4) << 20, kSlot = size_t(16) << 20;
+  constexpr size_t kSlots = CopyPool::kSlots;
   const size_t bytes = n * sizeof(double);
-  hipStream_t st = ctx->stream;
-  if (bytes <= 2 * kStage) {
-    LLFEM_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st));
-    LLFEM_HIP(hipStreamSynchronize(st));
+  if (bytes == 0) {
+    LLFEM_HIP(hipStreamSynchronize(ctx->stream));
     return LLFEM_OK;
   }
-  if (!ctx->h_stage[0]) {
-    for (int b = 0; b < 2; ++b) {
-      LLFEM_HIP(hipHostMalloc(&ctx->h_stage[b], kStage, hipHostMallocDefault));
-      LLFEM_HIP(hipEventCreateWithFlags(&ctx->stage_ev[b], hipEventDisableTiming));
-    }
-    ctx->stage_bytes = kStage;
-  }
-  const size_t chunk = kStage / sizeof(double);
-  const size_t nchunks = (n + chunk - 1) / chunk;
-  auto issue = [&](size_t i) -> int {
-    const size_t off = i * chunk, len = std::min(chunk, n - off);
-    LLFEM_HIP(hipMemcpyAsync(ctx->h_stage[i & 1], src + off, len * sizeof(double), hipMemcpyDeviceToHost, st));
-    LLFEM_HIP(hipEventRecord(ctx->stage_ev[i & 1], st));
+  hipStream_t st = ctx->stream;
+  char* dst = reinterpret_cast<char*>(dst_);
+  const char* src = reinterpret_cast<const char*>(src_);
+  auto slot = [&](size_t s) -> int {
+    if (ctx->h_stage[s]) return LLFEM_OK;
+    if (!ctx->stage_ev[s]) LLFEM_HIP(hipEventCreateWithFlags(&ctx->stage_ev[s], hipEventDisableTiming));
+    LLFEM_HIP(hipHostMalloc(&ctx->h_stage[s], kSlot, hipHostMallocDefault));
     return LLFEM_OK;
   };
-  LLFEM_TRY(issue(0));
-  if (nchunks > 1) LLFEM_TRY(issue(1));
-  const unsigned nt = std::max(1u, std::min(8u, std::thread::hardware_concurrency()));
-  for (size_t i = 0; i < nchunks; ++i) {
-    LLFEM_HIP(hipEventSynchronize(ctx->stage_ev[i & 1]));
-    const size_t off = i * chunk, len = std::min(chunk, n - off);
-    const double* from = static_cast<const double*>(ctx->h_stage[i & 1]);
-    std::vector<std::thread> th;
-    const size_t per = (len + nt - 1) / nt;
-    for (unsigned t = 0; t < nt; ++t) {
-      const size_t lo = t * per, hi = std::min(len, lo + per);
-      if (lo < hi) th.emplace_back([=] { std::memcpy(dst + off + lo, from + lo, (hi - lo) * sizeof(double)); });
-    }
-    for (auto& x : th) x.join();
-    if (i + 2 < nchunks) LLFEM_TRY(issue(i + 2));
+  LLFEM_TRY(slot(0));
+  if (bytes <= kOneCopy) {
+    LLFEM_HIP(hipMemcpyAsync(ctx->h_stage[0], src, bytes, hipMemcpyDeviceToHost, st));
+    LLFEM_HIP(hipStreamSynchronize(st));
+    std::memcpy(dst, ctx->h_stage[0], bytes);
+    return LLFEM_OK;
   }
-  return LLFEM_OK;
+  std::vector<std::pair<size_t, size_t>> chunk;   // offset, length
+  for (size_t off = 0; off < bytes;) {
+    const size_t left = bytes - off;
+    const size_t len = std::min(left, std::min(kSlot, std::max(kSmall, left / 4 / kSmall * kSmall)));
+    chunk.push_back({off, len});
+    off += len;
+  }
+  auto issue = [&](size_t i) -> int {
+    const size_t s = i % kSlots;
+    LLFEM_TRY(slot(s));
+    LLFEM_HIP(hipMemcpyAsync(ctx->h_stage[s], src + chunk[i].first, chunk[i].second, hipMemcpyDeviceToHost, st));
+    LLFEM_HIP(hipEventRecord(ctx->stage_ev[s], st));
+    return LLFEM_OK;
+  };
+  size_t issued = 0;
+  for (; issued < chunk.size() && issued < kSlots; ++issued) LLFEM_TRY(issue(issued));
+  if (!ctx->pool) ctx->pool = new CopyPool();
+  CopyPool& pool = *ctx->pool;
+  const bool threads = pool.threads() > 0;
+  if (threads) pool.begin(chunk.size());
+  auto drain = [&]() -> int {
+    for (size_t i = 0; i < chunk.size(); ++i) {
+      const size_t s = i % kSlots;
+      LLFEM_HIP(hipEventSynchronize(ctx->stage_ev[s]));
+      if (threads) pool.arrived(i, dst + chunk[i].first, static_cast<const char*>(ctx->h_stage[s]), chunk[i].second);
+      else std::memcpy(dst + chunk[i].first, ctx->h_stage[s], chunk[i].second);
+      // refill the slots emptied meanwhile: the one of the chunk before this one
+      if (i >= 1 && issued < chunk.size()) {
+        if (threads) pool.wait_free(issued % kSlots);
+        LLFEM_TRY(issue(issued));
+        ++issued;
+      }
+    }
+    return LLFEM_OK;
+  };
+  const int rc = drain();
+  if (threads) pool.finish(rc != LLFEM_OK);
+  return rc;
 }
 
 // Content hash for cache keys (not cryptographic): four independent 64-bit
@@ -263,7 +389,8 @@ int llfem_ctx_destroy(llfem_ctx* ctx) {
   if (ctx->h_poll) (void)hipHostFree(ctx->h_poll);
   for (auto& e : ctx->poll_ev)
     if (e) (void)hipEventDestroy(e);
-  for (int b = 0; b < 2; ++b) {
+  delete ctx->pool;
+  for (size_t b = 0; b < sizeof(ctx->h_stage) / sizeof(ctx->h_stage[0]); ++b) {
     if (ctx->h_stage[b]) (void)hipHostFree(ctx->h_stage[b]);
     if (ctx->stage_ev[b]) (void)hipEventDestroy(ctx->stage_ev[b]);
   }

@@ -376,10 +376,7 @@ void complete(llfem_server* S, Req* q) {
   const int status = sys_status(q->sys);
   rc = q->eng->finish(q->sys, q->d_u);
   if (rc == LLFEM_OK) {
-    const int64_t n = 3 * q->cm->m->N;
-    if (hipMemcpyAsync(q->in.u_out, q->d_u, sizeof(double) * n, hipMemcpyDeviceToHost, ctx->stream) != hipSuccess ||
-        hipStreamSynchronize(ctx->stream) != hipSuccess)
-      rc = fail(LLFEM_EHIP, "server: result copy failed");
+    rc = copy_to_host(ctx, q->in.u_out, q->d_u, 3 * (size_t)q->cm->m->N);
   }
   q->iterations = sys_iterations(q->sys);
   q->updates = sys_updates(q->sys);

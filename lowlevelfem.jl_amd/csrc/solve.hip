@@ -779,8 +779,7 @@ int solve_host(llfem_ctx* ctx, const Op& K, const double* val, const float* val3
   auto t0 = std::chrono::steady_clock::now();
   int s = solve_device(ctx, K, val, val32, d_mask, d_f, d_ufix, method, reltol, maxiter, d_u, stats);
   if (s != LLFEM_OK && s != LLFEM_ENOCONV) return s;
-  LLFEM_HIP(hipMemcpyAsync(u_out, d_u, sizeof(double) * n, hipMemcpyDeviceToHost, st));
-  LLFEM_HIP(hipStreamSynchronize(st));
+  LLFEM_TRY(copy_to_host(ctx, u_out, d_u, (size_t)n));
   if (stats)
     stats->total_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
   return s;
@@ -878,8 +877,7 @@ int solve_host_reliable(llfem_ctx* ctx, SysSpec sp, bool f64_vectors, const doub
     LLFEM_TRY(eng.run(chunk, &done));
   }
   LLFEM_TRY(eng.finish(s, d_u));
-  LLFEM_HIP(hipMemcpyAsync(u_out, d_u, sizeof(double) * n, hipMemcpyDeviceToHost, st));
-  LLFEM_HIP(hipStreamSynchronize(st));
+  LLFEM_TRY(copy_to_host(ctx, u_out, d_u, (size_t)n));
   const int status = sys_status(s);
   if (stats) {
     stats->iterations = sys_iterations(s);
