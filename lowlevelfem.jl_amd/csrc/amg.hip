@@ -25,7 +25,7 @@
 // Everything a level needs lives in 3-DoF "pseudo-node" block form: a
 // coarse aggregate's six DoFs are two pseudo-nodes, so every level uses the
 // same block-sparse layout as the fine operator ([slot][c][d] FP32 blocks,
-// node-major adjacency).  The V-cycle kernels run table-driven over all
+// node-major adjacency, block32.h).  The V-cycle kernels run table-driven over all
 // systems of a batch, one launch per kernel and level.
 #include <algorithm>
 #include <atomic>
@@ -39,6 +39,7 @@
 #include <thread>
 #include <vector>
 
+#include "block32.h"
 #include "common.h"
 
 namespace llfem {
@@ -46,12 +47,11 @@ namespace llfem {
 namespace {
 
 constexpr int kMB = 256;                 // threads per block
-constexpr int kMG = 8;                   // lanes per pseudo-node row in the level SpMV
-constexpr int kMSpN = kMB / kMG;         // pseudo-nodes per SpMV block
-// The level SpMV needs no per-block partials, so its grid is not capped (a
-// capped grid-stride version was 6 % slower on the 6.3M-DoF beam); the
+constexpr int kMG = 8;                   // lanes per aggregate in the restriction
+constexpr int kMSpN = kMB / kMG;         // aggregates per restriction block
+// The row kernels (products, block32.h) take one block per kRowNodes rows; the
 // vector and restriction kernels cap their blocks and stride.
-constexpr int64_t kMaxSB = int64_t(1) << 24, kMaxVB = 1024, kMaxAB = 1024;
+constexpr int64_t kMaxVB = 1024, kMaxAB = 1024;
 constexpr int kCheb = 2;                 // Chebyshev degree (pre and post)
 constexpr double kChebLo = 0.1, kChebHi = 1.1;
 constexpr float kOverCorrect = 1.5f;
@@ -84,12 +84,13 @@ struct MgEnt {
   int64_t N;                 // pseudo-nodes of the level (3 DoFs each)
   const int64_t* adj_ptr;
   const int32_t* adj;
-  const float* val;          // [nadj][c][d]
+  int64_t nadj;
+  const float* val;          // block32.h
   const uint8_t* mask;       // [3N] 1 = no DoF (constrained / dropped)
   const float* dinv;         // [3N] inverse diagonal, 0 on masked DoFs
   float* b;                  // right-hand side of the level
-  float* x;                  // iterate of the level
-  float* y;                  // A x
+  float* x;                  // iterate of the level; the smoothing steps alternate
+  float* y;                  // between x and y, and end in x
   float* d;                  // Chebyshev direction
   const int32_t* agg;        // [N] aggregate of each pseudo-node (-1: none)
   const float* Q;            // [N][3][6] tentative prolongator rows
@@ -102,7 +103,7 @@ struct MgEnt {
   int32_t nc;
   float inv_theta, inv_delta;
   const double* state;       // system state word: run only while it reads 0 (NULL: always)
-  double* rzpart;            // level 0: partial r.z of vector block lb at rzpart[2 lb + 1]
+  double* rzpart;            // level 0: partial r.z per row block
   int32_t sblk0, nsblk, vblk0, nvblk, ablk0, nablk;
 };
 
@@ -111,102 +112,76 @@ namespace {
 __device__ __forceinline__ bool mg_skip(const MgEnt& E) { return E.state && *E.state != 0.0; }
 
 
-// y = mask(A x) for every entry's level
-__global__ __launch_bounds__(kMB) void k_mg_spmv(const MgEnt* __restrict__ ents, const int32_t* __restrict__ map) {
-  const MgEnt& E = ents[map[blockIdx.x]];
-  if (mg_skip(E)) return;
-  // local restrict-qualified copies: the output never aliases the inputs
-  const int64_t N = E.N;
-  const auto* __restrict__ adj_ptr = gp(E.adj_ptr);
-  const auto* __restrict__ adj = gp(E.adj);
-  const auto* __restrict__ val = gp(E.val);
-  const auto* __restrict__ x = gp(E.x);
-  const auto* __restrict__ mask = gp(E.mask);
-  auto* __restrict__ y = gp(E.y);
-  const int lb = blockIdx.x - E.sblk0;
-  const int nsblk = E.nsblk;
-  const int l = threadIdx.x % kMG;
-  for (int64_t j = (int64_t)lb * kMSpN + threadIdx.x / kMG; j - threadIdx.x / kMG < N;
-       j += (int64_t)nsblk * kMSpN) {
-    float a0 = 0.f, a1 = 0.f, a2 = 0.f;
-    if (j < N) {
-      const int64_t p0 = adj_ptr[j];
-      const int R = (int)(adj_ptr[j + 1] - p0);
-      const auto* P = val + 9 * p0;
-#pragma unroll 2
-      for (int t = l; t < R; t += kMG) {
-        const int64_t i = adj[p0 + t];
-        const float x0 = x[3 * i], x1 = x[3 * i + 1], x2 = x[3 * i + 2];
-        const auto* B = P + 9 * t;
-        a0 += B[0] * x0 + B[1] * x1 + B[2] * x2;
-        a1 += B[3] * x0 + B[4] * x1 + B[5] * x2;
-        a2 += B[6] * x0 + B[7] * x1 + B[8] * x2;
-      }
-    }
-#pragma unroll
-    for (int o = kMG / 2; o > 0; o >>= 1) {
-      a0 += __shfl_xor(a0, o, kMG);
-      a1 += __shfl_xor(a1, o, kMG);
-      a2 += __shfl_xor(a2, o, kMG);
-    }
-    if (j < N && l == 0) {
-      y[3 * j] = mask[3 * j] ? 0.f : a0;
-      y[3 * j + 1] = mask[3 * j + 1] ? 0.f : a1;
-      y[3 * j + 2] = mask[3 * j + 2] ? 0.f : a2;
-    }
-  }
-}
-
-// first Chebyshev step from x = 0: x = d = D^-1 b / theta
+// first Chebyshev step from x = 0: y = d = D^-1 b / theta
 __global__ __launch_bounds__(kMB) void k_mg_cheb0(const MgEnt* __restrict__ ents, const int32_t* __restrict__ map) {
   const MgEnt& E = ents[map[blockIdx.x]];
   if (mg_skip(E)) return;
   const int lb = blockIdx.x - E.vblk0;
   const float* __restrict__ dinv = (const float*)gp(E.dinv);
   const float* __restrict__ b = (const float*)gp(E.b);
-  float* __restrict__ x = (float*)gp(E.x);
+  float* __restrict__ y = (float*)gp(E.y);
   float* __restrict__ d = (float*)gp(E.d);
   const float it = E.inv_theta;
   for (int64_t i = (int64_t)lb * kMB + threadIdx.x; i < 3 * E.N; i += (int64_t)E.nvblk * kMB) {
     const float v = it * dinv[i] * b[i];
-    x[i] = v;
+    y[i] = v;
     d[i] = v;
   }
 }
 
-// Chebyshev step: d = ca d + (cbt / theta + cbd / delta) D^-1 (b - y); x += d.
-// With rz set (level 0, last step): partial b.x of the block (b = r, x = z).
-__global__ __launch_bounds__(kMB) void k_mg_cheb(const MgEnt* __restrict__ ents, const int32_t* __restrict__ map,
-                                                 float ca, float cbt, float cbd, int rz) {
-  __shared__ double sh[kMB];
+// Chebyshev step: d = ca d + (cbt / theta + cbd / delta) D^-1 (b - A u),
+// w = u + d, with u, w = y, x (from_y) or x, y.  D^-1 is 0 on masked DoFs.
+// The product's block applies the step to its own rows, so neither A u nor a
+// second launch for the vectors is needed: 3 launches a level and a pass over
+// the vectors less.  With block32.h's layout, a solve of 2.1 M nodes (92
+// iterations) 413 -> 376 ms, eight systems on a server 55.8 -> 51.6 ms.  w is
+// another array than u because other blocks still read u.  rz (level 0, last
+// step): partial b.w per block.
+__global__ __launch_bounds__(kRowThreads) void k_mg_smooth(const MgEnt* __restrict__ ents,
+                                                           const int32_t* __restrict__ map, float ca, float cbt,
+                                                           float cbd, int from_y, int rz) {
+  __shared__ float sh[3 * kRowNodes];
   const MgEnt& E = ents[map[blockIdx.x]];
   if (mg_skip(E)) return;
-  const int lb = blockIdx.x - E.vblk0;
-  const float cb = cbt * E.inv_theta + cbd * E.inv_delta;
-  const float* __restrict__ b = (const float*)gp(E.b);
-  const float* __restrict__ y = (const float*)gp(E.y);
-  const float* __restrict__ dinv = (const float*)gp(E.dinv);
-  float* __restrict__ d = (float*)gp(E.d);
-  float* __restrict__ x = (float*)gp(E.x);
-  const int64_t n = 3 * E.N;
+  const int lb = blockIdx.x - E.sblk0;
+  const auto* __restrict__ u = gp((const float*)(from_y ? E.y : E.x));
+  block_rows<float>(E.N, E.nadj, gp(E.adj_ptr), gp(E.adj), gp(E.val), u, lb, sh);
+  if (threadIdx.x >= 64) return;
+  const int64_t i = (int64_t)lb * 3 * kRowNodes + threadIdx.x;
   double acc = 0.0;
-  for (int64_t i = (int64_t)lb * kMB + threadIdx.x; i < n; i += (int64_t)E.nvblk * kMB) {
-    const float bi = b[i];
-    const float dv = ca * d[i] + cb * dinv[i] * (bi - y[i]);
-    const float xv = x[i] + dv;
-    d[i] = dv;
-    x[i] = xv;
-    acc += (double)bi * (double)xv;
+  if (threadIdx.x < 3 * kRowNodes && i < 3 * E.N) {
+    const float cb = cbt * E.inv_theta + cbd * E.inv_delta;
+    const float bi = gp(E.b)[i];
+    const float dv = ca * gp(E.d)[i] + cb * gp(E.dinv)[i] * (bi - sh[threadIdx.x]);
+    const float wv = u[i] + dv;
+    gp(E.d)[i] = dv;
+    gp(from_y ? E.x : E.y)[i] = wv;
+    acc = (double)bi * (double)wv;
   }
   if (rz) {
-    acc = msum(acc, sh);
-    if (threadIdx.x == 0) ((double*)gp(E.rzpart))[2 * lb + 1] = acc;
+    acc = wave_sum(acc);
+    if (threadIdx.x == 0) gp(E.rzpart)[lb] = acc;
   }
 }
 
-// bc = Q^T (b - y): kMG lanes per aggregate stride over its members, then a
-// fixed shuffle tree sums the lanes.
-__global__ __launch_bounds__(kMB) void k_mg_restrict(const MgEnt* __restrict__ ents, const int32_t* __restrict__ map) {
+// residual of the level, w = mask(b - A u): u, w = y, x (from_y) or x, y
+__global__ __launch_bounds__(kRowThreads) void k_mg_resid(const MgEnt* __restrict__ ents,
+                                                          const int32_t* __restrict__ map, int from_y) {
+  __shared__ float sh[3 * kRowNodes];
+  const MgEnt& E = ents[map[blockIdx.x]];
+  if (mg_skip(E)) return;
+  const int lb = blockIdx.x - E.sblk0;
+  const auto* __restrict__ u = gp((const float*)(from_y ? E.y : E.x));
+  block_rows<float>(E.N, E.nadj, gp(E.adj_ptr), gp(E.adj), gp(E.val), u, lb, sh);
+  const int64_t i = (int64_t)lb * 3 * kRowNodes + threadIdx.x;
+  if (threadIdx.x < 3 * kRowNodes && i < 3 * E.N)
+    gp(from_y ? E.x : E.y)[i] = gp(E.mask)[i] ? 0.f : gp(E.b)[i] - sh[threadIdx.x];
+}
+
+// bc = Q^T r, r in y (in_y) or x: kMG lanes per aggregate stride over its
+// members, then a fixed shuffle tree sums the lanes.
+__global__ __launch_bounds__(kMB) void k_mg_restrict(const MgEnt* __restrict__ ents, const int32_t* __restrict__ map,
+                                                     int in_y) {
   const MgEnt& E = ents[map[blockIdx.x]];
   if (mg_skip(E)) return;
   const int lb = blockIdx.x - E.ablk0;
@@ -214,8 +189,7 @@ __global__ __launch_bounds__(kMB) void k_mg_restrict(const MgEnt* __restrict__ e
   const int32_t* __restrict__ mem_ptr = (const int32_t*)gp(E.mem_ptr);
   const int32_t* __restrict__ mem = (const int32_t*)gp(E.mem);
   const float* __restrict__ Q = (const float*)gp(E.Q);
-  const float* __restrict__ b = (const float*)gp(E.b);
-  const float* __restrict__ y = (const float*)gp(E.y);
+  const float* __restrict__ rv = (const float*)gp(in_y ? E.y : E.x);
   float* __restrict__ bc = (float*)gp(E.bc);
   for (int64_t a = (int64_t)lb * kMSpN + threadIdx.x / kMG; a - threadIdx.x / kMG < E.nagg;
        a += (int64_t)E.nablk * kMSpN) {
@@ -226,7 +200,7 @@ __global__ __launch_bounds__(kMB) void k_mg_restrict(const MgEnt* __restrict__ e
         const float* Qj = Q + 18 * j;
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
-          const float r = b[3 * j + c] - y[3 * j + c];
+          const float r = rv[3 * j + c];
 #pragma unroll
           for (int u = 0; u < 6; ++u) acc[u] += Qj[6 * c + u] * r;
         }
@@ -242,16 +216,16 @@ __global__ __launch_bounds__(kMB) void k_mg_restrict(const MgEnt* __restrict__ e
   }
 }
 
-// x += alpha Q xc
+// u += alpha Q xc, u = y (in_y) or x
 __global__ __launch_bounds__(kMB) void k_mg_prolong(const MgEnt* __restrict__ ents, const int32_t* __restrict__ map,
-                                                    float alpha) {
+                                                    float alpha, int in_y) {
   const MgEnt& E = ents[map[blockIdx.x]];
   if (mg_skip(E)) return;
   const int lb = blockIdx.x - E.vblk0;
   const int32_t* __restrict__ agg = (const int32_t*)gp(E.agg);
   const float* __restrict__ Q = (const float*)gp(E.Q);
   const float* __restrict__ xcv = (const float*)gp(E.xc);
-  float* __restrict__ x = (float*)gp(E.x);
+  float* __restrict__ x = (float*)gp(in_y ? E.y : E.x);
   for (int64_t j = (int64_t)lb * kMB + threadIdx.x; j < E.N; j += (int64_t)E.nvblk * kMB) {
     const int32_t a = agg[j];
     if (a < 0) continue;
@@ -289,7 +263,8 @@ __global__ __launch_bounds__(kMB) void k_mg_coarse(const MgEnt* __restrict__ ent
 // ---- per-request numeric set-up -------------------------------------------------
 
 // Galerkin product: thread per (coarse aggregate pair p, coarse row u).
-__global__ __launch_bounds__(kMB) void k_galerkin(int64_t npairs, const int64_t* __restrict__ gptr,
+__global__ __launch_bounds__(kMB) void k_galerkin(int64_t npairs, int64_t nadjf, int64_t nadjc,
+                                                  const int64_t* __restrict__ gptr,
                                                   const int32_t* __restrict__ gblk, const int32_t* __restrict__ gcol,
                                                   const int32_t* __restrict__ adjf, const float* __restrict__ Qf,
                                                   const float* __restrict__ valf, const int32_t* __restrict__ pair_o,
@@ -303,7 +278,8 @@ __global__ __launch_bounds__(kMB) void k_galerkin(int64_t npairs, const int64_t*
     const int64_t g = gblk[c];
     const int64_t j = gcol[c];
     const int64_t i = adjf[g];
-    const float* B = valf + 9 * g;      // B[3c+d] = A[(j,c),(i,d)]
+    const f4v ba = reinterpret_cast<const f4v*>(valf)[g], bb = reinterpret_cast<const f4v*>(valf + 4 * nadjf)[g];
+    const float B[9] = {ba.x, ba.y, ba.z, ba.w, bb.x, bb.y, bb.z, bb.w, valf[8 * nadjf + g]};   // [3c+d] = A[(j,c),(i,d)]
     const float* Qj = Qf + 18 * j;
     const float* Qi = Qf + 18 * i;
     const double q0 = Qj[u], q1 = Qj[6 + u], q2 = Qj[12 + u];
@@ -316,17 +292,18 @@ __global__ __launch_bounds__(kMB) void k_galerkin(int64_t npairs, const int64_t*
   const int s = u / 3, cc = u % 3;
   const int64_t o = pair_o[2 * p + s];
 #pragma unroll
-  for (int v = 0; v < 6; ++v) valc[9 * (o + v / 3) + 3 * cc + v % 3] = (float)acc[v];
+  for (int v = 0; v < 6; ++v) valc[block32_at(nadjc, o + v / 3, 3 * cc + v % 3)] = (float)acc[v];
 }
 
-__global__ void k_mg_dinv(int64_t N, const int64_t* __restrict__ adj_ptr, const int32_t* __restrict__ dslot,
+__global__ void k_mg_dinv(int64_t N, int64_t nadj, const int64_t* __restrict__ adj_ptr,
+                          const int32_t* __restrict__ dslot,
                           const float* __restrict__ val, const uint8_t* __restrict__ mask, float* __restrict__ dinv) {
   const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (j >= N) return;
-  const float* B = val + 9 * (adj_ptr[j] + dslot[j]);
+  const int64_t g = adj_ptr[j] + dslot[j];
 #pragma unroll
   for (int d = 0; d < 3; ++d) {
-    const float v = B[4 * d];
+    const float v = val[block32_at(nadj, g, 4 * d)];
     dinv[3 * j + d] = (mask[3 * j + d] || !(v > 0.f)) ? 0.f : 1.f / v;
   }
 }
@@ -341,42 +318,18 @@ __global__ void k_mg_rand(int64_t n, const float* __restrict__ dinv, float* __re
   v[i] = dinv[i] > 0.f ? (float)(h & 0xFFFFu) / 65536.f - 0.5f : 0.f;
 }
 
-__global__ __launch_bounds__(kMB) void k_mg_spmv1(int64_t N, const int64_t* __restrict__ adj_ptr,
-                                                  const int32_t* __restrict__ adj, const float* __restrict__ val,
-                                                  const uint8_t* __restrict__ mask, const float* __restrict__ x,
-                                                  float* __restrict__ y) {
-  const int64_t gt = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t j = gt / kMG;
-  const int l = (int)(gt % kMG);
-  float a0 = 0.f, a1 = 0.f, a2 = 0.f;
-  if (j < N) {
-    const int64_t p0 = adj_ptr[j];
-    const int R = (int)(adj_ptr[j + 1] - p0);
-    for (int t = l; t < R; t += kMG) {
-      const int64_t i = adj[p0 + t];
-      const float* B = val + 9 * (p0 + t);
-      a0 += B[0] * x[3 * i] + B[1] * x[3 * i + 1] + B[2] * x[3 * i + 2];
-      a1 += B[3] * x[3 * i] + B[4] * x[3 * i + 1] + B[5] * x[3 * i + 2];
-      a2 += B[6] * x[3 * i] + B[7] * x[3 * i + 1] + B[8] * x[3 * i + 2];
-    }
-  }
-#pragma unroll
-  for (int o = kMG / 2; o > 0; o >>= 1) {
-    a0 += __shfl_xor(a0, o, kMG);
-    a1 += __shfl_xor(a1, o, kMG);
-    a2 += __shfl_xor(a2, o, kMG);
-  }
-  if (j < N && l == 0) {
-    y[3 * j] = mask[3 * j] ? 0.f : a0;
-    y[3 * j + 1] = mask[3 * j + 1] ? 0.f : a1;
-    y[3 * j + 2] = mask[3 * j + 2] ? 0.f : a2;
-  }
-}
-
-__global__ void k_mg_dscale(int64_t n, const float* __restrict__ dinv, const float* __restrict__ y,
-                            float* __restrict__ v) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) v[i] = dinv[i] * y[i];
+// y = mask(A x), or with dinv D^-1 A x (one power step)
+__global__ __launch_bounds__(kRowThreads) void k_mg_spmv1(int64_t N, int64_t nadj, const int64_t* __restrict__ adj_ptr,
+                                                          const int32_t* __restrict__ adj,
+                                                          const float* __restrict__ val,
+                                                          const uint8_t* __restrict__ mask,
+                                                          const float* __restrict__ dinv,
+                                                          const float* __restrict__ x, float* __restrict__ y) {
+  __shared__ float sh[3 * kRowNodes];
+  block_rows<float>(N, nadj, adj_ptr, adj, gp(val), x, blockIdx.x, sh);
+  const int64_t i = (int64_t)blockIdx.x * 3 * kRowNodes + threadIdx.x;
+  if (threadIdx.x < 3 * kRowNodes && i < 3 * N)
+    y[i] = dinv ? dinv[i] * sh[threadIdx.x] : mask[i] ? 0.f : sh[threadIdx.x];
 }
 
 // partial (v.y, v.D v) per block
@@ -1189,27 +1142,32 @@ int run_vcycle(llfem_ctx* ctx, const std::vector<AmgSys::Tab>& T) {
   static thread_local std::vector<ChebCoef> pre, post;
   if (post.empty()) cheb_coefs(pre, post);
   const int L = (int)T.size();
+  // the iterate starts in y and changes array with each of the 2 kCheb - 1
+  // (odd) smoothing steps, so it ends in x
+  static_assert((2 * kCheb - 1) % 2 == 1, "the V-cycle's result has to end in x");
   for (int l = 0; l < L; ++l) {
     const AmgSys::Tab& t = T[l];
     if (t.nent) {
+      int in_y = 1;
       k_mg_cheb0<<<(unsigned)t.nvb, kMB, 0, st>>>(t.ents, t.vmap);
       for (const ChebCoef& c : pre) {
-        k_mg_spmv<<<(unsigned)t.nsb, kMB, 0, st>>>(t.ents, t.smap);
-        k_mg_cheb<<<(unsigned)t.nvb, kMB, 0, st>>>(t.ents, t.vmap, c.ca, c.cbt, c.cbd, 0);
+        k_mg_smooth<<<(unsigned)t.nsb, kRowThreads, 0, st>>>(t.ents, t.smap, c.ca, c.cbt, c.cbd, in_y, 0);
+        in_y ^= 1;
       }
-      k_mg_spmv<<<(unsigned)t.nsb, kMB, 0, st>>>(t.ents, t.smap);
-      k_mg_restrict<<<(unsigned)t.nab, kMB, 0, st>>>(t.ents, t.amap);
+      k_mg_resid<<<(unsigned)t.nsb, kRowThreads, 0, st>>>(t.ents, t.smap, in_y);
+      k_mg_restrict<<<(unsigned)t.nab, kMB, 0, st>>>(t.ents, t.amap, in_y ^ 1);
     }
     if (t.ncent) k_mg_coarse<<<(unsigned)t.ncent, kMB, 0, st>>>(t.cents);
   }
   for (int l = L - 1; l >= 0; --l) {
     const AmgSys::Tab& t = T[l];
     if (!t.nent) continue;
-    k_mg_prolong<<<(unsigned)t.nvb, kMB, 0, st>>>(t.ents, t.vmap, kOverCorrect);
+    int in_y = (int)((pre.size() + 1) % 2);
+    k_mg_prolong<<<(unsigned)t.nvb, kMB, 0, st>>>(t.ents, t.vmap, kOverCorrect, in_y);
     for (size_t s = 0; s < post.size(); ++s) {
-      k_mg_spmv<<<(unsigned)t.nsb, kMB, 0, st>>>(t.ents, t.smap);
-      k_mg_cheb<<<(unsigned)t.nvb, kMB, 0, st>>>(t.ents, t.vmap, post[s].ca, post[s].cbt, post[s].cbd,
-                                                  (l == 0 && s + 1 == post.size()) ? 1 : 0);
+      k_mg_smooth<<<(unsigned)t.nsb, kRowThreads, 0, st>>>(t.ents, t.smap, post[s].ca, post[s].cbt, post[s].cbd, in_y,
+                                                           (l == 0 && s + 1 == post.size()) ? 1 : 0);
+      in_y ^= 1;
     }
   }
   LLFEM_HIP(hipGetLastError());
@@ -1264,7 +1222,7 @@ void amg_sys_free(llfem_ctx* ctx, AmgSys* s) {
 // Chebyshev bounds, dense coarsest inverse, launch tables for restarts.
 // r, z, q: the system's FP32 residual, preconditioned residual and a free
 // work vector (level 0's b, x and y); rzpart: where level 0 leaves the
-// partial r.z per vector block (vector blocks as the engine's update kernel).
+// partial r.z per row block (row_groups(N) of them, as the engine's product).
 int amg_sys_create(llfem_ctx* ctx, const AmgHier* h, const float* val32, float* r, float* z, float* q,
                    double* rzpart, AmgSys** out) {
   hipStream_t st = ctx->stream;
@@ -1301,6 +1259,7 @@ int amg_sys_create(llfem_ctx* ctx, const AmgHier* h, const float* val32, float* 
     e.N = D.N;
     e.adj_ptr = D.adj_ptr;
     e.adj = D.adj;
+    e.nadj = D.nadj;
     e.mask = D.mask;
     if (l == 0) {
       dinv[0] = (float*)take(4 * 3 * (size_t)D.N);
@@ -1318,10 +1277,8 @@ int amg_sys_create(llfem_ctx* ctx, const AmgHier* h, const float* val32, float* 
     }
     e.val = val[l];
     e.dinv = dinv[l];
-    e.nsblk = (int32_t)cap(D.N, kMSpN, kMaxSB);
-    // level 0 uses the engine's vector blocks (256 nodes, at most 1024 blocks),
-    // so its r.z partials line up with the engine's r.r partials
-    e.nvblk = (int32_t)(l == 0 ? cap(D.N, kMB, kMaxVB) : cap(3 * D.N, kMB, kMaxVB));
+    e.nsblk = (int32_t)row_groups(D.N);   // as the engine's product
+    e.nvblk = (int32_t)cap(3 * D.N, kMB, kMaxVB);
     e.agg = D.agg;
     e.Q = D.Q;
     e.mem_ptr = D.mem_ptr;
@@ -1344,12 +1301,12 @@ int amg_sys_create(llfem_ctx* ctx, const AmgHier* h, const float* val32, float* 
   // Galerkin operators, inverse diagonals
   for (int l = 0; l < L; ++l) {
     const auto& D = h->lev[l];
-    k_galerkin<<<nblk(6 * D.npairs), kMB, 0, st>>>(D.npairs, D.gptr, D.gblk, D.gcol, D.adj, D.Q, val[l], D.pair_o,
-                                                  val[l + 1]);
+    k_galerkin<<<nblk(6 * D.npairs), kMB, 0, st>>>(D.npairs, D.nadj, h->lev[l + 1].nadj, D.gptr, D.gblk, D.gcol, D.adj,
+                                                  D.Q, val[l], D.pair_o, val[l + 1]);
   }
   for (int l = 0; l <= L; ++l) {
     const auto& D = h->lev[l];
-    k_mg_dinv<<<nblk(D.N), kMB, 0, st>>>(D.N, D.adj_ptr, D.dslot, val[l], D.mask, dinv[l]);
+    k_mg_dinv<<<nblk(D.N), kMB, 0, st>>>(D.N, D.nadj, D.adj_ptr, D.dslot, val[l], D.mask, dinv[l]);
   }
   // largest eigenvalue of D^-1 A per smoothed level (power steps, Rayleigh quotient)
   for (int l = 0; l < L; ++l) {
@@ -1359,11 +1316,13 @@ int amg_sys_create(llfem_ctx* ctx, const AmgHier* h, const float* val32, float* 
     float* v = e.d;
     float* y = e.y;
     k_mg_rand<<<nblk(n), kMB, 0, st>>>(n, dinv[l], v);
-    for (int k = 0; k < kPowerSteps; ++k) {
-      k_mg_spmv1<<<nblk(D.N * kMG), kMB, 0, st>>>(D.N, D.adj_ptr, D.adj, val[l], D.mask, v, y);
-      k_mg_dscale<<<nblk(n), kMB, 0, st>>>(n, dinv[l], y, v);
+    for (int k = 0; k < kPowerSteps; ++k) {   // D^-1 A, back and forth between the two arrays
+      k_mg_spmv1<<<(unsigned)row_groups(D.N), kRowThreads, 0, st>>>(D.N, D.nadj, D.adj_ptr, D.adj, val[l], D.mask,
+                                                                    dinv[l], v, y);
+      std::swap(v, y);
     }
-    k_mg_spmv1<<<nblk(D.N * kMG), kMB, 0, st>>>(D.N, D.adj_ptr, D.adj, val[l], D.mask, v, y);
+    k_mg_spmv1<<<(unsigned)row_groups(D.N), kRowThreads, 0, st>>>(D.N, D.nadj, D.adj_ptr, D.adj, val[l], D.mask,
+                                                                  nullptr, v, y);
     k_mg_rq<<<nblk(n), kMB, 0, st>>>(n, v, y, dinv[l], part);
     k_mg_sum2<<<1, kMB, 0, st>>>(nblk(n), part, lam + 2 * l);
   }
@@ -1395,7 +1354,8 @@ int amg_sys_create(llfem_ctx* ctx, const AmgHier* h, const float* val32, float* 
       for (int64_t g = h->c_adj_ptr[j]; g < h->c_adj_ptr[j + 1]; ++g) {
         const int64_t i = h->c_adj[g];
         for (int c = 0; c < 3; ++c)
-          for (int d = 0; d < 3; ++d) A[(size_t)(3 * j + c) * n + 3 * i + d] = cval[9 * g + 3 * c + d];
+          for (int d = 0; d < 3; ++d)
+            A[(size_t)(3 * j + c) * n + 3 * i + d] = cval[block32_at(h->lev[L].nadj, g, 3 * c + d)];
       }
     std::vector<uint8_t> dead(n, 0);
     for (int i = 0; i < n; ++i) dead[i] = h->c_mask[i] || !(A[(size_t)i * n + i] > 0.0);
@@ -1456,6 +1416,8 @@ int amg_batch_apply(llfem_ctx* ctx, AmgBatch* b) {
   if (!b || b->tab.empty()) return LLFEM_OK;
   return run_vcycle(ctx, b->tab);
 }
+
+bool amg_batch_any(const AmgBatch* b) { return b && !b->tab.empty(); }
 
 void amg_batch_free(llfem_ctx* ctx, AmgBatch* b) {
   if (!b) return;

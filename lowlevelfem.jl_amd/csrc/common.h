@@ -317,6 +317,7 @@ class BatchSolver {
   hipGraphExec_t chunk_exec_ = nullptr;
   int chunk_iters_ = 0;
   bool f64v_;
+  bool fold_ = false;                // some live system's product partials need folding
   std::vector<SolveSys*> sys_, live_;
   bool dirty_ = true;
   void* tables_ = nullptr;
@@ -352,6 +353,7 @@ int amg_apply_solo(llfem_ctx* ctx, AmgSys* s);
 int amg_batch_build(llfem_ctx* ctx, const std::vector<AmgSys*>& sys, const std::vector<const double*>& states,
                     AmgBatch** b);
 int amg_batch_apply(llfem_ctx* ctx, AmgBatch* b);
+bool amg_batch_any(const AmgBatch* b);
 void amg_batch_free(llfem_ctx* ctx, AmgBatch* b);
 // One-call hierarchy build for a system (gather + host build + upload).
 int amg_build(llfem_ctx* ctx, const SysSpec& sp, const double* d_xyz, AmgHier** out);

@@ -33,6 +33,7 @@
 #include <cstring>
 #include <vector>
 
+#include "block32.h"
 #include "common.h"
 #include "engine_policy.h"
 
@@ -41,13 +42,18 @@ namespace llfem {
 namespace {
 
 constexpr int kSB = 256;                 // threads per block
-constexpr int kSG = 8;                   // lanes per node row in the SpMV
-constexpr int kSpmvNodes = kSB / kSG;    // nodes per SpMV block
+constexpr int kSG = 8;                   // lanes per node row in the FP64 product of an update
 constexpr int kVecNodes = kSB;           // nodes per vector block pass
-// Blocks per system are capped (the blocks stride over the system's nodes),
-// so the per-system reductions sum at most a few thousand partials.
-constexpr int64_t kMaxSpmvBlocks = 2048;
+// Vector blocks per system are capped (they stride over the system's nodes).
+// The product's are not: 2,048 striding blocks of 8 lanes a row over 36-byte
+// records took 627 us at 2.1 M nodes (tet10, 59.5 M blocks), one block per 16
+// rows of block32.h's layout 515 us (4.6 TB/s).  Its partials lie in y, which
+// is free between updates; more than kFoldMax of them (8 per thread of a
+// summing block) are summed by kFoldBlocks blocks first, a 6 us launch that a
+// smaller system does not need.
 constexpr int64_t kMaxVecBlocks = 1024;
+constexpr int64_t kFoldMax = 2048;
+constexpr int kFoldBlocks = 64;
 
 // scal words of a system; SC_LAST: iteration count at the last FP64 update,
 // SC_MAXRUN: force an update after this many iterations (0: never)
@@ -59,14 +65,16 @@ struct SysDev {
   int64_t N;               // nodes (3 DoFs each)
   const int64_t* adj_ptr;
   const int32_t* adj;
-  const float* val;        // FP32 node blocks, block-contiguous: [adj slot][c][d]
+  int64_t nadj;
+  const float* val;        // FP32 node blocks (block32.h)
   const uint8_t* fixed;    // [3N] 1 = constrained
-  const float* binv;       // [N][9] inverse diagonal blocks (free part)
+  const float* dinv;       // [N][3] inverse diagonal (0 on constrained DoFs)
   void *x, *r, *z, *p, *q; // Krylov vectors, FP32 or FP64 (the kernels' VT)
   double* scal;            // [SC_N]
-  double* part;            // [nsblk] SpMV partials, then [2 * nvblk]
+  double* spart;           // [nsblk] partials of a product, then [kFoldBlocks] sums of them if nsblk > kFoldMax
+  double* part;            // [nvblk][2] (r.r, r.z) of a vector kernel
   int32_t sblk0, nsblk, vblk0, nvblk;
-  int32_t amg;             // 1: z and the r.z partials come from the AMG V-cycle
+  int32_t amg;             // 1: z and the r.z partials (in spart) come from the AMG V-cycle
 };
 
 __device__ __forceinline__ double bsum(double v, double* sh) {
@@ -84,54 +92,46 @@ __device__ __forceinline__ double bsum(double v, double* sh) {
 
 // q = mask(K32 p) for RUNNING systems; partial p.q per block.
 template <typename VT>
-__global__ __launch_bounds__(kSB) void k_bs_spmv(const SysDev* __restrict__ sys, const int32_t* __restrict__ bsys) {
-  __shared__ double sh[kSB];
+__global__ __launch_bounds__(kRowThreads) void k_bs_spmv(const SysDev* __restrict__ sys,
+                                                         const int32_t* __restrict__ bsys) {
+  __shared__ VT sh[3 * kRowNodes];
   const SysDev& S = sys[bsys[blockIdx.x]];
   if (S.scal[SC_STATE] != ST_RUN) return;   // block-uniform
-  const VT* __restrict__ pv = (const VT*)gp(static_cast<const VT*>(S.p));
-  VT* __restrict__ qv = (VT*)gp(static_cast<VT*>(S.q));
-  const int64_t* __restrict__ adj_ptr = (const int64_t*)gp(S.adj_ptr);
-  const int32_t* __restrict__ adj = (const int32_t*)gp(S.adj);
-  const float* __restrict__ val = (const float*)gp(S.val);
-  const uint8_t* __restrict__ fixed = (const uint8_t*)gp(S.fixed);
+  const auto* __restrict__ pv = gp(static_cast<const VT*>(S.p));
   const int lb = blockIdx.x - S.sblk0;
-  const int l = threadIdx.x % kSG;
+  block_rows<VT>(S.N, S.nadj, gp(S.adj_ptr), gp(S.adj), gp(S.val), pv, lb, sh);
+  if (threadIdx.x >= 64) return;
+  const int64_t i = (int64_t)lb * 3 * kRowNodes + threadIdx.x;
   double d = 0.0;
-  for (int64_t j = (int64_t)lb * kSpmvNodes + threadIdx.x / kSG; j - threadIdx.x / kSG < S.N;
-       j += (int64_t)S.nsblk * kSpmvNodes) {
-  VT a0 = 0, a1 = 0, a2 = 0;
-  if (j < S.N) {
-    const int64_t p0 = adj_ptr[j];
-    const int R = (int)(adj_ptr[j + 1] - p0);
-    const float* P = val + 9 * p0;
-#pragma unroll 2
-    for (int t = l; t < R; t += kSG) {
-      const int64_t i = adj[p0 + t];
-      const VT x0 = pv[3 * i], x1 = pv[3 * i + 1], x2 = pv[3 * i + 2];
-      const float* B = P + 9 * t;   // block t: [c][d], 36 contiguous bytes
-      a0 += (VT)B[0] * x0 + (VT)B[1] * x1 + (VT)B[2] * x2;
-      a1 += (VT)B[3] * x0 + (VT)B[4] * x1 + (VT)B[5] * x2;
-      a2 += (VT)B[6] * x0 + (VT)B[7] * x1 + (VT)B[8] * x2;
-    }
+  if (threadIdx.x < 3 * kRowNodes && i < 3 * S.N) {
+    const VT v = gp(S.fixed)[i] ? (VT)0 : sh[threadIdx.x];
+    gp(static_cast<VT*>(S.q))[i] = v;
+    d = (double)pv[i] * (double)v;
   }
-#pragma unroll
-  for (int o = kSG / 2; o > 0; o >>= 1) {
-    a0 += __shfl_xor(a0, o, kSG);
-    a1 += __shfl_xor(a1, o, kSG);
-    a2 += __shfl_xor(a2, o, kSG);
-  }
-  if (j < S.N && l == 0) {
-    const VT a[3] = {a0, a1, a2};
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-      const VT v = fixed[3 * j + c] ? (VT)0 : a[c];
-      qv[3 * j + c] = v;
-      d += (double)pv[3 * j + c] * (double)v;
-    }
-  }
-  }
-  d = bsum(d, sh);
-  if (threadIdx.x == 0) S.part[lb] = d;
+  d = wave_sum(d);
+  if (threadIdx.x == 0) S.spart[lb] = d;
+}
+
+// spart of systems with more than kFoldMax product blocks -> kFoldBlocks sums
+// of contiguous runs, behind them.  kFoldBlocks blocks per system.
+__global__ __launch_bounds__(kSB) void k_bs_fold(const SysDev* __restrict__ sys) {
+  __shared__ double sh[kSB];
+  const SysDev& S = sys[blockIdx.x / kFoldBlocks];
+  if (S.nsblk <= kFoldMax || S.scal[SC_STATE] != ST_RUN) return;
+  const int b = blockIdx.x % kFoldBlocks;
+  const int per = (S.nsblk + kFoldBlocks - 1) / kFoldBlocks, i1 = min(S.nsblk, (b + 1) * per);
+  double v = 0.0;
+  for (int i = b * per + threadIdx.x; i < i1; i += kSB) v += S.spart[i];
+  v = bsum(v, sh);
+  if (threadIdx.x == 0) S.spart[S.nsblk + b] = v;
+}
+
+__device__ __forceinline__ double sum_spart(const SysDev& S, double* sh) {
+  const double* q = S.spart + (S.nsblk > kFoldMax ? S.nsblk : 0);
+  const int n = S.nsblk > kFoldMax ? kFoldBlocks : S.nsblk;
+  double v = 0.0;
+  for (int i = threadIdx.x; i < n; i += kSB) v += q[i];
+  return bsum(v, sh);
 }
 
 // alpha = rho / p.q (one block per system).  A system flagged PENDING at the
@@ -145,9 +145,7 @@ __global__ __launch_bounds__(kSB) void k_bs_alpha(const SysDev* __restrict__ sys
     return;
   }
   if (st != ST_RUN) return;
-  double v = 0.0;
-  for (int i = threadIdx.x; i < S.nsblk; i += kSB) v += S.part[i];
-  v = bsum(v, sh);
+  const double v = sum_spart(S, sh);
   if (threadIdx.x == 0) {
     S.scal[SC_PQ] = v;
     if (v > 0.0) {
@@ -159,7 +157,7 @@ __global__ __launch_bounds__(kSB) void k_bs_alpha(const SysDev* __restrict__ sys
   }
 }
 
-// x += alpha p; r -= alpha q; z = Binv r; partials (r.r, r.z).  Thread per node.
+// x += alpha p; r -= alpha q; z = Dinv r; partials (r.r, r.z).  Thread per node.
 template <typename VT>
 __global__ __launch_bounds__(kSB) void k_bs_update(const SysDev* __restrict__ sys, const int32_t* __restrict__ bsys) {
   __shared__ double sh[kSB];
@@ -170,7 +168,7 @@ __global__ __launch_bounds__(kSB) void k_bs_update(const SysDev* __restrict__ sy
   VT* __restrict__ zv = (VT*)gp(static_cast<VT*>(S.z));
   const VT* __restrict__ pv = (const VT*)gp(static_cast<const VT*>(S.p));
   const VT* __restrict__ qv = (const VT*)gp(static_cast<const VT*>(S.q));
-  const float* __restrict__ binv = (const float*)gp(S.binv);
+  const float* __restrict__ dinv = (const float*)gp(S.dinv);
   const int lb = blockIdx.x - S.vblk0;
   double rr = 0.0, rz = 0.0;
   const VT alpha = (VT)S.scal[SC_ALPHA];
@@ -186,10 +184,9 @@ __global__ __launch_bounds__(kSB) void k_bs_update(const SysDev* __restrict__ sy
 #pragma unroll
     for (int c = 0; c < 3; ++c) rr += (double)r[c] * (double)r[c];
     if (S.amg) continue;
-    const float* B = binv + 9 * j;
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
-      const VT z = (VT)B[3 * c] * r[0] + (VT)B[3 * c + 1] * r[1] + (VT)B[3 * c + 2] * r[2];
+      const VT z = (VT)dinv[3 * j + c] * r[c];
       zv[3 * j + c] = z;
       rz += (double)r[c] * (double)z;
     }
@@ -197,8 +194,8 @@ __global__ __launch_bounds__(kSB) void k_bs_update(const SysDev* __restrict__ sy
   rr = bsum(rr, sh);
   rz = bsum(rz, sh);
   if (threadIdx.x == 0) {
-    S.part[S.nsblk + 2 * lb] = rr;
-    if (!S.amg) S.part[S.nsblk + 2 * lb + 1] = rz;
+    S.part[2 * lb] = rr;
+    if (!S.amg) S.part[2 * lb + 1] = rz;
   }
 }
 
@@ -209,11 +206,11 @@ __global__ __launch_bounds__(kSB) void k_bs_beta(const SysDev* __restrict__ sys)
   if (S.scal[SC_STATE] != ST_RUN) return;
   double rr = 0.0, rz = 0.0;
   for (int i = threadIdx.x; i < S.nvblk; i += kSB) {
-    rr += S.part[S.nsblk + 2 * i];
-    rz += S.part[S.nsblk + 2 * i + 1];
+    rr += S.part[2 * i];
+    if (!S.amg) rz += S.part[2 * i + 1];
   }
   rr = bsum(rr, sh);
-  rz = bsum(rz, sh);
+  rz = S.amg ? sum_spart(S, sh) : bsum(rz, sh);
   if (threadIdx.x == 0) {
     const double rho = S.scal[SC_RHO];
     S.scal[SC_BETA] = rho != 0.0 ? rz / rho : 0.0;
@@ -321,10 +318,10 @@ __global__ __launch_bounds__(kSB) void k_sum(int64_t n, const double* __restrict
   if (threadIdx.x == 0) out[0] = v;
 }
 
-// r = rh * s; p = pscale * p (= z when init); z = Binv r; partials (r.r, r.z)
+// r = rh * s; p = pscale * p (= z when init); z = Dinv r; partials (r.r, r.z)
 template <typename VT>
 __global__ __launch_bounds__(kSB) void k_ru_restart(int64_t N, const double* __restrict__ rh, double s, double pscale,
-                                                    int init, const float* __restrict__ binv, VT* __restrict__ r32,
+                                                    int init, const float* __restrict__ dinv, VT* __restrict__ r32,
                                                     VT* __restrict__ z32, VT* __restrict__ p32,
                                                     double* __restrict__ part) {
   __shared__ double sh[kSB];
@@ -337,10 +334,9 @@ __global__ __launch_bounds__(kSB) void k_ru_restart(int64_t N, const double* __r
       r[c] = (VT)(rh[3 * j + c] * s);
       r32[3 * j + c] = r[c];
     }
-    const float* B = binv + 9 * j;
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
-      const VT z = (VT)B[3 * c] * r[0] + (VT)B[3 * c + 1] * r[1] + (VT)B[3 * c + 2] * r[2];
+      const VT z = (VT)dinv[3 * j + c] * r[c];
       z32[3 * j + c] = z;
       p32[3 * j + c] = init ? z : (VT)pscale * p32[3 * j + c];
       rr += (double)r[c] * (double)r[c];
@@ -429,16 +425,18 @@ __global__ __launch_bounds__(kSB) void k_ru_rescale_amg(int64_t N, int32_t nvblk
   }
 }
 
-// AMG restart, second half: scalars from the partials (one block).
-__global__ __launch_bounds__(kSB) void k_ru_scal_amg(int32_t nvblk, const double* __restrict__ part,
-                                                     double* __restrict__ scal, double tol2, double delta2,
-                                                     double maxrun) {
+// AMG restart, second half: scalars from the partials (one block); r.z from
+// the V-cycle's nrz partials where there was one.
+__global__ __launch_bounds__(kSB) void k_ru_scal_amg(int32_t nvblk, const double* __restrict__ part, int64_t nrz,
+                                                     const double* __restrict__ rzpart, double* __restrict__ scal,
+                                                     double tol2, double delta2, double maxrun) {
   __shared__ double sh[kSB];
   double rr = 0.0, rz = 0.0;
   for (int i = threadIdx.x; i < nvblk; i += kSB) {
     rr += part[2 * i];
-    rz += part[2 * i + 1];
+    if (nrz == 0) rz += part[2 * i + 1];
   }
+  for (int64_t i = threadIdx.x; i < nrz; i += kSB) rz += rzpart[i];
   rr = bsum(rr, sh);
   rz = bsum(rz, sh);
   if (threadIdx.x == 0) {
@@ -454,12 +452,11 @@ __global__ __launch_bounds__(kSB) void k_ru_scal_amg(int32_t nvblk, const double
   }
 }
 
-// Jacobi preconditioner, stored as 3x3 blocks: the inverse diagonal of K on
-// the free components, zero elsewhere.  (Scalar Jacobi converged faster than
-// the inverse 3x3 diagonal blocks on the elasticity systems measured; the
-// block storage lets the update kernel take either.)
-__global__ void k_binv(int64_t N, const int64_t* __restrict__ adj_ptr, const int32_t* __restrict__ dslot,
-                       const double* __restrict__ val, const uint8_t* __restrict__ fixed, float* __restrict__ binv) {
+// Jacobi preconditioner: the inverse diagonal of K on the free components,
+// zero elsewhere.  (Scalar Jacobi converged faster than the inverse 3x3
+// diagonal blocks on the elasticity systems measured.)
+__global__ void k_dinv(int64_t N, const int64_t* __restrict__ adj_ptr, const int32_t* __restrict__ dslot,
+                       const double* __restrict__ val, const uint8_t* __restrict__ fixed, float* __restrict__ dinv) {
   const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (j >= N) return;
   const int64_t a0 = adj_ptr[j];
@@ -469,25 +466,30 @@ __global__ void k_binv(int64_t N, const int64_t* __restrict__ adj_ptr, const int
   for (int d = 0; d < 3; ++d) {
     const double kdd = val[9 * a0 + d * 3 * R + 3 * s + d];   // K[(j,d),(j,d)] = panel[d][s][d]
     const bool free = fixed[3 * j + d] == 0 && kdd != 0.0;
-#pragma unroll
-    for (int c = 0; c < 3; ++c) binv[9 * j + d * 3 + c] = (c == d && free) ? (float)(1.0 / kdd) : 0.f;
+    dinv[3 * j + d] = free ? (float)(1.0 / kdd) : 0.f;
   }
 }
 
-// FP32 operator in block-contiguous order: out[(a0+t)*9 + c*3 + d] = panel
-// entry [c][t][d] of node j (thread per node block).
-__global__ void k_to32_blocks(int64_t N, const int64_t* __restrict__ adj_ptr, const double* __restrict__ val,
-                              float* __restrict__ out) {
+// FP32 operator (block32.h) from the FP64 panels: lane t of a node takes its
+// blocks t, t + 32, ...
+__global__ void k_to32_blocks(int64_t N, int64_t nadj, const int64_t* __restrict__ adj_ptr,
+                              const double* __restrict__ val, float* __restrict__ out) {
   const int64_t j = (int64_t)blockIdx.x * blockDim.y + threadIdx.y;
   if (j >= N) return;
   const int64_t a0 = adj_ptr[j];
   const int64_t R = adj_ptr[j + 1] - a0;
   const double* P = val + 9 * a0;
-  for (int64_t t = threadIdx.x; t < R; t += blockDim.x)
+  for (int64_t t = threadIdx.x; t < R; t += blockDim.x) {
+    float e[9];
 #pragma unroll
     for (int c = 0; c < 3; ++c)
 #pragma unroll
-      for (int d = 0; d < 3; ++d) out[9 * (a0 + t) + 3 * c + d] = (float)P[c * 3 * R + 3 * t + d];
+      for (int d = 0; d < 3; ++d) e[3 * c + d] = (float)P[c * 3 * R + 3 * t + d];
+    const int64_t g = a0 + t;
+    reinterpret_cast<f4v*>(out)[g] = f4v{e[0], e[1], e[2], e[3]};
+    reinterpret_cast<f4v*>(out + 4 * nadj)[g] = f4v{e[4], e[5], e[6], e[7]};
+    out[8 * nadj + g] = e[8];
+  }
 }
 
 __global__ void k_fill_u(int64_t n, const uint8_t* __restrict__ fixed, const double* __restrict__ ufix,
@@ -498,9 +500,6 @@ __global__ void k_fill_u(int64_t n, const uint8_t* __restrict__ fixed, const dou
 }
 
 inline unsigned blocks(int64_t n, int bs = kSB) { return (unsigned)std::max<int64_t>(1, (n + bs - 1) / bs); }
-inline int64_t spmv_blocks(int64_t N) {
-  return std::max<int64_t>(1, std::min<int64_t>((N + kSpmvNodes - 1) / kSpmvNodes, kMaxSpmvBlocks));
-}
 inline int64_t vec_blocks(int64_t N) {
   return std::max<int64_t>(1, std::min<int64_t>((N + kVecNodes - 1) / kVecNodes, kMaxVecBlocks));
 }
@@ -519,7 +518,7 @@ struct SolveSys {
   UpdateBook book;          // rollbacks, consecutive non-finite corrections, updates
   int64_t refreshes = 0;    // AMG updates whose z had to be recomputed (drift or r.z <= 0)
   void *x = nullptr, *r = nullptr, *z = nullptr, *p = nullptr, *q = nullptr;   // Krylov vectors (VT)
-  float *binv = nullptr, *val32 = nullptr;
+  float *dinv = nullptr, *val32 = nullptr;
   int64_t npart = 0;
   double bnorm = 0.0, scale = 1.0, relres = 0.0;
   int64_t iters = 0;
@@ -547,11 +546,11 @@ void BatchSolver::release(SolveSys* s) {
 
 size_t BatchSolver::bytes_needed(int64_t N, int64_t nadj, bool f64_vectors) {
   const int64_t n = 3 * N;
-  const int64_t nsblk = spmv_blocks(N), nvblk = vec_blocks(N);
-  const int64_t npart = std::max<int64_t>(nsblk + 3 * nvblk, blocks(n)) + 64;
+  const int64_t nvblk = vec_blocks(N);
+  const int64_t npart = std::max<int64_t>(3 * nvblk, blocks(n)) + 64;
   return sizeof(double) * (5 * (size_t)n + SC_N + (size_t)npart) +
          (f64_vectors ? sizeof(double) : sizeof(float)) * 5 * (size_t)n +
-         sizeof(float) * (9 * (size_t)N + 9 * (size_t)nadj) + 16 * 256;   // 14 buffers, 256-B aligned
+         sizeof(float) * ((size_t)n + 9 * (size_t)nadj) + 16 * 256;   // 14 buffers, 256-B aligned
 }
 
 // Pinned host slots for the update readbacks (grown on demand).
@@ -657,8 +656,8 @@ int BatchSolver::update_many(const std::vector<SolveSys*>& ss, bool init) {
     const double tol = sp.reltol * s->bnorm * s_new[i];
     tol2[i] = tol * tol;
     if (s->amg) {
-      const int32_t nsblk = (int32_t)spmv_blocks(sp.N), nvblk = (int32_t)vec_blocks(sp.N);
-      double* vpart = s->part + nsblk;
+      const int32_t nvblk = (int32_t)vec_blocks(sp.N);
+      double* vpart = s->part;
       if (fresh[i]) {   // z = M r by a V-cycle of this system alone, p = z
         k_ru_restart_amg<<<(unsigned)nvblk, kSB, 0, st>>>(sp.N, nvblk, s->rh, s_new[i], pscale[i], 1, (float*)s->r,
                                                           (float*)s->p, vpart);
@@ -668,7 +667,8 @@ int BatchSolver::update_many(const std::vector<SolveSys*>& ss, bool init) {
         k_ru_rescale_amg<<<(unsigned)nvblk, kSB, 0, st>>>(sp.N, nvblk, s->rh, s_new[i], (float)pscale[i],
                                                           (float*)s->r, (float*)s->z, (float*)s->p, vpart);
       }
-      k_ru_scal_amg<<<1, kSB, 0, st>>>(nvblk, vpart, s->scal, tol2[i], kDeltaAmg * kDeltaAmg, (double)kMaxRunAmg);
+      k_ru_scal_amg<<<1, kSB, 0, st>>>(nvblk, vpart, fresh[i] ? row_groups(sp.N) : 0, s->y, s->scal, tol2[i],
+                                       kDeltaAmg * kDeltaAmg, (double)kMaxRunAmg);
       if (!fresh[i]) {
         // the rescaled z is consistent only if r.z > 0 and the true residual
         // is close to the rescaled recursive one (amg_keep_rescaled)
@@ -682,10 +682,10 @@ int BatchSolver::update_many(const std::vector<SolveSys*>& ss, bool init) {
     }
     const int64_t nb = blocks(sp.N);
     if (f64v_)
-      k_ru_restart<double><<<(unsigned)nb, kSB, 0, st>>>(sp.N, s->rh, s_new[i], pscale[i], fresh[i] ? 1 : 0, s->binv,
+      k_ru_restart<double><<<(unsigned)nb, kSB, 0, st>>>(sp.N, s->rh, s_new[i], pscale[i], fresh[i] ? 1 : 0, s->dinv,
                                                          (double*)s->r, (double*)s->z, (double*)s->p, s->part);
     else
-      k_ru_restart<float><<<(unsigned)nb, kSB, 0, st>>>(sp.N, s->rh, s_new[i], pscale[i], fresh[i] ? 1 : 0, s->binv,
+      k_ru_restart<float><<<(unsigned)nb, kSB, 0, st>>>(sp.N, s->rh, s_new[i], pscale[i], fresh[i] ? 1 : 0, s->dinv,
                                                         (float*)s->r, (float*)s->z, (float*)s->p, s->part);
     k_ru_scal<<<1, kSB, 0, st>>>(nb, s->part, s->scal, tol2[i], kDelta * kDelta);
   }
@@ -696,14 +696,15 @@ int BatchSolver::update_many(const std::vector<SolveSys*>& ss, bool init) {
       if (!check[i] || amg_keep_rescaled(h[4 * i + 2], h[4 * i + 3], kDriftAmg)) continue;
       SolveSys* s = ss[i];
       const SysSpec& sp = s->spec;
-      const int32_t nsblk = (int32_t)spmv_blocks(sp.N), nvblk = (int32_t)vec_blocks(sp.N);
-      double* vpart = s->part + nsblk;
+      const int32_t nvblk = (int32_t)vec_blocks(sp.N);
+      double* vpart = s->part;
       ++s->refreshes;
       k_ru_restart_amg<<<(unsigned)nvblk, kSB, 0, st>>>(sp.N, nvblk, s->rh, s_new[i], pscale[i], 1, (float*)s->r,
                                                         (float*)s->p, vpart);
       LLFEM_TRY(amg_apply_solo(ctx_, s->amg));
       LLFEM_HIP(hipMemcpyAsync(s->p, s->z, sizeof(float) * s->n, hipMemcpyDeviceToDevice, st));
-      k_ru_scal_amg<<<1, kSB, 0, st>>>(nvblk, vpart, s->scal, tol2[i], kDeltaAmg * kDeltaAmg, (double)kMaxRunAmg);
+      k_ru_scal_amg<<<1, kSB, 0, st>>>(nvblk, vpart, row_groups(sp.N), s->y, s->scal, tol2[i], kDeltaAmg * kDeltaAmg,
+                                       (double)kMaxRunAmg);
     }
   }
   LLFEM_HIP(hipGetLastError());
@@ -723,8 +724,8 @@ int BatchSolver::add(const SysSpec& spec, SolveSys** out) {
     return rc;
   }
   const int64_t n = s->n, N = spec.N;
-  const int64_t nsblk = spmv_blocks(N), nvblk = vec_blocks(N);
-  s->npart = std::max<int64_t>(nsblk + 3 * nvblk, blocks(n)) + 64;   // SpMV, V-cycle r.z and drift partials
+  const int64_t nvblk = vec_blocks(N);
+  s->npart = std::max<int64_t>(3 * nvblk, blocks(n)) + 64;   // vector and drift partials
   char* m = static_cast<char*>(s->mem);
   auto take = [&](size_t bytes) -> char* {
     char* p = m;
@@ -744,7 +745,7 @@ int BatchSolver::add(const SysSpec& spec, SolveSys** out) {
   s->z = take(vsz * n);
   s->p = take(vsz * n);
   s->q = take(vsz * n);
-  s->binv = (float*)take(sizeof(float) * 9 * N);
+  s->dinv = (float*)take(sizeof(float) * n);
   s->val32 = (float*)take(sizeof(float) * 9 * spec.nadj);
   if ((size_t)(m - static_cast<char*>(s->mem)) > s->bytes) {
     release(s);
@@ -754,8 +755,8 @@ int BatchSolver::add(const SysSpec& spec, SolveSys** out) {
   k_fill_u<<<blocks(n), kSB, 0, st>>>(n, spec.fixed, spec.ufix, nullptr, s->y);
   k_spmv64<<<blocks(N * kSG), kSB, 0, st>>>(N, spec.adj_ptr, spec.adj, spec.val64, s->y, nullptr, s->rh);
   k_ru_resid<<<blocks(n), kSB, 0, st>>>(n, spec.f, s->rh, spec.fixed, s->b, s->part);
-  k_to32_blocks<<<blocks(N, 8), dim3(32, 8), 0, st>>>(N, spec.adj_ptr, spec.val64, s->val32);
-  k_binv<<<blocks(N), kSB, 0, st>>>(N, spec.adj_ptr, spec.dslot, spec.val64, spec.fixed, s->binv);
+  k_to32_blocks<<<blocks(N, 8), dim3(32, 8), 0, st>>>(N, spec.nadj, spec.adj_ptr, spec.val64, s->val32);
+  k_dinv<<<blocks(N), kSB, 0, st>>>(N, spec.adj_ptr, spec.dslot, spec.val64, spec.fixed, s->dinv);
   LLFEM_HIP(hipMemsetAsync(s->xh, 0, sizeof(double) * n, st));
   LLFEM_HIP(hipMemsetAsync(s->x, 0, vsz * n, st));
   LLFEM_HIP(hipMemsetAsync(s->scal, 0, sizeof(double) * SC_N, st));
@@ -765,7 +766,7 @@ int BatchSolver::add(const SysSpec& spec, SolveSys** out) {
       release(s);
       return fail(LLFEM_EUNSUP, "engine: the AMG preconditioner runs with FP32 Krylov vectors");
     }
-    rc = amg_sys_create(ctx_, spec.amg, s->val32, (float*)s->r, (float*)s->z, (float*)s->q, s->part + nsblk, &s->amg);
+    rc = amg_sys_create(ctx_, spec.amg, s->val32, (float*)s->r, (float*)s->z, (float*)s->q, s->y, &s->amg);
     if (rc != LLFEM_OK) {
       release(s);
       return rc;
@@ -786,6 +787,7 @@ int BatchSolver::rebuild_tables() {
   std::vector<SysDev> dev;
   std::vector<int32_t> sb, vb;
   live_.clear();
+  fold_ = false;
   for (SolveSys* s : sys_) {
     if (s->status != 0) continue;
     const SysSpec& sp = s->spec;
@@ -793,13 +795,16 @@ int BatchSolver::rebuild_tables() {
     d.N = sp.N;
     d.adj_ptr = sp.adj_ptr;
     d.adj = sp.adj;
+    d.nadj = sp.nadj;
     d.val = s->val32;
     d.fixed = sp.fixed;
-    d.binv = s->binv;
+    d.dinv = s->dinv;
     d.x = s->x; d.r = s->r; d.z = s->z; d.p = s->p; d.q = s->q;
     d.scal = s->scal;
+    d.spart = s->y;
     d.part = s->part;
-    d.nsblk = (int32_t)spmv_blocks(sp.N);
+    d.nsblk = (int32_t)row_groups(sp.N);
+    fold_ = fold_ || d.nsblk > kFoldMax;
     d.nvblk = (int32_t)vec_blocks(sp.N);
     d.amg = s->amg ? 1 : 0;
     d.sblk0 = (int32_t)sb.size();
@@ -919,21 +924,23 @@ int BatchSolver::run(int iters, std::vector<SolveSys*>* finished) {
 int BatchSolver::launch_chunk(int iters) {
   hipStream_t st = ctx_->stream;
   const SysDev* sys = static_cast<const SysDev*>(d_sys_);
+  const unsigned nf = (unsigned)(nsys_ * kFoldBlocks);
   for (int k = 0; k < iters; ++k) {
+    if (f64v_) k_bs_spmv<double><<<(unsigned)nsb_, kRowThreads, 0, st>>>(sys, d_sb_);
+    else k_bs_spmv<float><<<(unsigned)nsb_, kRowThreads, 0, st>>>(sys, d_sb_);
+    if (fold_) k_bs_fold<<<nf, kSB, 0, st>>>(sys);
+    k_bs_alpha<<<(unsigned)nsys_, kSB, 0, st>>>(sys);
     if (f64v_) {
-      k_bs_spmv<double><<<(unsigned)nsb_, kSB, 0, st>>>(sys, d_sb_);
-      k_bs_alpha<<<(unsigned)nsys_, kSB, 0, st>>>(sys);
       k_bs_update<double><<<(unsigned)nvb_, kSB, 0, st>>>(sys, d_vb_);
-      k_bs_beta<<<(unsigned)nsys_, kSB, 0, st>>>(sys);
-      k_bs_pupd<double><<<(unsigned)nvb_, kSB, 0, st>>>(sys, d_vb_);
     } else {
-      k_bs_spmv<float><<<(unsigned)nsb_, kSB, 0, st>>>(sys, d_sb_);
-      k_bs_alpha<<<(unsigned)nsys_, kSB, 0, st>>>(sys);
       k_bs_update<float><<<(unsigned)nvb_, kSB, 0, st>>>(sys, d_vb_);
+      const bool amg = amg_batch_any(amgb_);
       LLFEM_TRY(amg_batch_apply(ctx_, amgb_));
-      k_bs_beta<<<(unsigned)nsys_, kSB, 0, st>>>(sys);
-      k_bs_pupd<float><<<(unsigned)nvb_, kSB, 0, st>>>(sys, d_vb_);
+      if (fold_ && amg) k_bs_fold<<<nf, kSB, 0, st>>>(sys);
     }
+    k_bs_beta<<<(unsigned)nsys_, kSB, 0, st>>>(sys);
+    if (f64v_) k_bs_pupd<double><<<(unsigned)nvb_, kSB, 0, st>>>(sys, d_vb_);
+    else k_bs_pupd<float><<<(unsigned)nvb_, kSB, 0, st>>>(sys, d_vb_);
   }
   return LLFEM_OK;
 }

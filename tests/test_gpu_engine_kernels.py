@@ -1,0 +1,39 @@
+"""Mixed-precision PCG engine and V-cycle kernels at the sizes where their
+launch shape changes: fewer nodes than a row block, remainders of 16 rows,
+2,048 row blocks and more (partials folded first).  The reference is the FP64
+residual of the assembled matrix on the host; the solver is asked for 1e-10."""
+import numpy as np
+import pytest
+import scipy.sparse as sp
+
+from lowlevelfem import _lib
+from lowlevelfem import mesh as M
+from lowlevelfem import refelem as R
+
+pytestmark = pytest.mark.gpu
+
+
+# nodes: 8, 27, 64 (4 row blocks), 125 (8 rows left), 32,768 (2,048 blocks), 35,937 (2,247)
+@pytest.mark.parametrize("method", [_lib.PCG_MIXED_RELIABLE, _lib.PCG_AMG_RELIABLE])
+@pytest.mark.parametrize("n", [1, 2, 3, 4, 31, 32])
+def test_row_blocks(gpu_ctx, n, method):
+    m = M.structured_box_mesh(n=n)
+    dev = _lib.DeviceMesh(gpu_ctx, m.coords, m.etype, m.conn)
+    val, _ = dev.assemble(_lib.OP_STIFFNESS, R.rule_tables(m.etype, 3), E=1.0)
+    cp, rv = dev.pattern()
+    K = sp.csc_matrix((val, rv, cp), shape=(3 * m.N, 3 * m.N))
+    f = np.random.default_rng(n).uniform(-1.0, 1.0, 3 * m.N)
+    left = m.nodes_on("left")
+    fixed = (3 * left[:, None] + np.arange(3)).ravel()
+    ufix = np.linspace(-1e-3, 1e-3, fixed.size)
+    u, st = dev.solve(f, fixed, ufix, method=method, reltol=1e-10)
+    free = np.ones(3 * m.N, bool)
+    free[fixed] = False
+    u0 = np.zeros(3 * m.N)
+    u0[fixed] = ufix
+    b = (f - K @ u0)[free]
+    assert np.array_equal(u[fixed], ufix)
+    assert np.linalg.norm((K @ u - f)[free]) <= 2e-10 * np.linalg.norm(b)
+    u2, st2 = dev.solve(f, fixed, ufix, method=method, reltol=1e-10)
+    assert np.array_equal(u, u2) and st2.iterations == st.iterations
+    dev.close()
