@@ -37,3 +37,24 @@ def test_row_blocks(gpu_ctx, n, method):
     u2, st2 = dev.solve(f, fixed, ufix, method=method, reltol=1e-10)
     assert np.array_equal(u, u2) and st2.iterations == st.iterations
     dev.close()
+
+
+# 28^3 x 6 tet10: 185,193 nodes, more than 131,072 aggregate pairs on the fine
+# level (16 lanes a pair); 12^3: a wave a pair on every level.  A coarse
+# operator that lacks a block or counts one twice is no Galerkin product: the
+# cycle would then converge slowly or not at all, so the iterations of the
+# larger box stay within twice those of the smaller.
+def test_galerkin_lanes(gpu_ctx):
+    its = []
+    for n in (12, 28):
+        m = M.structured_box_mesh(n=n, elem="tet", order=2)
+        dev = _lib.DeviceMesh(gpu_ctx, m.coords, m.etype, m.conn)
+        dev.assemble(_lib.OP_STIFFNESS, R.rule_tables(m.etype, 2), E=1.0, copy_out=False)
+        f = np.random.default_rng(n).uniform(-1.0, 1.0, 3 * m.N)
+        left = m.nodes_on("left")
+        fixed = (3 * left[:, None] + np.arange(3)).ravel()
+        _, st = dev.solve(f, fixed, method=_lib.PCG_AMG_RELIABLE, reltol=1e-10)
+        assert st.relres <= 1e-10
+        its.append(st.iterations)
+        dev.close()
+    assert its[1] <= 2 * its[0]
