@@ -1,5 +1,5 @@
 // Batched mixed-precision PCG engine: FP32 Krylov iterations with FP64
-// reliable updates, 3x3 block-Jacobi preconditioner, many systems per launch.
+// reliable updates, Jacobi or AMG preconditioner, many systems per launch.
 //
 // Reference: solveDisplacement(K, f; support, iterative=true, reltol, ...)
 // (src/linear.jl:3711-3743): u = u_fixed on the constrained DoFs and
@@ -48,17 +48,16 @@ constexpr int kVecNodes = kSB;           // nodes per vector block pass
 // The product's are not: 2,048 striding blocks of 8 lanes a row over 36-byte
 // records took 627 us at 2.1 M nodes (tet10, 59.5 M blocks), one block per 16
 // rows of block32.h's layout 515 us (4.6 TB/s).  Its partials lie in y, which
-// is free between updates; more than kFoldMax of them (8 per thread of a
-// summing block) are summed by kFoldBlocks blocks first, a 6 us launch that a
-// smaller system does not need.
+// is free between updates; more than kFoldMax of them (16 per thread of a
+// summing block) are summed by kFoldBlocks blocks first, a 4 to 6 us launch.
 constexpr int64_t kMaxVecBlocks = 1024;
-constexpr int64_t kFoldMax = 2048;
+constexpr int64_t kFoldMax = 4096;
 constexpr int kFoldBlocks = 64;
 
-// scal words of a system; SC_LAST: iteration count at the last FP64 update,
-// SC_MAXRUN: force an update after this many iterations (0: never)
-enum { SC_RHO = 0, SC_ALPHA, SC_BETA, SC_RR, SC_MAXRR, SC_TOL2, SC_DELTA2, SC_STATE, SC_ITER, SC_PQ, SC_LAST,
-       SC_MAXRUN, SC_N = 16 };
+// scal words of a system; SC_RHOP: r.z that the running iteration began with,
+// SC_LAST: iteration count at the last FP64 update, SC_MAXRUN: force an update
+// after this many iterations (0: never)
+enum { SC_RHO = 0, SC_RHOP, SC_RR, SC_MAXRR, SC_TOL2, SC_DELTA2, SC_STATE, SC_ITER, SC_LAST, SC_MAXRUN, SC_N = 16 };
 enum { ST_RUN = 0, ST_PENDING = 1, ST_PAUSED = 2, ST_IDLE = 3 };
 
 struct SysDev {
@@ -77,15 +76,12 @@ struct SysDev {
   int32_t amg;             // 1: z and the r.z partials (in spart) come from the AMG V-cycle
 };
 
+// Sum over the block's four waves in a fixed order; sh may be used again at once.
 __device__ __forceinline__ double bsum(double v, double* sh) {
-  const int t = threadIdx.x;
-  sh[t] = v;
+  v = wave_sum(v);
+  if (threadIdx.x % 64 == 0) sh[threadIdx.x / 64] = v;
   __syncthreads();
-  for (int o = blockDim.x / 2; o > 0; o >>= 1) {
-    if (t < o) sh[t] += sh[t + o];
-    __syncthreads();
-  }
-  const double r = sh[0];
+  const double r = (sh[0] + sh[1]) + (sh[2] + sh[3]);
   __syncthreads();
   return r;
 }
@@ -115,7 +111,7 @@ __global__ __launch_bounds__(kRowThreads) void k_bs_spmv(const SysDev* __restric
 // spart of systems with more than kFoldMax product blocks -> kFoldBlocks sums
 // of contiguous runs, behind them.  kFoldBlocks blocks per system.
 __global__ __launch_bounds__(kSB) void k_bs_fold(const SysDev* __restrict__ sys) {
-  __shared__ double sh[kSB];
+  __shared__ double sh[kSB / 64];
   const SysDev& S = sys[blockIdx.x / kFoldBlocks];
   if (S.nsblk <= kFoldMax || S.scal[SC_STATE] != ST_RUN) return;
   const int b = blockIdx.x % kFoldBlocks;
@@ -134,44 +130,39 @@ __device__ __forceinline__ double sum_spart(const SysDev& S, double* sh) {
   return bsum(v, sh);
 }
 
-// alpha = rho / p.q (one block per system).  A system flagged PENDING at the
-// end of the previous iteration becomes PAUSED here.
-__global__ __launch_bounds__(kSB) void k_bs_alpha(const SysDev* __restrict__ sys) {
-  __shared__ double sh[kSB];
-  const SysDev& S = sys[blockIdx.x];
-  const double st = S.scal[SC_STATE];
-  if (st == ST_PENDING) {
-    if (threadIdx.x == 0) S.scal[SC_STATE] = ST_PAUSED;
-    return;
-  }
-  if (st != ST_RUN) return;
-  const double v = sum_spart(S, sh);
-  if (threadIdx.x == 0) {
-    S.scal[SC_PQ] = v;
-    if (v > 0.0) {
-      S.scal[SC_ALPHA] = S.scal[SC_RHO] / v;
-    } else {   // breakdown (p = 0 or K not SPD on the free set): check the true residual
-      S.scal[SC_ALPHA] = 0.0;
-      S.scal[SC_STATE] = ST_PAUSED;
-    }
-  }
-}
-
-// x += alpha p; r -= alpha q; z = Dinv r; partials (r.r, r.z).  Thread per node.
+// alpha = rho / p.q; x += alpha p; r -= alpha q; z = Dinv r; partials
+// (r.r, r.z).  Thread per node.  Every block sums the product's partials for
+// itself, in the same order, instead of reading alpha from a launch of one
+// block per system (4 us each for alpha and beta; eight systems on a server
+// 41.5 -> 38.8 ms); block 0 keeps the words.  A system flagged PENDING at the
+// end of the previous iteration becomes PAUSED here.  Blocks that read the
+// state before or after that, or before or after a breakdown is noted, leave
+// alike.
 template <typename VT>
 __global__ __launch_bounds__(kSB) void k_bs_update(const SysDev* __restrict__ sys, const int32_t* __restrict__ bsys) {
-  __shared__ double sh[kSB];
+  __shared__ double sh[kSB / 64];
   const SysDev& S = sys[bsys[blockIdx.x]];
-  if (S.scal[SC_STATE] != ST_RUN) return;
+  const int lb = blockIdx.x - S.vblk0;
+  const bool keeper = lb == 0 && threadIdx.x == 0;
+  const double st = S.scal[SC_STATE];
+  if (st != ST_RUN) {   // block-uniform
+    if (keeper && st == ST_PENDING) S.scal[SC_STATE] = ST_PAUSED;
+    return;
+  }
+  const double rho = S.scal[SC_RHO], pq = sum_spart(S, sh);
+  if (!(pq > 0.0)) {   // breakdown (p = 0 or K not SPD on the free set): check the true residual
+    if (keeper) S.scal[SC_STATE] = ST_PAUSED;
+    return;
+  }
+  if (keeper) S.scal[SC_RHOP] = rho;
+  const VT alpha = (VT)(rho / pq);
   VT* __restrict__ xv = (VT*)gp(static_cast<VT*>(S.x));
   VT* __restrict__ rv = (VT*)gp(static_cast<VT*>(S.r));
   VT* __restrict__ zv = (VT*)gp(static_cast<VT*>(S.z));
   const VT* __restrict__ pv = (const VT*)gp(static_cast<const VT*>(S.p));
   const VT* __restrict__ qv = (const VT*)gp(static_cast<const VT*>(S.q));
   const float* __restrict__ dinv = (const float*)gp(S.dinv);
-  const int lb = blockIdx.x - S.vblk0;
   double rr = 0.0, rz = 0.0;
-  const VT alpha = (VT)S.scal[SC_ALPHA];
   for (int64_t j = (int64_t)lb * kVecNodes + threadIdx.x; j < S.N; j += (int64_t)S.nvblk * kVecNodes) {
     VT r[3];
 #pragma unroll
@@ -199,41 +190,39 @@ __global__ __launch_bounds__(kSB) void k_bs_update(const SysDev* __restrict__ sy
   }
 }
 
-// beta = rz / rho; reliable-update / convergence triggers (one block per system).
-__global__ __launch_bounds__(kSB) void k_bs_beta(const SysDev* __restrict__ sys) {
-  __shared__ double sh[kSB];
-  const SysDev& S = sys[blockIdx.x];
-  if (S.scal[SC_STATE] != ST_RUN) return;
+// beta = r.z / rho; p = z + beta p; reliable-update / convergence triggers.
+// The sums as in k_bs_update; block 0 writes no word that another block reads
+// but the state, which only turns from RUN to PENDING here, and both finish
+// their iteration.
+template <typename VT>
+__global__ __launch_bounds__(kSB) void k_bs_pupd(const SysDev* __restrict__ sys, const int32_t* __restrict__ bsys) {
+  __shared__ double sh[kSB / 64];
+  const SysDev& S = sys[bsys[blockIdx.x]];
+  const double st = S.scal[SC_STATE];
+  if (st != ST_RUN && st != ST_PENDING) return;   // block-uniform
+  const int lb = blockIdx.x - S.vblk0;
   double rr = 0.0, rz = 0.0;
   for (int i = threadIdx.x; i < S.nvblk; i += kSB) {
     rr += S.part[2 * i];
     if (!S.amg) rz += S.part[2 * i + 1];
   }
-  rr = bsum(rr, sh);
   rz = S.amg ? sum_spart(S, sh) : bsum(rz, sh);
-  if (threadIdx.x == 0) {
-    const double rho = S.scal[SC_RHO];
-    S.scal[SC_BETA] = rho != 0.0 ? rz / rho : 0.0;
-    S.scal[SC_RHO] = rz;
-    S.scal[SC_RR] = rr;
-    S.scal[SC_ITER] += 1.0;
-    const double maxrun = S.scal[SC_MAXRUN];
-    if (rr <= S.scal[SC_TOL2] || rr < S.scal[SC_DELTA2] * S.scal[SC_MAXRR] || !(rz > 0.0) ||
-        (maxrun > 0.0 && S.scal[SC_ITER] - S.scal[SC_LAST] >= maxrun))
-      S.scal[SC_STATE] = ST_PENDING;
+  const double rho = S.scal[SC_RHOP];
+  if (lb == 0) {
+    rr = bsum(rr, sh);
+    if (threadIdx.x == 0) {
+      S.scal[SC_RHO] = rz;
+      S.scal[SC_RR] = rr;
+      S.scal[SC_ITER] += 1.0;
+      const double maxrun = S.scal[SC_MAXRUN];
+      if (rr <= S.scal[SC_TOL2] || rr < S.scal[SC_DELTA2] * S.scal[SC_MAXRR] || !(rz > 0.0) ||
+          (maxrun > 0.0 && S.scal[SC_ITER] - S.scal[SC_LAST] >= maxrun))
+        S.scal[SC_STATE] = ST_PENDING;
+    }
   }
-}
-
-// p = z + beta p (RUNNING, and PENDING systems finishing their iteration).
-template <typename VT>
-__global__ __launch_bounds__(kSB) void k_bs_pupd(const SysDev* __restrict__ sys, const int32_t* __restrict__ bsys) {
-  const SysDev& S = sys[bsys[blockIdx.x]];
-  const double st = S.scal[SC_STATE];
-  if (st != ST_RUN && st != ST_PENDING) return;
   VT* __restrict__ pv = (VT*)gp(static_cast<VT*>(S.p));
   const VT* __restrict__ zv = (const VT*)gp(static_cast<const VT*>(S.z));
-  const int lb = blockIdx.x - S.vblk0;
-  const VT beta = (VT)S.scal[SC_BETA];
+  const VT beta = (VT)(rho != 0.0 ? rz / rho : 0.0);
   for (int64_t j = (int64_t)lb * kVecNodes + threadIdx.x; j < S.N; j += (int64_t)S.nvblk * kVecNodes)
 #pragma unroll
     for (int c = 0; c < 3; ++c) pv[3 * j + c] = zv[3 * j + c] + beta * pv[3 * j + c];
@@ -296,7 +285,7 @@ __global__ __launch_bounds__(kSB) void k_spmv64(int64_t N, const int64_t* __rest
 __global__ __launch_bounds__(kSB) void k_ru_resid(int64_t n, const double* __restrict__ b, const double* __restrict__ y,
                                                   const uint8_t* __restrict__ fixed, double* __restrict__ out,
                                                   double* __restrict__ part) {
-  __shared__ double sh[kSB];
+  __shared__ double sh[kSB / 64];
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   double v = 0.0;
   if (i < n) {
@@ -311,7 +300,7 @@ __global__ __launch_bounds__(kSB) void k_ru_resid(int64_t n, const double* __res
 __global__ void k_set_state(double* __restrict__ scal, double v) { scal[SC_STATE] = v; }
 
 __global__ __launch_bounds__(kSB) void k_sum(int64_t n, const double* __restrict__ part, double* __restrict__ out) {
-  __shared__ double sh[kSB];
+  __shared__ double sh[kSB / 64];
   double v = 0.0;
   for (int64_t i = threadIdx.x; i < n; i += kSB) v += part[i];
   v = bsum(v, sh);
@@ -324,7 +313,7 @@ __global__ __launch_bounds__(kSB) void k_ru_restart(int64_t N, const double* __r
                                                     int init, const float* __restrict__ dinv, VT* __restrict__ r32,
                                                     VT* __restrict__ z32, VT* __restrict__ p32,
                                                     double* __restrict__ part) {
-  __shared__ double sh[kSB];
+  __shared__ double sh[kSB / 64];
   const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   double rr = 0.0, rz = 0.0;
   if (j < N) {
@@ -353,7 +342,7 @@ __global__ __launch_bounds__(kSB) void k_ru_restart(int64_t N, const double* __r
 
 __global__ __launch_bounds__(kSB) void k_ru_scal(int64_t nb, const double* __restrict__ part, double* __restrict__ scal,
                                                  double tol2, double delta2) {
-  __shared__ double sh[kSB];
+  __shared__ double sh[kSB / 64];
   double rr = 0.0, rz = 0.0;
   for (int64_t i = threadIdx.x; i < nb; i += kSB) {
     rr += part[2 * i];
@@ -367,7 +356,6 @@ __global__ __launch_bounds__(kSB) void k_ru_scal(int64_t nb, const double* __res
     scal[SC_MAXRR] = rr;
     scal[SC_TOL2] = tol2;
     scal[SC_DELTA2] = delta2;
-    scal[SC_BETA] = 0.0;
     scal[SC_STATE] = ST_RUN;
   }
 }
@@ -377,7 +365,7 @@ __global__ __launch_bounds__(kSB) void k_ru_scal(int64_t nb, const double* __res
 __global__ __launch_bounds__(kSB) void k_ru_restart_amg(int64_t N, int32_t nvblk, const double* __restrict__ rh,
                                                         double s, double pscale, int init, float* __restrict__ r32,
                                                         float* __restrict__ p32, double* __restrict__ part) {
-  __shared__ double sh[kSB];
+  __shared__ double sh[kSB / 64];
   double rr = 0.0;
   for (int64_t j = (int64_t)blockIdx.x * kVecNodes + threadIdx.x; j < N; j += (int64_t)nvblk * kVecNodes)
 #pragma unroll
@@ -400,7 +388,7 @@ __global__ __launch_bounds__(kSB) void k_ru_rescale_amg(int64_t N, int32_t nvblk
                                                         double s, float pscale, float* __restrict__ r32,
                                                         float* __restrict__ z32, float* __restrict__ p32,
                                                         double* __restrict__ part) {
-  __shared__ double sh[kSB];
+  __shared__ double sh[kSB / 64];
   double rr = 0.0, rz = 0.0, dd = 0.0;
   for (int64_t j = (int64_t)blockIdx.x * kVecNodes + threadIdx.x; j < N; j += (int64_t)nvblk * kVecNodes)
 #pragma unroll
@@ -430,7 +418,7 @@ __global__ __launch_bounds__(kSB) void k_ru_rescale_amg(int64_t N, int32_t nvblk
 __global__ __launch_bounds__(kSB) void k_ru_scal_amg(int32_t nvblk, const double* __restrict__ part, int64_t nrz,
                                                      const double* __restrict__ rzpart, double* __restrict__ scal,
                                                      double tol2, double delta2, double maxrun) {
-  __shared__ double sh[kSB];
+  __shared__ double sh[kSB / 64];
   double rr = 0.0, rz = 0.0;
   for (int i = threadIdx.x; i < nvblk; i += kSB) {
     rr += part[2 * i];
@@ -445,7 +433,6 @@ __global__ __launch_bounds__(kSB) void k_ru_scal_amg(int32_t nvblk, const double
     scal[SC_MAXRR] = rr;
     scal[SC_TOL2] = tol2;
     scal[SC_DELTA2] = delta2;
-    scal[SC_BETA] = 0.0;
     scal[SC_LAST] = scal[SC_ITER];
     scal[SC_MAXRUN] = maxrun;
     scal[SC_STATE] = ST_RUN;
@@ -929,7 +916,6 @@ int BatchSolver::launch_chunk(int iters) {
     if (f64v_) k_bs_spmv<double><<<(unsigned)nsb_, kRowThreads, 0, st>>>(sys, d_sb_);
     else k_bs_spmv<float><<<(unsigned)nsb_, kRowThreads, 0, st>>>(sys, d_sb_);
     if (fold_) k_bs_fold<<<nf, kSB, 0, st>>>(sys);
-    k_bs_alpha<<<(unsigned)nsys_, kSB, 0, st>>>(sys);
     if (f64v_) {
       k_bs_update<double><<<(unsigned)nvb_, kSB, 0, st>>>(sys, d_vb_);
     } else {
@@ -938,7 +924,6 @@ int BatchSolver::launch_chunk(int iters) {
       LLFEM_TRY(amg_batch_apply(ctx_, amgb_));
       if (fold_ && amg) k_bs_fold<<<nf, kSB, 0, st>>>(sys);
     }
-    k_bs_beta<<<(unsigned)nsys_, kSB, 0, st>>>(sys);
     if (f64v_) k_bs_pupd<double><<<(unsigned)nvb_, kSB, 0, st>>>(sys, d_vb_);
     else k_bs_pupd<float><<<(unsigned)nvb_, kSB, 0, st>>>(sys, d_vb_);
   }
