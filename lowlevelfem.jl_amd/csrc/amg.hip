@@ -47,7 +47,7 @@ namespace llfem {
 namespace {
 
 constexpr int kMB = 256;                 // threads per block
-constexpr int kMG = 8;                   // lanes per aggregate in the restriction
+constexpr int kMG = 16;                  // lanes per aggregate in the restriction
 constexpr int kMSpN = kMB / kMG;         // aggregates per restriction block
 // The row kernels (products, block32.h) take one block per kRowNodes rows; the
 // vector and restriction kernels cap their blocks and stride.
@@ -60,6 +60,9 @@ constexpr int kPowerSteps = 15;
 constexpr int64_t kCoarseAggs = 24;      // coarsest level: at most this many aggregates
 constexpr int kMaxLevels = 12;
 constexpr int64_t kMaxDense = 1536;      // DoFs of the dense coarsest solve
+constexpr int kTB = 1024;                // threads of the tail kernel
+constexpr int64_t kTailN = 320;          // pseudo-nodes of a tail's levels together (the coarsest alone: kMaxDense / 3)
+constexpr int64_t kTailMax = kTailN > kMaxDense / 3 ? kTailN : kMaxDense / 3;
 
 inline unsigned nblk(int64_t n, int bs = kMB) { return (unsigned)std::max<int64_t>(1, (n + bs - 1) / bs); }
 inline int64_t cap(int64_t n, int64_t per, int64_t mx) { return std::max<int64_t>(1, std::min<int64_t>((n + per - 1) / per, mx)); }
@@ -99,6 +102,9 @@ struct MgEnt {
   int64_t nagg;
   float* bc;                 // next level's b
   const float* xc;           // next level's x
+  float *yc, *dc;            // next level's y, d and inverse diagonal (NULL: that level is in the tail)
+  const float* dinvc;
+  float inv_thetac;
   const float* Ainv;         // coarsest: dense inverse [nc][nc]
   int32_t nc;
   float inv_theta, inv_delta;
@@ -107,14 +113,34 @@ struct MgEnt {
   int32_t sblk0, nsblk, vblk0, nvblk, ablk0, nablk;
 };
 
+// A system's last levels in the tail kernel: entries first .. first + count - 1.
+struct MgTail {
+  int32_t first, count;
+};
+
 namespace {
+
+struct ChebCoef {
+  float ca, cbt, cbd;
+};
+struct ChebSet {
+  ChebCoef pre[kCheb - 1], post[kCheb];
+};
 
 __device__ __forceinline__ bool mg_skip(const MgEnt& E) { return E.state && *E.state != 0.0; }
 
+// entry of a block; the map is a dependent load that one entry needs none of
+__device__ __forceinline__ const MgEnt& mg_ent(const MgEnt* ents, const int32_t* map, int nent) {
+  return ents[nent == 1 ? 0 : map[blockIdx.x]];
+}
 
-// first Chebyshev step from x = 0: y = d = D^-1 b / theta
-__global__ __launch_bounds__(kMB) void k_mg_cheb0(const MgEnt* __restrict__ ents, const int32_t* __restrict__ map) {
-  const MgEnt& E = ents[map[blockIdx.x]];
+
+// First Chebyshev step from x = 0: y = d = D^-1 b / theta.  Only where level 0
+// starts outside the engine's iteration: there the update kernel does it, and
+// k_mg_restrict for the other levels.
+__global__ __launch_bounds__(kMB) void k_mg_cheb0(const MgEnt* __restrict__ ents, const int32_t* __restrict__ map,
+                                                  int nent) {
+  const MgEnt& E = mg_ent(ents, map, nent);
   if (mg_skip(E)) return;
   const int lb = blockIdx.x - E.vblk0;
   const float* __restrict__ dinv = (const float*)gp(E.dinv);
@@ -138,22 +164,30 @@ __global__ __launch_bounds__(kMB) void k_mg_cheb0(const MgEnt* __restrict__ ents
 // another array than u because other blocks still read u.  rz (level 0, last
 // step): partial b.w per block.
 __global__ __launch_bounds__(kRowThreads) void k_mg_smooth(const MgEnt* __restrict__ ents,
-                                                           const int32_t* __restrict__ map, float ca, float cbt,
-                                                           float cbd, int from_y, int rz) {
+                                                           const int32_t* __restrict__ map, int nent, float ca,
+                                                           float cbt, float cbd, int from_y, int rz) {
   __shared__ float sh[3 * kRowNodes];
-  const MgEnt& E = ents[map[blockIdx.x]];
-  if (mg_skip(E)) return;
+  const MgEnt& E = mg_ent(ents, map, nent);
   const int lb = blockIdx.x - E.sblk0;
+  const RowSpan rs = row_span(E.N, gp(E.adj_ptr), lb);
+  if (mg_skip(E)) return;
   const auto* __restrict__ u = gp((const float*)(from_y ? E.y : E.x));
-  block_rows<float>(E.N, E.nadj, gp(E.adj_ptr), gp(E.adj), gp(E.val), u, lb, sh);
-  if (threadIdx.x >= 64) return;
   const int64_t i = (int64_t)lb * 3 * kRowNodes + threadIdx.x;
+  const bool own = threadIdx.x < 3 * kRowNodes && i < 3 * E.N;
+  float bi = 0.f, di = 0.f, vi = 0.f, ui = 0.f;
+  if (own) {   // loaded now, beside the product's
+    bi = gp(E.b)[i];
+    di = gp(E.d)[i];
+    vi = gp(E.dinv)[i];
+    ui = u[i];
+  }
+  block_rows<float>(E.nadj, rs, gp(E.adj), gp(E.val), u, sh);
+  if (threadIdx.x >= 64) return;
   double acc = 0.0;
-  if (threadIdx.x < 3 * kRowNodes && i < 3 * E.N) {
+  if (own) {
     const float cb = cbt * E.inv_theta + cbd * E.inv_delta;
-    const float bi = gp(E.b)[i];
-    const float dv = ca * gp(E.d)[i] + cb * gp(E.dinv)[i] * (bi - sh[threadIdx.x]);
-    const float wv = u[i] + dv;
+    const float dv = ca * di + cb * vi * (bi - sh[threadIdx.x]);
+    const float wv = ui + dv;
     gp(E.d)[i] = dv;
     gp(from_y ? E.x : E.y)[i] = wv;
     acc = (double)bi * (double)wv;
@@ -166,23 +200,30 @@ __global__ __launch_bounds__(kRowThreads) void k_mg_smooth(const MgEnt* __restri
 
 // residual of the level, w = mask(b - A u): u, w = y, x (from_y) or x, y
 __global__ __launch_bounds__(kRowThreads) void k_mg_resid(const MgEnt* __restrict__ ents,
-                                                          const int32_t* __restrict__ map, int from_y) {
+                                                          const int32_t* __restrict__ map, int nent, int from_y) {
   __shared__ float sh[3 * kRowNodes];
-  const MgEnt& E = ents[map[blockIdx.x]];
-  if (mg_skip(E)) return;
+  const MgEnt& E = mg_ent(ents, map, nent);
   const int lb = blockIdx.x - E.sblk0;
+  const RowSpan rs = row_span(E.N, gp(E.adj_ptr), lb);
+  if (mg_skip(E)) return;
   const auto* __restrict__ u = gp((const float*)(from_y ? E.y : E.x));
-  block_rows<float>(E.N, E.nadj, gp(E.adj_ptr), gp(E.adj), gp(E.val), u, lb, sh);
   const int64_t i = (int64_t)lb * 3 * kRowNodes + threadIdx.x;
-  if (threadIdx.x < 3 * kRowNodes && i < 3 * E.N)
-    gp(from_y ? E.x : E.y)[i] = gp(E.mask)[i] ? 0.f : gp(E.b)[i] - sh[threadIdx.x];
+  const bool own = threadIdx.x < 3 * kRowNodes && i < 3 * E.N;
+  float bi = 0.f;
+  uint8_t mi = 1;
+  if (own) {
+    bi = gp(E.b)[i];
+    mi = gp(E.mask)[i];
+  }
+  block_rows<float>(E.nadj, rs, gp(E.adj), gp(E.val), u, sh);
+  if (own) gp(from_y ? E.x : E.y)[i] = mi ? 0.f : bi - sh[threadIdx.x];
 }
 
 // bc = Q^T r, r in y (in_y) or x: kMG lanes per aggregate stride over its
 // members, then a fixed shuffle tree sums the lanes.
 __global__ __launch_bounds__(kMB) void k_mg_restrict(const MgEnt* __restrict__ ents, const int32_t* __restrict__ map,
-                                                     int in_y) {
-  const MgEnt& E = ents[map[blockIdx.x]];
+                                                     int nent, int in_y) {
+  const MgEnt& E = mg_ent(ents, map, nent);
   if (mg_skip(E)) return;
   const int lb = blockIdx.x - E.ablk0;
   const int l = threadIdx.x % kMG;
@@ -210,16 +251,25 @@ __global__ __launch_bounds__(kMB) void k_mg_restrict(const MgEnt* __restrict__ e
     for (int o = kMG / 2; o > 0; o >>= 1)
 #pragma unroll
       for (int u = 0; u < 6; ++u) acc[u] += __shfl_xor(acc[u], o, kMG);
-    if (a < E.nagg && l == 0)
+    if (a < E.nagg && l < 6) {
+      float v = acc[0];
 #pragma unroll
-      for (int u = 0; u < 6; ++u) bc[6 * a + u] = acc[u];
+      for (int u = 1; u < 6; ++u) v = l == u ? acc[u] : v;
+      const int64_t i = 6 * a + l;
+      bc[i] = v;
+      if (E.yc) {   // the next level's first Chebyshev step
+        const float w = E.inv_thetac * gp(E.dinvc)[i] * v;
+        gp(E.yc)[i] = w;
+        gp(E.dc)[i] = w;
+      }
+    }
   }
 }
 
 // u += alpha Q xc, u = y (in_y) or x
 __global__ __launch_bounds__(kMB) void k_mg_prolong(const MgEnt* __restrict__ ents, const int32_t* __restrict__ map,
-                                                    float alpha, int in_y) {
-  const MgEnt& E = ents[map[blockIdx.x]];
+                                                    int nent, float alpha, int in_y) {
+  const MgEnt& E = mg_ent(ents, map, nent);
   if (mg_skip(E)) return;
   const int lb = blockIdx.x - E.vblk0;
   const int32_t* __restrict__ agg = (const int32_t*)gp(E.agg);
@@ -244,19 +294,140 @@ __global__ __launch_bounds__(kMB) void k_mg_prolong(const MgEnt* __restrict__ en
   }
 }
 
-// coarsest level: x = Ainv b (block per entry)
-__global__ __launch_bounds__(kMB) void k_mg_coarse(const MgEnt* __restrict__ ents) {
-  const MgEnt& E = ents[blockIdx.x];
-  if (mg_skip(E)) return;
-  const int n = E.nc;
-  const float* __restrict__ Ainv = (const float*)gp(E.Ainv);
-  const float* __restrict__ b = (const float*)gp(E.b);
-  float* __restrict__ x = (float*)gp(E.x);
-  for (int i = threadIdx.x; i < n; i += kMB) {
-    const float* row = Ainv + (int64_t)i * n;
-    float s = 0.f;
-    for (int k = 0; k < n; ++k) s += row[k] * b[k];
-    x[i] = s;
+// The levels from a system's tail to its coarsest (x = Ainv b there), one block
+// per system: their vectors lie in LDS and a barrier stands for the end of a
+// launch.  As launches of their own these levels take 4.5 us a kernel, seven a
+// level and 8 us for the coarsest, whatever their size; here one CU fetches the
+// operator (28 KB a pass of 64 rows) four times over, so a level pays while it
+// has few rows: up to 320 23 us instead of 40, up to 1,000 45 us (eight systems
+// on a server 44.5 and 47.0 ms under the same load).  Rows kept in registers
+// spilled and lost.
+__global__ __launch_bounds__(kTB) void k_mg_tail(const MgTail* __restrict__ tails, const MgEnt* __restrict__ ents,
+                                                 ChebSet cs, float alpha) {
+  __shared__ float sb[3 * kTailMax], sx[3 * kTailMax], sy[3 * kTailMax], sd[3 * kTailMax];
+  const MgTail T = tails[blockIdx.x];
+  const MgEnt* L = ents + T.first;
+  if (mg_skip(L[0])) return;
+  const int t = threadIdx.x, l = t % kRowLanes;
+  // one Chebyshev step of level E at offset o: u -> w (k_mg_smooth)
+  auto smooth = [&](const MgEnt& E, int o, const ChebCoef& c, const float* u, float* w) {
+    const float cb = c.cbt * E.inv_theta + c.cbd * E.inv_delta;
+    const auto ap = gp(E.adj_ptr);
+    const auto dinv = gp(E.dinv);
+    for (int j = t / kRowLanes; j < (int)E.N; j += kTB / kRowLanes) {
+      const int64_t p0 = ap[j];
+      float a0, a1, a2;
+      row_product<float>(E.nadj, gp(E.adj), gp(E.val), u + o, p0, (int)(ap[j + 1] - p0), l, a0, a1, a2);
+      if (l < 3) {
+        const int i = 3 * j + l;
+        const float dv = c.ca * sd[o + i] + cb * dinv[i] * (sb[o + i] - (l == 0 ? a0 : l == 1 ? a1 : a2));
+        sd[o + i] = dv;
+        w[o + i] = u[o + i] + dv;
+      }
+    }
+    __syncthreads();
+  };
+  int o = 0;
+  for (int i = t; i < 3 * (int)L[0].N; i += kTB) sb[i] = gp((const float*)L[0].b)[i];
+  __syncthreads();
+  for (int k = 0; k + 1 < T.count; ++k) {
+    const MgEnt& E = L[k];
+    const int n = 3 * (int)E.N;
+    for (int i = t; i < n; i += kTB) {
+      const float v = E.inv_theta * gp(E.dinv)[i] * sb[o + i];
+      sy[o + i] = v;
+      sd[o + i] = v;
+    }
+    __syncthreads();
+    float *u = sy, *w = sx;
+#pragma unroll
+    for (int s = 0; s < kCheb - 1; ++s) {
+      smooth(E, o, cs.pre[s], u, w);
+      float* h = u;
+      u = w;
+      w = h;
+    }
+    const auto ap = gp(E.adj_ptr);
+    for (int j = t / kRowLanes; j < (int)E.N; j += kTB / kRowLanes) {   // w = mask(b - A u)
+      const int64_t p0 = ap[j];
+      float a0, a1, a2;
+      row_product<float>(E.nadj, gp(E.adj), gp(E.val), u + o, p0, (int)(ap[j + 1] - p0), l, a0, a1, a2);
+      if (l < 3) {
+        const int i = 3 * j + l;
+        w[o + i] = gp(E.mask)[i] ? 0.f : sb[o + i] - (l == 0 ? a0 : l == 1 ? a1 : a2);
+      }
+    }
+    __syncthreads();
+    const auto mp = gp(E.mem_ptr);
+    const auto mem = gp(E.mem);
+    const auto Q = gp(E.Q);
+    const int lm = t % kMG;
+    for (int a = t / kMG; a < (int)E.nagg; a += kTB / kMG) {   // next b = Q^T w
+      float acc[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+      for (int32_t m = mp[a] + lm; m < mp[a + 1]; m += kMG) {
+        const int j = mem[m];
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+          const float r = w[o + 3 * j + c];
+#pragma unroll
+          for (int v = 0; v < 6; ++v) acc[v] += Q[18 * j + 6 * c + v] * r;
+        }
+      }
+#pragma unroll
+      for (int q = kMG / 2; q > 0; q >>= 1)
+#pragma unroll
+        for (int v = 0; v < 6; ++v) acc[v] += __shfl_xor(acc[v], q, kMG);
+      if (lm < 6) {
+        float r = acc[0];
+#pragma unroll
+        for (int v = 1; v < 6; ++v) r = lm == v ? acc[v] : r;
+        sb[o + n + 6 * a + lm] = r;
+      }
+    }
+    __syncthreads();
+    o += n;
+  }
+  {
+    const MgEnt& E = L[T.count - 1];
+    const auto Ai = gp(E.Ainv);
+    for (int i = t / kRowLanes; i < E.nc; i += kTB / kRowLanes) {
+      float s = 0.f;
+      for (int k = l; k < E.nc; k += kRowLanes) s += Ai[(int64_t)i * E.nc + k] * sb[o + k];
+#pragma unroll
+      for (int q = kRowLanes / 2; q > 0; q >>= 1) s += __shfl_xor(s, q, kRowLanes);
+      if (l == 0) sx[o + i] = s;
+    }
+    __syncthreads();
+  }
+  for (int k = T.count - 2; k >= 0; --k) {
+    const MgEnt& E = L[k];
+    const int n = 3 * (int)E.N;
+    o -= n;
+    float* u = kCheb % 2 ? sy : sx;
+    float* w = kCheb % 2 ? sx : sy;
+    for (int i = t; i < n; i += kTB) {   // u += alpha Q x of the next level
+      const int a = gp(E.agg)[i / 3];
+      if (a < 0) continue;
+      float s = 0.f;
+#pragma unroll
+      for (int v = 0; v < 6; ++v) s += gp(E.Q)[6 * i + v] * sx[o + n + 6 * a + v];
+      u[o + i] += alpha * s;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < kCheb; ++s) {
+      smooth(E, o, cs.post[s], u, w);
+      float* h = u;
+      u = w;
+      w = h;
+    }
+  }
+  for (int i = t; i < 3 * (int)L[0].N; i += kTB) gp(L[0].x)[i] = sx[i];
+  if (L[0].rzpart && t < (int)L[0].nsblk) {   // a whole system in the tail
+    const int i0 = 3 * kRowNodes * t, i1 = min(3 * (int)L[0].N, i0 + 3 * kRowNodes);
+    double acc = 0.0;
+    for (int i = i0; i < i1; ++i) acc += (double)sb[i] * (double)sx[i];
+    gp(L[0].rzpart)[t] = acc;
   }
 }
 
@@ -372,7 +543,7 @@ __global__ __launch_bounds__(kRowThreads) void k_mg_spmv1(int64_t N, int64_t nad
                                                           const float* __restrict__ dinv,
                                                           const float* __restrict__ x, float* __restrict__ y) {
   __shared__ float sh[3 * kRowNodes];
-  block_rows<float>(N, nadj, adj_ptr, adj, gp(val), x, blockIdx.x, sh);
+  block_rows<float>(nadj, row_span(N, adj_ptr, blockIdx.x), adj, gp(val), x, sh);
   const int64_t i = (int64_t)blockIdx.x * 3 * kRowNodes + threadIdx.x;
   if (threadIdx.x < 3 * kRowNodes && i < 3 * N)
     y[i] = dinv ? dinv[i] * sh[threadIdx.x] : mask[i] ? 0.f : sh[threadIdx.x];
@@ -1073,57 +1244,57 @@ struct AmgSys {
     int32_t *smap = nullptr, *vmap = nullptr, *amap = nullptr;
     int nent = 0;
     int64_t nsb = 0, nvb = 0, nab = 0;
-    MgEnt* cents = nullptr;
-    int ncent = 0;
+    MgEnt* tents = nullptr;          // the levels of tails that begin on this level
+    MgTail* tails = nullptr;
+    int ntail = 0;
   };
+  int tail = 0;                      // first level in the tail kernel
   std::vector<Tab> solo;
   std::vector<double> lambda;
 };
 
 namespace {
 
-struct ChebCoef {
-  float ca, cbt, cbd;
-};
-
 // Chebyshev recurrence coefficients for the interval [lo, hi] x lambda: the
 // same for every level and system (only theta and delta scale with lambda).
-void cheb_coefs(std::vector<ChebCoef>& pre, std::vector<ChebCoef>& post) {
+ChebSet cheb_coefs() {
   const double theta = 0.5 * (kChebHi + kChebLo), delta = 0.5 * (kChebHi - kChebLo);
   const double sigma = theta / delta;
-  pre.clear();
-  post.clear();
+  ChebSet cs{};
   double rho = 1.0 / sigma;
-  for (int s = 1; s < kCheb; ++s) {   // pre: step 0 is k_mg_cheb0
+  for (int s = 1; s < kCheb; ++s) {   // pre: step 0 starts from x = 0
     const double rn = 1.0 / (2.0 * sigma - rho);
-    pre.push_back({(float)(rn * rho), 0.f, (float)(2.0 * rn)});
+    cs.pre[s - 1] = {(float)(rn * rho), 0.f, (float)(2.0 * rn)};
     rho = rn;
   }
   rho = 1.0 / sigma;
-  post.push_back({0.f, 1.f, 0.f});
+  cs.post[0] = {0.f, 1.f, 0.f};
   for (int s = 1; s < kCheb; ++s) {
     const double rn = 1.0 / (2.0 * sigma - rho);
-    post.push_back({(float)(rn * rho), 0.f, (float)(2.0 * rn)});
+    cs.post[s] = {(float)(rn * rho), 0.f, (float)(2.0 * rn)};
     rho = rn;
   }
+  return cs;
 }
 
 // Launch tables for a set of systems (block -> entry maps per level).
 struct TabBuild {
-  std::vector<std::vector<MgEnt>> ents, cents;
+  std::vector<std::vector<MgEnt>> ents, tents;
+  std::vector<std::vector<MgTail>> tails;
   std::vector<std::vector<int32_t>> smap, vmap, amap;
 };
 
 void tab_add(TabBuild& T, const AmgSys* s, const double* state) {
-  const int L = (int)s->ent.size() - 1;
-  if ((int)T.ents.size() < L + 1) {
-    T.ents.resize(L + 1);
-    T.cents.resize(L + 1);
-    T.smap.resize(L + 1);
-    T.vmap.resize(L + 1);
-    T.amap.resize(L + 1);
+  const int t = s->tail;
+  if ((int)T.ents.size() < t + 1) {
+    T.ents.resize(t + 1);
+    T.tents.resize(t + 1);
+    T.tails.resize(t + 1);
+    T.smap.resize(t + 1);
+    T.vmap.resize(t + 1);
+    T.amap.resize(t + 1);
   }
-  for (int l = 0; l < L; ++l) {
+  for (int l = 0; l < t; ++l) {
     MgEnt e = s->ent[l];
     e.state = state;
     const int32_t id = (int32_t)T.ents[l].size();
@@ -1135,16 +1306,19 @@ void tab_add(TabBuild& T, const AmgSys* s, const double* state) {
     T.amap[l].insert(T.amap[l].end(), (size_t)e.nablk, id);
     T.ents[l].push_back(e);
   }
-  MgEnt c = s->ent[L];
-  c.state = state;
-  T.cents[L].push_back(c);
+  T.tails[t].push_back({(int32_t)T.tents[t].size(), (int32_t)(s->ent.size() - t)});
+  for (size_t l = t; l < s->ent.size(); ++l) {
+    T.tents[t].push_back(s->ent[l]);
+    T.tents[t].back().state = state;
+  }
 }
 
 int tab_upload(llfem_ctx* ctx, const TabBuild& T, void** mem, size_t* bytes, std::vector<AmgSys::Tab>* out) {
   size_t need = 0;
   auto al = [](size_t b) { return (b + 255) / 256 * 256; };
   for (size_t l = 0; l < T.ents.size(); ++l)
-    need += al(sizeof(MgEnt) * T.ents[l].size()) + al(sizeof(MgEnt) * T.cents[l].size()) +
+    need += al(sizeof(MgEnt) * T.ents[l].size()) + al(sizeof(MgEnt) * T.tents[l].size()) +
+            al(sizeof(MgTail) * T.tails[l].size()) +
             al(4 * T.smap[l].size()) + al(4 * T.vmap[l].size()) + al(4 * T.amap[l].size());
   need += 256;
   if (*bytes < need) {
@@ -1168,51 +1342,52 @@ int tab_upload(llfem_ctx* ctx, const TabBuild& T, void** mem, size_t* bytes, std
   for (size_t l = 0; l < T.ents.size(); ++l) {
     AmgSys::Tab& t = (*out)[l];
     t.nent = (int)T.ents[l].size();
-    t.ncent = (int)T.cents[l].size();
+    t.ntail = (int)T.tails[l].size();
     t.nsb = (int64_t)T.smap[l].size();
     t.nvb = (int64_t)T.vmap[l].size();
     t.nab = (int64_t)T.amap[l].size();
     t.ents = reinterpret_cast<MgEnt*>(put(T.ents[l].data(), sizeof(MgEnt) * T.ents[l].size()));
-    t.cents = reinterpret_cast<MgEnt*>(put(T.cents[l].data(), sizeof(MgEnt) * T.cents[l].size()));
+    t.tents = reinterpret_cast<MgEnt*>(put(T.tents[l].data(), sizeof(MgEnt) * T.tents[l].size()));
+    t.tails = reinterpret_cast<MgTail*>(put(T.tails[l].data(), sizeof(MgTail) * T.tails[l].size()));
     t.smap = reinterpret_cast<int32_t*>(put(T.smap[l].data(), 4 * T.smap[l].size()));
     t.vmap = reinterpret_cast<int32_t*>(put(T.vmap[l].data(), 4 * T.vmap[l].size()));
     t.amap = reinterpret_cast<int32_t*>(put(T.amap[l].data(), 4 * T.amap[l].size()));
-    if (!t.ents || !t.cents || !t.smap || !t.vmap || !t.amap) return fail(LLFEM_EHIP, "AMG: table upload failed");
+    if (!t.ents || !t.tents || !t.tails || !t.smap || !t.vmap || !t.amap) return fail(LLFEM_EHIP, "AMG: table upload failed");
   }
   LLFEM_HIP(hipStreamSynchronize(st));   // host tables go out of scope
   return LLFEM_OK;
 }
 
-int run_vcycle(llfem_ctx* ctx, const std::vector<AmgSys::Tab>& T) {
+// head: level 0's first Chebyshev step is still to be done
+int run_vcycle(llfem_ctx* ctx, const std::vector<AmgSys::Tab>& T, bool head) {
   hipStream_t st = ctx->stream;
-  static thread_local std::vector<ChebCoef> pre, post;
-  if (post.empty()) cheb_coefs(pre, post);
+  static const ChebSet cs = cheb_coefs();
   const int L = (int)T.size();
   // the iterate starts in y and changes array with each of the 2 kCheb - 1
   // (odd) smoothing steps, so it ends in x
   static_assert((2 * kCheb - 1) % 2 == 1, "the V-cycle's result has to end in x");
   for (int l = 0; l < L; ++l) {
     const AmgSys::Tab& t = T[l];
-    if (t.nent) {
-      int in_y = 1;
-      k_mg_cheb0<<<(unsigned)t.nvb, kMB, 0, st>>>(t.ents, t.vmap);
-      for (const ChebCoef& c : pre) {
-        k_mg_smooth<<<(unsigned)t.nsb, kRowThreads, 0, st>>>(t.ents, t.smap, c.ca, c.cbt, c.cbd, in_y, 0);
-        in_y ^= 1;
-      }
-      k_mg_resid<<<(unsigned)t.nsb, kRowThreads, 0, st>>>(t.ents, t.smap, in_y);
-      k_mg_restrict<<<(unsigned)t.nab, kMB, 0, st>>>(t.ents, t.amap, in_y ^ 1);
+    if (t.ntail) k_mg_tail<<<(unsigned)t.ntail, kTB, 0, st>>>(t.tails, t.tents, cs, kOverCorrect);
+    if (!t.nent) continue;
+    int in_y = 1;
+    if (l == 0 && head) k_mg_cheb0<<<(unsigned)t.nvb, kMB, 0, st>>>(t.ents, t.vmap, t.nent);
+    for (const ChebCoef& c : cs.pre) {
+      k_mg_smooth<<<(unsigned)t.nsb, kRowThreads, 0, st>>>(t.ents, t.smap, t.nent, c.ca, c.cbt, c.cbd, in_y, 0);
+      in_y ^= 1;
     }
-    if (t.ncent) k_mg_coarse<<<(unsigned)t.ncent, kMB, 0, st>>>(t.cents);
+    k_mg_resid<<<(unsigned)t.nsb, kRowThreads, 0, st>>>(t.ents, t.smap, t.nent, in_y);
+    k_mg_restrict<<<(unsigned)t.nab, kMB, 0, st>>>(t.ents, t.amap, t.nent, in_y ^ 1);
   }
   for (int l = L - 1; l >= 0; --l) {
     const AmgSys::Tab& t = T[l];
     if (!t.nent) continue;
-    int in_y = (int)((pre.size() + 1) % 2);
-    k_mg_prolong<<<(unsigned)t.nvb, kMB, 0, st>>>(t.ents, t.vmap, kOverCorrect, in_y);
-    for (size_t s = 0; s < post.size(); ++s) {
-      k_mg_smooth<<<(unsigned)t.nsb, kRowThreads, 0, st>>>(t.ents, t.smap, post[s].ca, post[s].cbt, post[s].cbd, in_y,
-                                                           (l == 0 && s + 1 == post.size()) ? 1 : 0);
+    int in_y = kCheb % 2;
+    k_mg_prolong<<<(unsigned)t.nvb, kMB, 0, st>>>(t.ents, t.vmap, t.nent, kOverCorrect, in_y);
+    for (int s = 0; s < kCheb; ++s) {
+      const ChebCoef& c = cs.post[s];
+      k_mg_smooth<<<(unsigned)t.nsb, kRowThreads, 0, st>>>(t.ents, t.smap, t.nent, c.ca, c.cbt, c.cbd, in_y,
+                                                           (l == 0 && s + 1 == kCheb) ? 1 : 0);
       in_y ^= 1;
     }
   }
@@ -1332,6 +1507,11 @@ int amg_sys_create(llfem_ctx* ctx, const AmgHier* h, const float* val32, float* 
     e.nagg = D.nagg;
     e.nablk = (int32_t)cap(D.nagg, kMSpN, kMaxAB);
   }
+  s->tail = L;
+  for (int64_t n = h->lev[L].N; s->tail > 0; --s->tail) {
+    n += h->lev[s->tail - 1].N;
+    if (n > kTailN) break;
+  }
   for (int l = 0; l < L; ++l) {
     s->ent[l].bc = s->ent[l + 1].b;
     s->ent[l].xc = s->ent[l + 1].x;
@@ -1395,6 +1575,12 @@ int amg_sys_create(llfem_ctx* ctx, const AmgHier* h, const float* val32, float* 
     s->ent[l].inv_theta = (float)(1.0 / (0.5 * (kChebHi + kChebLo) * lmb));
     s->ent[l].inv_delta = (float)(1.0 / (0.5 * (kChebHi - kChebLo) * lmb));
   }
+  for (int l = 0; l + 1 < s->tail; ++l) {
+    s->ent[l].yc = s->ent[l + 1].y;
+    s->ent[l].dc = s->ent[l + 1].d;
+    s->ent[l].dinvc = s->ent[l + 1].dinv;
+    s->ent[l].inv_thetac = s->ent[l + 1].inv_theta;
+  }
   // dense coarsest inverse (masked DoFs: identity in, zero out)
   {
     const int n = (int)nc;
@@ -1440,7 +1626,20 @@ int amg_sys_create(llfem_ctx* ctx, const AmgHier* h, const float* val32, float* 
 }
 
 // z = M r for one system (reliable-update restarts); partial r.z as above.
-int amg_apply_solo(llfem_ctx* ctx, AmgSys* s) { return run_vcycle(ctx, s->solo); }
+// amg_batch_apply expects amg_head's step done.
+int amg_apply_solo(llfem_ctx* ctx, AmgSys* s) { return run_vcycle(ctx, s->solo, true); }
+
+// Level 0's first Chebyshev step, for the kernel that writes its right-hand
+// side: *y = *d = inv_theta dinv b.  False: the tail kernel does it.
+bool amg_head(const AmgSys* s, float** y, float** d, const float** dinv, float* inv_theta) {
+  if (s->tail == 0) return false;
+  const MgEnt& e = s->ent[0];
+  *y = e.y;
+  *d = e.d;
+  *dinv = e.dinv;
+  *inv_theta = e.inv_theta;
+  return true;
+}
 
 struct AmgBatch {
   void* mem = nullptr;
@@ -1464,7 +1663,7 @@ int amg_batch_build(llfem_ctx* ctx, const std::vector<AmgSys*>& sys, const std::
 
 int amg_batch_apply(llfem_ctx* ctx, AmgBatch* b) {
   if (!b || b->tab.empty()) return LLFEM_OK;
-  return run_vcycle(ctx, b->tab);
+  return run_vcycle(ctx, b->tab, false);
 }
 
 bool amg_batch_any(const AmgBatch* b) { return b && !b->tab.empty(); }

@@ -72,6 +72,9 @@ struct SysDev {
   double* scal;            // [SC_N]
   double* spart;           // [nsblk] partials of a product, then [kFoldBlocks] sums of them if nsblk > kFoldMax
   double* part;            // [nvblk][2] (r.r, r.z) of a vector kernel
+  float *mgy, *mgd;        // AMG: the V-cycle's first step y = d = mgt mgdinv r goes here (NULL: the tail kernel does it)
+  const float* mgdinv;
+  float mgt;
   int32_t sblk0, nsblk, vblk0, nvblk;
   int32_t amg;             // 1: z and the r.z partials (in spart) come from the AMG V-cycle
 };
@@ -86,23 +89,53 @@ __device__ __forceinline__ double bsum(double v, double* sh) {
   return r;
 }
 
+// system of a block; the map is a dependent load that one system needs none of
+__device__ __forceinline__ const SysDev& sys_of(const SysDev* sys, const int32_t* bsys, int nsys) {
+  return sys[nsys == 1 ? 0 : bsys[blockIdx.x]];
+}
+
+// Sum of q[i * stride], i < n, over the block, eight loads under way a thread:
+// one at a time, 3,165 partials took 5 us on an idle chip.
+__device__ __forceinline__ double sum_strided(const double* q, int n, int stride, double* sh) {
+  double v = 0.0;
+  for (int i0 = threadIdx.x; i0 < n; i0 += 8 * kSB) {
+    double a[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const int i = i0 + k * kSB;
+      a[k] = i < n ? q[(int64_t)stride * i] : 0.0;
+    }
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v += a[k];
+  }
+  return bsum(v, sh);
+}
+
 // q = mask(K32 p) for RUNNING systems; partial p.q per block.
 template <typename VT>
 __global__ __launch_bounds__(kRowThreads) void k_bs_spmv(const SysDev* __restrict__ sys,
-                                                         const int32_t* __restrict__ bsys) {
+                                                         const int32_t* __restrict__ bsys, int nsys) {
   __shared__ VT sh[3 * kRowNodes];
-  const SysDev& S = sys[bsys[blockIdx.x]];
+  const SysDev& S = sys_of(sys, bsys, nsys);
+  const int lb = blockIdx.x - S.sblk0;
+  const RowSpan rs = row_span(S.N, gp(S.adj_ptr), lb);
   if (S.scal[SC_STATE] != ST_RUN) return;   // block-uniform
   const auto* __restrict__ pv = gp(static_cast<const VT*>(S.p));
-  const int lb = blockIdx.x - S.sblk0;
-  block_rows<VT>(S.N, S.nadj, gp(S.adj_ptr), gp(S.adj), gp(S.val), pv, lb, sh);
-  if (threadIdx.x >= 64) return;
   const int64_t i = (int64_t)lb * 3 * kRowNodes + threadIdx.x;
+  const bool own = threadIdx.x < 3 * kRowNodes && i < 3 * S.N;
+  VT pi = 0;
+  uint8_t fi = 1;
+  if (own) {   // loaded now, beside the product's
+    pi = pv[i];
+    fi = gp(S.fixed)[i];
+  }
+  block_rows<VT>(S.nadj, rs, gp(S.adj), gp(S.val), pv, sh);
+  if (threadIdx.x >= 64) return;
   double d = 0.0;
-  if (threadIdx.x < 3 * kRowNodes && i < 3 * S.N) {
-    const VT v = gp(S.fixed)[i] ? (VT)0 : sh[threadIdx.x];
+  if (own) {
+    const VT v = fi ? (VT)0 : sh[threadIdx.x];
     gp(static_cast<VT*>(S.q))[i] = v;
-    d = (double)pv[i] * (double)v;
+    d = (double)pi * (double)v;
   }
   d = wave_sum(d);
   if (threadIdx.x == 0) S.spart[lb] = d;
@@ -124,10 +157,7 @@ __global__ __launch_bounds__(kSB) void k_bs_fold(const SysDev* __restrict__ sys)
 
 __device__ __forceinline__ double sum_spart(const SysDev& S, double* sh) {
   const double* q = S.spart + (S.nsblk > kFoldMax ? S.nsblk : 0);
-  const int n = S.nsblk > kFoldMax ? kFoldBlocks : S.nsblk;
-  double v = 0.0;
-  for (int i = threadIdx.x; i < n; i += kSB) v += q[i];
-  return bsum(v, sh);
+  return sum_strided(q, S.nsblk > kFoldMax ? kFoldBlocks : S.nsblk, 1, sh);
 }
 
 // alpha = rho / p.q; x += alpha p; r -= alpha q; z = Dinv r; partials
@@ -139,9 +169,10 @@ __device__ __forceinline__ double sum_spart(const SysDev& S, double* sh) {
 // state before or after that, or before or after a breakdown is noted, leave
 // alike.
 template <typename VT>
-__global__ __launch_bounds__(kSB) void k_bs_update(const SysDev* __restrict__ sys, const int32_t* __restrict__ bsys) {
+__global__ __launch_bounds__(kSB) void k_bs_update(const SysDev* __restrict__ sys, const int32_t* __restrict__ bsys,
+                                                   int nsys) {
   __shared__ double sh[kSB / 64];
-  const SysDev& S = sys[bsys[blockIdx.x]];
+  const SysDev& S = sys_of(sys, bsys, nsys);
   const int lb = blockIdx.x - S.vblk0;
   const bool keeper = lb == 0 && threadIdx.x == 0;
   const double st = S.scal[SC_STATE];
@@ -149,6 +180,25 @@ __global__ __launch_bounds__(kSB) void k_bs_update(const SysDev* __restrict__ sy
     if (keeper && st == ST_PENDING) S.scal[SC_STATE] = ST_PAUSED;
     return;
   }
+  auto* __restrict__ xv = gp(static_cast<VT*>(S.x));
+  auto* __restrict__ rv = gp(static_cast<VT*>(S.r));
+  auto* __restrict__ zv = gp(static_cast<VT*>(S.z));
+  const auto* __restrict__ pv = gp(static_cast<const VT*>(S.p));
+  const auto* qv = gp(static_cast<const VT*>(S.q));   // may be mgy
+  const auto* __restrict__ dinv = gp(S.dinv);
+  int64_t j = (int64_t)lb * kVecNodes + threadIdx.x;
+  VT x[3], p[3], r[3], q[3];   // of the node under way; the first one's load beside the partials
+  auto load = [&]() {
+    if (j < S.N)
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        x[c] = xv[3 * j + c];
+        p[c] = pv[3 * j + c];
+        r[c] = rv[3 * j + c];
+        q[c] = qv[3 * j + c];
+      }
+  };
+  load();
   const double rho = S.scal[SC_RHO], pq = sum_spart(S, sh);
   if (!(pq > 0.0)) {   // breakdown (p = 0 or K not SPD on the free set): check the true residual
     if (keeper) S.scal[SC_STATE] = ST_PAUSED;
@@ -156,25 +206,26 @@ __global__ __launch_bounds__(kSB) void k_bs_update(const SysDev* __restrict__ sy
   }
   if (keeper) S.scal[SC_RHOP] = rho;
   const VT alpha = (VT)(rho / pq);
-  VT* __restrict__ xv = (VT*)gp(static_cast<VT*>(S.x));
-  VT* __restrict__ rv = (VT*)gp(static_cast<VT*>(S.r));
-  VT* __restrict__ zv = (VT*)gp(static_cast<VT*>(S.z));
-  const VT* __restrict__ pv = (const VT*)gp(static_cast<const VT*>(S.p));
-  const VT* __restrict__ qv = (const VT*)gp(static_cast<const VT*>(S.q));
-  const float* __restrict__ dinv = (const float*)gp(S.dinv);
   double rr = 0.0, rz = 0.0;
-  for (int64_t j = (int64_t)lb * kVecNodes + threadIdx.x; j < S.N; j += (int64_t)S.nvblk * kVecNodes) {
-    VT r[3];
+  for (; j < S.N; j += (int64_t)S.nvblk * kVecNodes, load()) {
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
-      const int64_t i = 3 * j + c;
-      xv[i] += alpha * pv[i];
-      r[c] = rv[i] - alpha * qv[i];
-      rv[i] = r[c];
+      xv[3 * j + c] = x[c] + alpha * p[c];
+      r[c] -= alpha * q[c];
+      rv[3 * j + c] = r[c];
+      rr += (double)r[c] * (double)r[c];
     }
+    if (S.amg) {
+      if (S.mgy)   // q, whose values are used up, is the level's y
 #pragma unroll
-    for (int c = 0; c < 3; ++c) rr += (double)r[c] * (double)r[c];
-    if (S.amg) continue;
+        for (int c = 0; c < 3; ++c) {
+          const int64_t i = 3 * j + c;
+          const float v = S.mgt * gp(S.mgdinv)[i] * (float)r[c];
+          gp(S.mgy)[i] = v;
+          gp(S.mgd)[i] = v;
+        }
+      continue;
+    }
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
       const VT z = (VT)dinv[3 * j + c] * r[c];
@@ -195,21 +246,30 @@ __global__ __launch_bounds__(kSB) void k_bs_update(const SysDev* __restrict__ sy
 // but the state, which only turns from RUN to PENDING here, and both finish
 // their iteration.
 template <typename VT>
-__global__ __launch_bounds__(kSB) void k_bs_pupd(const SysDev* __restrict__ sys, const int32_t* __restrict__ bsys) {
+__global__ __launch_bounds__(kSB) void k_bs_pupd(const SysDev* __restrict__ sys, const int32_t* __restrict__ bsys,
+                                                 int nsys) {
   __shared__ double sh[kSB / 64];
-  const SysDev& S = sys[bsys[blockIdx.x]];
+  const SysDev& S = sys_of(sys, bsys, nsys);
   const double st = S.scal[SC_STATE];
   if (st != ST_RUN && st != ST_PENDING) return;   // block-uniform
   const int lb = blockIdx.x - S.vblk0;
-  double rr = 0.0, rz = 0.0;
-  for (int i = threadIdx.x; i < S.nvblk; i += kSB) {
-    rr += S.part[2 * i];
-    if (!S.amg) rz += S.part[2 * i + 1];
-  }
-  rz = S.amg ? sum_spart(S, sh) : bsum(rz, sh);
+  auto* __restrict__ pv = gp(static_cast<VT*>(S.p));
+  const auto* __restrict__ zv = gp(static_cast<const VT*>(S.z));
+  int64_t j = (int64_t)lb * kVecNodes + threadIdx.x;
+  VT z[3], p[3];   // of the node under way; the first one's load beside the partials
+  auto load = [&]() {
+    if (j < S.N)
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        z[c] = zv[3 * j + c];
+        p[c] = pv[3 * j + c];
+      }
+  };
+  load();
   const double rho = S.scal[SC_RHOP];
+  const double rz = S.amg ? sum_spart(S, sh) : sum_strided(S.part + 1, S.nvblk, 2, sh);
   if (lb == 0) {
-    rr = bsum(rr, sh);
+    const double rr = sum_strided(S.part, S.nvblk, 2, sh);
     if (threadIdx.x == 0) {
       S.scal[SC_RHO] = rz;
       S.scal[SC_RR] = rr;
@@ -220,12 +280,10 @@ __global__ __launch_bounds__(kSB) void k_bs_pupd(const SysDev* __restrict__ sys,
         S.scal[SC_STATE] = ST_PENDING;
     }
   }
-  VT* __restrict__ pv = (VT*)gp(static_cast<VT*>(S.p));
-  const VT* __restrict__ zv = (const VT*)gp(static_cast<const VT*>(S.z));
   const VT beta = (VT)(rho != 0.0 ? rz / rho : 0.0);
-  for (int64_t j = (int64_t)lb * kVecNodes + threadIdx.x; j < S.N; j += (int64_t)S.nvblk * kVecNodes)
+  for (; j < S.N; j += (int64_t)S.nvblk * kVecNodes, load())
 #pragma unroll
-    for (int c = 0; c < 3; ++c) pv[3 * j + c] = zv[3 * j + c] + beta * pv[3 * j + c];
+    for (int c = 0; c < 3; ++c) pv[3 * j + c] = z[c] + beta * p[c];
 }
 
 __global__ void k_bs_states(const SysDev* __restrict__ sys, int nsys, double* __restrict__ out) {
@@ -794,6 +852,7 @@ int BatchSolver::rebuild_tables() {
     fold_ = fold_ || d.nsblk > kFoldMax;
     d.nvblk = (int32_t)vec_blocks(sp.N);
     d.amg = s->amg ? 1 : 0;
+    if (s->amg) (void)amg_head(s->amg, &d.mgy, &d.mgd, &d.mgdinv, &d.mgt);
     d.sblk0 = (int32_t)sb.size();
     d.vblk0 = (int32_t)vb.size();
     const int32_t id = (int32_t)dev.size();
@@ -913,19 +972,19 @@ int BatchSolver::launch_chunk(int iters) {
   const SysDev* sys = static_cast<const SysDev*>(d_sys_);
   const unsigned nf = (unsigned)(nsys_ * kFoldBlocks);
   for (int k = 0; k < iters; ++k) {
-    if (f64v_) k_bs_spmv<double><<<(unsigned)nsb_, kRowThreads, 0, st>>>(sys, d_sb_);
-    else k_bs_spmv<float><<<(unsigned)nsb_, kRowThreads, 0, st>>>(sys, d_sb_);
+    if (f64v_) k_bs_spmv<double><<<(unsigned)nsb_, kRowThreads, 0, st>>>(sys, d_sb_, nsys_);
+    else k_bs_spmv<float><<<(unsigned)nsb_, kRowThreads, 0, st>>>(sys, d_sb_, nsys_);
     if (fold_) k_bs_fold<<<nf, kSB, 0, st>>>(sys);
     if (f64v_) {
-      k_bs_update<double><<<(unsigned)nvb_, kSB, 0, st>>>(sys, d_vb_);
+      k_bs_update<double><<<(unsigned)nvb_, kSB, 0, st>>>(sys, d_vb_, nsys_);
     } else {
-      k_bs_update<float><<<(unsigned)nvb_, kSB, 0, st>>>(sys, d_vb_);
+      k_bs_update<float><<<(unsigned)nvb_, kSB, 0, st>>>(sys, d_vb_, nsys_);
       const bool amg = amg_batch_any(amgb_);
       LLFEM_TRY(amg_batch_apply(ctx_, amgb_));
       if (fold_ && amg) k_bs_fold<<<nf, kSB, 0, st>>>(sys);
     }
-    if (f64v_) k_bs_pupd<double><<<(unsigned)nvb_, kSB, 0, st>>>(sys, d_vb_);
-    else k_bs_pupd<float><<<(unsigned)nvb_, kSB, 0, st>>>(sys, d_vb_);
+    if (f64v_) k_bs_pupd<double><<<(unsigned)nvb_, kSB, 0, st>>>(sys, d_vb_, nsys_);
+    else k_bs_pupd<float><<<(unsigned)nvb_, kSB, 0, st>>>(sys, d_vb_, nsys_);
   }
   return LLFEM_OK;
 }

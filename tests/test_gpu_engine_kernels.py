@@ -13,9 +13,10 @@ from lowlevelfem import refelem as R
 pytestmark = pytest.mark.gpu
 
 
-# nodes: 8, 27, 64 (4 row blocks), 125 (13 rows left), 64,000 (4,000 blocks), 68,921 (4,308)
+# nodes: 8, 27, 64 (4 row blocks), 125 (13 rows left), 216 (all levels in the tail kernel), 343 and 729 (the fine one
+# not), 64,000 (4,000 blocks, a level between), 68,921 (4,308)
 @pytest.mark.parametrize("method", [_lib.PCG_MIXED_RELIABLE, _lib.PCG_AMG_RELIABLE])
-@pytest.mark.parametrize("n", [1, 2, 3, 4, 39, 40])
+@pytest.mark.parametrize("n", [1, 2, 3, 4, 5, 6, 8, 39, 40])
 def test_row_blocks(gpu_ctx, n, method):
     m = M.structured_box_mesh(n=n)
     dev = _lib.DeviceMesh(gpu_ctx, m.coords, m.etype, m.conn)
