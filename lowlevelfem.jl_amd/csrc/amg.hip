@@ -104,10 +104,10 @@ struct MgEnt {
   const float* xc;           // next level's x
   float *yc, *dc;            // next level's y, d and inverse diagonal (NULL: that level is in the tail)
   const float* dinvc;
-  float inv_thetac;
+  const float* chebc;        // its cheb
   const float* Ainv;         // coarsest: dense inverse [nc][nc]
   int32_t nc;
-  float inv_theta, inv_delta;
+  const float* cheb;         // 1 / theta, 1 / delta of the smoother's interval
   const double* state;       // system state word: run only while it reads 0 (NULL: always)
   double* rzpart;            // level 0: partial r.z per row block
   int32_t sblk0, nsblk, vblk0, nvblk, ablk0, nablk;
@@ -147,7 +147,7 @@ __global__ __launch_bounds__(kMB) void k_mg_cheb0(const MgEnt* __restrict__ ents
   const float* __restrict__ b = (const float*)gp(E.b);
   float* __restrict__ y = (float*)gp(E.y);
   float* __restrict__ d = (float*)gp(E.d);
-  const float it = E.inv_theta;
+  const float it = gp(E.cheb)[0];
   for (int64_t i = (int64_t)lb * kMB + threadIdx.x; i < 3 * E.N; i += (int64_t)E.nvblk * kMB) {
     const float v = it * dinv[i] * b[i];
     y[i] = v;
@@ -174,8 +174,9 @@ __global__ __launch_bounds__(kRowThreads) void k_mg_smooth(const MgEnt* __restri
   const auto* __restrict__ u = gp((const float*)(from_y ? E.y : E.x));
   const int64_t i = (int64_t)lb * 3 * kRowNodes + threadIdx.x;
   const bool own = threadIdx.x < 3 * kRowNodes && i < 3 * E.N;
-  float bi = 0.f, di = 0.f, vi = 0.f, ui = 0.f;
+  float bi = 0.f, di = 0.f, vi = 0.f, ui = 0.f, cb = 0.f;
   if (own) {   // loaded now, beside the product's
+    cb = cbt * gp(E.cheb)[0] + cbd * gp(E.cheb)[1];
     bi = gp(E.b)[i];
     di = gp(E.d)[i];
     vi = gp(E.dinv)[i];
@@ -185,7 +186,6 @@ __global__ __launch_bounds__(kRowThreads) void k_mg_smooth(const MgEnt* __restri
   if (threadIdx.x >= 64) return;
   double acc = 0.0;
   if (own) {
-    const float cb = cbt * E.inv_theta + cbd * E.inv_delta;
     const float dv = ca * di + cb * vi * (bi - sh[threadIdx.x]);
     const float wv = ui + dv;
     gp(E.d)[i] = dv;
@@ -258,7 +258,7 @@ __global__ __launch_bounds__(kMB) void k_mg_restrict(const MgEnt* __restrict__ e
       const int64_t i = 6 * a + l;
       bc[i] = v;
       if (E.yc) {   // the next level's first Chebyshev step
-        const float w = E.inv_thetac * gp(E.dinvc)[i] * v;
+        const float w = gp(E.chebc)[0] * gp(E.dinvc)[i] * v;
         gp(E.yc)[i] = w;
         gp(E.dc)[i] = w;
       }
@@ -311,7 +311,7 @@ __global__ __launch_bounds__(kTB) void k_mg_tail(const MgTail* __restrict__ tail
   const int t = threadIdx.x, l = t % kRowLanes;
   // one Chebyshev step of level E at offset o: u -> w (k_mg_smooth)
   auto smooth = [&](const MgEnt& E, int o, const ChebCoef& c, const float* u, float* w) {
-    const float cb = c.cbt * E.inv_theta + c.cbd * E.inv_delta;
+    const float cb = c.cbt * gp(E.cheb)[0] + c.cbd * gp(E.cheb)[1];
     const auto ap = gp(E.adj_ptr);
     const auto dinv = gp(E.dinv);
     for (int j = t / kRowLanes; j < (int)E.N; j += kTB / kRowLanes) {
@@ -334,7 +334,7 @@ __global__ __launch_bounds__(kTB) void k_mg_tail(const MgTail* __restrict__ tail
     const MgEnt& E = L[k];
     const int n = 3 * (int)E.N;
     for (int i = t; i < n; i += kTB) {
-      const float v = E.inv_theta * gp(E.dinv)[i] * sb[o + i];
+      const float v = gp(E.cheb)[0] * gp(E.dinv)[i] * sb[o + i];
       sy[o + i] = v;
       sd[o + i] = v;
     }
@@ -512,74 +512,191 @@ __global__ __launch_bounds__(kMB) void k_galerkin(int64_t npairs, int64_t nadjf,
   }
 }
 
-__global__ void k_mg_dinv(int64_t N, int64_t nadj, const int64_t* __restrict__ adj_ptr,
-                          const int32_t* __restrict__ dslot,
-                          const float* __restrict__ val, const uint8_t* __restrict__ mask, float* __restrict__ dinv) {
-  const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= N) return;
-  const int64_t g = adj_ptr[j] + dslot[j];
-#pragma unroll
-  for (int d = 0; d < 3; ++d) {
-    const float v = val[block32_at(nadj, g, 4 * d)];
-    dinv[3 * j + d] = (mask[3 * j + d] || !(v > 0.f)) ? 0.f : 1.f / v;
-  }
+// The smoothed levels of a system for the kernels below, one block per 16 rows
+// of any level: levels in one launch, since most of them are small and a
+// launch costs 3 us whatever it does.
+struct SetLev {
+  int64_t N, nadj;
+  const int64_t* adj_ptr;
+  const int32_t *adj, *dslot;
+  const float* val;
+  const uint8_t* mask;
+  float *dinv, *v, *y;
+};
+struct SetArgs {
+  SetLev lev[kMaxLevels];
+  int32_t first[kMaxLevels + 1];   // first block of each level, then the number of blocks
+  int32_t n;
+  double* part;                    // [blocks][2]
+};
+
+__device__ __forceinline__ int set_level(const SetArgs& S, int block) {
+  int l = 0;
+  while (l + 1 < S.n && block >= S.first[l + 1]) ++l;
+  return l;
 }
 
-__global__ void k_mg_rand(int64_t n, const float* __restrict__ dinv, float* __restrict__ v) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
+// D^-1, and the start of the power steps: pseudo-random, 0 on masked DoFs
+__global__ __launch_bounds__(64) void k_mg_start(SetArgs S) {
+  const int l = set_level(S, blockIdx.x);
+  const SetLev& E = S.lev[l];
+  const int64_t i = (int64_t)(blockIdx.x - S.first[l]) * 3 * kRowNodes + threadIdx.x;
+  if (threadIdx.x >= 3 * kRowNodes || i >= 3 * E.N) return;
+  const int64_t j = i / 3;
+  const int d = (int)(i % 3);
+  const float k = E.val[block32_at(E.nadj, E.adj_ptr[j] + E.dslot[j], 4 * d)];
+  const float di = (E.mask[i] || !(k > 0.f)) ? 0.f : 1.f / k;
+  E.dinv[i] = di;
   uint32_t h = (uint32_t)i * 2654435761u;
   h ^= h >> 15;
   h *= 2246822519u;
   h ^= h >> 13;
-  v[i] = dinv[i] > 0.f ? (float)(h & 0xFFFFu) / 65536.f - 0.5f : 0.f;
+  E.v[i] = di > 0.f ? (float)(h & 0xFFFFu) / 65536.f - 0.5f : 0.f;
 }
 
-// y = mask(A x), or with dinv D^-1 A x (one power step)
-__global__ __launch_bounds__(kRowThreads) void k_mg_spmv1(int64_t N, int64_t nadj, const int64_t* __restrict__ adj_ptr,
-                                                          const int32_t* __restrict__ adj,
-                                                          const float* __restrict__ val,
-                                                          const uint8_t* __restrict__ mask,
-                                                          const float* __restrict__ dinv,
-                                                          const float* __restrict__ x, float* __restrict__ y) {
+// One power step, D^-1 A, from v to y (or from y to v).  last: A v instead,
+// only for the partials (v.A v, v.D v) of the Rayleigh quotient.
+__global__ __launch_bounds__(kRowThreads) void k_mg_power(SetArgs S, int from_y, int last) {
   __shared__ float sh[3 * kRowNodes];
-  block_rows<float>(nadj, row_span(N, adj_ptr, blockIdx.x), adj, gp(val), x, sh);
-  const int64_t i = (int64_t)blockIdx.x * 3 * kRowNodes + threadIdx.x;
-  if (threadIdx.x < 3 * kRowNodes && i < 3 * N)
-    y[i] = dinv ? dinv[i] * sh[threadIdx.x] : mask[i] ? 0.f : sh[threadIdx.x];
+  const int l = set_level(S, blockIdx.x);
+  const SetLev& E = S.lev[l];
+  const int lb = blockIdx.x - S.first[l];
+  const auto* __restrict__ x = gp((const float*)(from_y ? E.y : E.v));
+  block_rows<float>(E.nadj, row_span(E.N, gp(E.adj_ptr), lb), gp(E.adj), gp(E.val), x, sh);
+  if (threadIdx.x >= 64) return;
+  const int64_t i = (int64_t)lb * 3 * kRowNodes + threadIdx.x;
+  const bool own = threadIdx.x < 3 * kRowNodes && i < 3 * E.N;
+  const float di = own ? gp(E.dinv)[i] : 0.f;
+  if (!last) {
+    if (own) gp(from_y ? E.v : E.y)[i] = di * sh[threadIdx.x];
+    return;
+  }
+  double a = 0.0, b = 0.0;
+  if (di > 0.f) {
+    a = (double)x[i] * sh[threadIdx.x];
+    b = (double)x[i] * x[i] / di;
+  }
+  a = wave_sum(a);
+  b = wave_sum(b);
+  if (threadIdx.x == 0) {
+    S.part[2 * (int64_t)blockIdx.x] = a;
+    S.part[2 * (int64_t)blockIdx.x + 1] = b;
+  }
 }
 
-// partial (v.y, v.D v) per block
-__global__ __launch_bounds__(kMB) void k_mg_rq(int64_t n, const float* __restrict__ v, const float* __restrict__ y,
-                                               const float* __restrict__ dinv, double* __restrict__ part) {
+// Block per level: the largest eigenvalue of D^-1 A from the partials, and the
+// smoother's 1 / theta, 1 / delta.
+__global__ __launch_bounds__(kMB) void k_mg_lambda(SetArgs S, float* __restrict__ cheb) {
   __shared__ double sh[kMB];
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int l = blockIdx.x;
   double a = 0.0, b = 0.0;
-  if (i < n && dinv[i] > 0.f) {
-    a = (double)v[i] * y[i];
-    b = (double)v[i] * v[i] / dinv[i];
+#pragma unroll 8
+  for (int64_t i = S.first[l] + threadIdx.x; i < S.first[l + 1]; i += kMB) {
+    a += S.part[2 * i];
+    b += S.part[2 * i + 1];
   }
   a = msum(a, sh);
   b = msum(b, sh);
   if (threadIdx.x == 0) {
-    part[2 * blockIdx.x] = a;
-    part[2 * blockIdx.x + 1] = b;
+    double lmb = b > 0.0 ? a / b : 0.0;
+    if (!(lmb > 0.0) || !isfinite(lmb)) lmb = 1.0;   // empty level: any positive scale
+    cheb[2 * l] = (float)(1.0 / (0.5 * (kChebHi + kChebLo) * lmb));
+    cheb[2 * l + 1] = (float)(1.0 / (0.5 * (kChebHi - kChebLo) * lmb));
   }
 }
 
-__global__ __launch_bounds__(kMB) void k_mg_sum2(int64_t nb, const double* __restrict__ part, double* __restrict__ out) {
-  __shared__ double sh[kMB];
-  double a = 0.0, b = 0.0;
-  for (int64_t i = threadIdx.x; i < nb; i += kMB) {
-    a += part[2 * i];
-    b += part[2 * i + 1];
+// Inverse of the coarsest operator, n <= 160, in one block: FP64 Gauss-Jordan on
+// the diagonal, in place, each thread a 5x5 piece of the matrix in registers
+// (rows ti + 32 r, columns tj + 32 c).  The operator is symmetric and positive
+// definite but for rounding, so no pivot is searched for; one that is not
+// clearly positive leaves *status = 1, and the host inverts with pivoting.
+// Masked DoFs: identity in, zero out.  What bounds it is the chain of n steps,
+// a barrier and a division each: 0.7 us a step, 98 us at n = 144 (265 us with a
+// pivot search and 16 waves, 250 us with 4).  On the host
+// the elimination took 0.8 ms at n = 96 and 2.8 ms at n = 144, with two copies
+// and a wait around it.
+constexpr int kInvT = 32, kInvR = 5, kInvMax = kInvT * kInvR;
+constexpr double kInvTiny = 1e-10;   // of the diagonal's original value
+
+__global__ __launch_bounds__(kInvT * kInvT) void k_mg_inverse(int n, int64_t NL, int64_t nadj,
+                                                              const int64_t* __restrict__ adj_ptr,
+                                                              const int32_t* __restrict__ adj,
+                                                              const float* __restrict__ val,
+                                                              const uint8_t* __restrict__ mask,
+                                                              float* __restrict__ Ainv, double* __restrict__ status) {
+  __shared__ double col[2][kInvMax], row[2][kInvMax];
+  __shared__ float tiny[kInvMax];
+  __shared__ uint8_t dead[kInvMax];
+  constexpr int kT = kInvT * kInvT;
+  const int t = threadIdx.x, ti = t / kInvT, tj = t % kInvT;
+  for (int i = t; i < n * n; i += kT) Ainv[i] = 0.f;   // the dense matrix passes through the result's memory
+  __syncthreads();
+  for (int64_t j = ti; j < NL; j += kInvT)
+    for (int64_t g = adj_ptr[j] + tj; g < adj_ptr[j + 1]; g += kInvT) {
+      const int64_t i = adj[g];
+      for (int e = 0; e < 9; ++e) Ainv[(3 * j + e / 3) * n + 3 * i + e % 3] = val[block32_at(nadj, g, e)];
+    }
+  __syncthreads();
+  for (int i = t; i < n; i += kT) {
+    const float d = Ainv[i * n + i];
+    dead[i] = mask[i] || !(d > 0.f);
+    tiny[i] = dead[i] ? 0.f : (float)kInvTiny * d;
   }
-  a = msum(a, sh);
-  b = msum(b, sh);
-  if (threadIdx.x == 0) {
-    out[0] = a;
-    out[1] = b;
+  __syncthreads();
+  double a[kInvR][kInvR];
+#pragma unroll
+  for (int r = 0; r < kInvR; ++r)
+#pragma unroll
+    for (int c = 0; c < kInvR; ++c) {
+      const int i = ti + kInvT * r, j = tj + kInvT * c;
+      a[r][c] = 0.0;
+      if (i < n && j < n) a[r][c] = dead[i] || dead[j] ? (i == j ? 1.0 : 0.0) : (double)Ainv[i * n + j];
+    }
+  __syncthreads();   // Ainv is written again only after this
+  for (int k = 0; k < n; ++k) {
+    double* C = col[k & 1];   // two of each: the step before may still be read
+    double* R = row[k & 1];
+#pragma unroll
+    for (int q = 0; q < kInvR; ++q)
+      if (q == k / kInvT) {   // column k and row k out, 0 in their place
+        if (tj == k % kInvT)
+#pragma unroll
+          for (int r = 0; r < kInvR; ++r) C[ti + kInvT * r] = a[r][q];
+        if (ti == k % kInvT)
+#pragma unroll
+          for (int c = 0; c < kInvR; ++c) R[tj + kInvT * c] = a[q][c];
+        if (tj == k % kInvT)
+#pragma unroll
+          for (int r = 0; r < kInvR; ++r) a[r][q] = 0.0;
+        if (ti == k % kInvT)
+#pragma unroll
+          for (int c = 0; c < kInvR; ++c) a[q][c] = 0.0;
+      }
+    __syncthreads();
+    const double d = C[k];
+    if (!(d > (double)tiny[k])) {   // the same in every thread
+      if (t == 0) *status = 1.0;
+      return;
+    }
+    const double inv = 1.0 / d;
+    double rs[kInvR];
+#pragma unroll
+    for (int c = 0; c < kInvR; ++c) rs[c] = tj + kInvT * c == k ? inv : R[tj + kInvT * c] * inv;
+#pragma unroll
+    for (int r = 0; r < kInvR; ++r) {
+      const double f = ti + kInvT * r == k ? -1.0 : C[ti + kInvT * r];
+#pragma unroll
+      for (int c = 0; c < kInvR; ++c) a[r][c] -= f * rs[c];
+    }
   }
+#pragma unroll
+  for (int r = 0; r < kInvR; ++r)
+#pragma unroll
+    for (int c = 0; c < kInvR; ++c) {
+      const int i = ti + kInvT * r, j = tj + kInvT * c;
+      if (i < n && j < n) Ainv[i * n + j] = dead[i] || dead[j] ? 0.f : (float)a[r][c];
+    }
+  if (t == 0) *status = 0.0;
 }
 
 // per block: the largest off-diagonal block norm of node j, then strong flags
@@ -1236,8 +1353,9 @@ struct AmgSys {
   void* mem = nullptr;
   size_t bytes = 0;
   std::vector<MgEnt> ent;          // one per level (the last: coarsest)
-  MgEnt* d_solo = nullptr;         // device copy of `ent` with state = NULL (restarts)
+  double* status = nullptr;        // device word: 1 = k_mg_inverse has left the inverse to the host
   void* solo_tab = nullptr;
+  std::vector<char> solo_src;      // host source of solo_tab's upload
   size_t solo_bytes = 0;
   struct Tab {
     MgEnt* ents = nullptr;
@@ -1250,7 +1368,6 @@ struct AmgSys {
   };
   int tail = 0;                      // first level in the tail kernel
   std::vector<Tab> solo;
-  std::vector<double> lambda;
 };
 
 namespace {
@@ -1313,7 +1430,10 @@ void tab_add(TabBuild& T, const AmgSys* s, const double* state) {
   }
 }
 
-int tab_upload(llfem_ctx* ctx, const TabBuild& T, void** mem, size_t* bytes, std::vector<AmgSys::Tab>* out) {
+// The tables in one copy.  src keeps their host source until the caller has
+// next waited for the stream.
+int tab_upload(llfem_ctx* ctx, const TabBuild& T, void** mem, size_t* bytes, std::vector<char>* src,
+               std::vector<AmgSys::Tab>* out) {
   size_t need = 0;
   auto al = [](size_t b) { return (b + 255) / 256 * 256; };
   for (size_t l = 0; l < T.ents.size(); ++l)
@@ -1328,16 +1448,14 @@ int tab_upload(llfem_ctx* ctx, const TabBuild& T, void** mem, size_t* bytes, std
     LLFEM_TRY(dmalloc(ctx, mem, need * 2));
     *bytes = need * 2;
   }
-  hipStream_t st = ctx->stream;
-  char* m = static_cast<char*>(*mem);
   out->assign(T.ents.size(), AmgSys::Tab{});
-  auto put = [&](const void* src, size_t b) -> char* {
-    char* p = m;
-    if (b) {
-      if (hipMemcpyAsync(p, src, b, hipMemcpyHostToDevice, st) != hipSuccess) return nullptr;
-    }
-    m += al(b);
-    return p;
+  src->resize(need);
+  size_t ofs = 0;
+  auto put = [&](const void* p, size_t b) -> char* {
+    if (b) std::memcpy(src->data() + ofs, p, b);
+    char* d = static_cast<char*>(*mem) + ofs;
+    ofs += al(b);
+    return d;
   };
   for (size_t l = 0; l < T.ents.size(); ++l) {
     AmgSys::Tab& t = (*out)[l];
@@ -1352,9 +1470,8 @@ int tab_upload(llfem_ctx* ctx, const TabBuild& T, void** mem, size_t* bytes, std
     t.smap = reinterpret_cast<int32_t*>(put(T.smap[l].data(), 4 * T.smap[l].size()));
     t.vmap = reinterpret_cast<int32_t*>(put(T.vmap[l].data(), 4 * T.vmap[l].size()));
     t.amap = reinterpret_cast<int32_t*>(put(T.amap[l].data(), 4 * T.amap[l].size()));
-    if (!t.ents || !t.tents || !t.tails || !t.smap || !t.vmap || !t.amap) return fail(LLFEM_EHIP, "AMG: table upload failed");
   }
-  LLFEM_HIP(hipStreamSynchronize(st));   // host tables go out of scope
+  LLFEM_HIP(hipMemcpyAsync(*mem, src->data(), ofs, hipMemcpyHostToDevice, ctx->stream));
   return LLFEM_OK;
 }
 
@@ -1430,6 +1547,41 @@ bool invert_dense(int n, std::vector<double>& A) {
   return true;
 }
 
+// Inverse of a coarsest operator that k_mg_inverse cannot hold (more than 26
+// aggregates: coarsening stalled) or that is near singular.
+int host_inverse(llfem_ctx* ctx, const AmgHier* h, const float* val, float* Ainv, double* status) {
+  hipStream_t st = ctx->stream;
+  const auto& D = h->lev.back();
+  const int n = (int)(3 * D.N);
+  std::vector<float> cval((size_t)9 * D.nadj);
+  LLFEM_HIP(hipMemcpyAsync(cval.data(), val, sizeof(float) * cval.size(), hipMemcpyDeviceToHost, st));
+  LLFEM_HIP(hipMemsetAsync(status, 0, sizeof(double), st));
+  LLFEM_HIP(hipStreamSynchronize(st));
+  std::vector<double> A((size_t)n * n, 0.0);
+  for (int64_t j = 0; j < D.N; ++j)
+    for (int64_t g = h->c_adj_ptr[j]; g < h->c_adj_ptr[j + 1]; ++g) {
+      const int64_t i = h->c_adj[g];
+      for (int c = 0; c < 3; ++c)
+        for (int d = 0; d < 3; ++d)
+          A[(size_t)(3 * j + c) * n + 3 * i + d] = cval[block32_at(D.nadj, g, 3 * c + d)];
+    }
+  std::vector<uint8_t> dead(n, 0);   // masked DoFs: identity in, zero out
+  for (int i = 0; i < n; ++i) dead[i] = h->c_mask[i] || !(A[(size_t)i * n + i] > 0.0);
+  for (int i = 0; i < n; ++i)
+    if (dead[i]) {
+      for (int k = 0; k < n; ++k) A[(size_t)i * n + k] = A[(size_t)k * n + i] = 0.0;
+      A[(size_t)i * n + i] = 1.0;
+    }
+  if (!invert_dense(n, A)) return fail(LLFEM_EINVAL, "AMG: singular coarsest operator");
+  std::vector<float> Af((size_t)n * n);
+  for (int i = 0; i < n; ++i)
+    for (int k = 0; k < n; ++k)
+      Af[(size_t)i * n + k] = (dead[i] || dead[k]) ? 0.f : (float)A[(size_t)i * n + k];
+  LLFEM_HIP(hipMemcpyAsync(Ainv, Af.data(), sizeof(float) * Af.size(), hipMemcpyHostToDevice, st));
+  LLFEM_HIP(hipStreamSynchronize(st));
+  return LLFEM_OK;
+}
+
 }  // namespace
 
 void amg_sys_free(llfem_ctx* ctx, AmgSys* s) {
@@ -1457,8 +1609,9 @@ int amg_sys_create(llfem_ctx* ctx, const AmgHier* h, const float* val32, float* 
   for (int l = 1; l <= L; ++l)
     need += al(4 * 9 * (size_t)h->lev[l].nadj) + 5 * al(4 * 3 * (size_t)h->lev[l].N);
   need += al(4 * (size_t)nc * nc);
-  const int64_t maxn = 3 * h->lev[0].N;
-  need += al(sizeof(double) * (2 * (size_t)nblk(maxn) + 2 * (size_t)(L + 1) + 8));
+  int64_t nset = 0;   // row blocks of the smoothed levels
+  for (int l = 0; l < L; ++l) nset += row_groups(h->lev[l].N);
+  need += al(sizeof(double) * (2 * (size_t)nset + (size_t)(L + 1) + 8));
   s->bytes = need;
   int rc = dmalloc(ctx, &s->mem, need);
   if (rc != LLFEM_OK) {
@@ -1518,8 +1671,9 @@ int amg_sys_create(llfem_ctx* ctx, const AmgHier* h, const float* val32, float* 
   }
   s->ent[0].rzpart = rzpart;
   float* Ainv = (float*)take(4 * (size_t)nc * nc);
-  double* part = (double*)take(sizeof(double) * (2 * (size_t)nblk(maxn) + 2 * (size_t)(L + 1) + 8));
-  double* lam = part + 2 * (size_t)nblk(maxn);
+  double* part = (double*)take(sizeof(double) * (2 * (size_t)nset + (size_t)(L + 1) + 8));
+  s->status = part + 2 * nset;
+  float* cheb = (float*)(s->status + 1);
   if ((size_t)(m - static_cast<char*>(s->mem)) > s->bytes) {
     amg_sys_free(ctx, s);
     return fail(LLFEM_EINVAL, "AMG: workspace layout overflow");
@@ -1534,89 +1688,46 @@ int amg_sys_create(llfem_ctx* ctx, const AmgHier* h, const float* val32, float* 
       k_galerkin<16><<<nblk(16 * D.npairs), kMB, 0, st>>>(D.npairs, D.nadj, h->lev[l + 1].nadj, D.gptr, D.gblk, D.gcol,
                                                           D.adj, D.Q, val[l], D.pair_o, val[l + 1]);
   }
-  for (int l = 0; l <= L; ++l) {
-    const auto& D = h->lev[l];
-    k_mg_dinv<<<nblk(D.N), kMB, 0, st>>>(D.N, D.nadj, D.adj_ptr, D.dslot, val[l], D.mask, dinv[l]);
-  }
-  // largest eigenvalue of D^-1 A per smoothed level (power steps, Rayleigh quotient)
+  // inverse diagonals; largest eigenvalue of D^-1 A per smoothed level (power
+  // steps, Rayleigh quotient)
+  SetArgs S{};
+  S.n = L;
+  S.part = part;
   for (int l = 0; l < L; ++l) {
     const auto& D = h->lev[l];
-    const MgEnt& e = s->ent[l];
-    const int64_t n = 3 * D.N;
-    float* v = e.d;
-    float* y = e.y;
-    k_mg_rand<<<nblk(n), kMB, 0, st>>>(n, dinv[l], v);
-    for (int k = 0; k < kPowerSteps; ++k) {   // D^-1 A, back and forth between the two arrays
-      k_mg_spmv1<<<(unsigned)row_groups(D.N), kRowThreads, 0, st>>>(D.N, D.nadj, D.adj_ptr, D.adj, val[l], D.mask,
-                                                                    dinv[l], v, y);
-      std::swap(v, y);
-    }
-    k_mg_spmv1<<<(unsigned)row_groups(D.N), kRowThreads, 0, st>>>(D.N, D.nadj, D.adj_ptr, D.adj, val[l], D.mask,
-                                                                  nullptr, v, y);
-    k_mg_rq<<<nblk(n), kMB, 0, st>>>(n, v, y, dinv[l], part);
-    k_mg_sum2<<<1, kMB, 0, st>>>(nblk(n), part, lam + 2 * l);
+    S.lev[l] = {D.N, D.nadj, D.adj_ptr, D.adj, D.dslot, val[l], D.mask, dinv[l], s->ent[l].d, s->ent[l].y};
+    S.first[l + 1] = S.first[l] + (int32_t)row_groups(D.N);
+    s->ent[l].cheb = cheb + 2 * l;
   }
-  std::vector<double> hl(2 * (size_t)(L + 1), 0.0);
-  std::vector<float> cval((size_t)9 * h->lev[L].nadj);
-  hipError_t e = hipMemcpyAsync(hl.data(), lam, sizeof(double) * 2 * L, hipMemcpyDeviceToHost, st);
-  if (e == hipSuccess)
-    e = hipMemcpyAsync(cval.data(), val[L], sizeof(float) * cval.size(), hipMemcpyDeviceToHost, st);
-  if (e == hipSuccess) e = hipStreamSynchronize(st);
-  if (e == hipSuccess) e = hipGetLastError();
-  if (e != hipSuccess) {
-    amg_sys_free(ctx, s);
-    return fail(LLFEM_EHIP, std::string("AMG set-up: ") + hipGetErrorString(e));
-  }
-  s->lambda.assign(L, 0.0);
-  for (int l = 0; l < L; ++l) {
-    double lmb = hl[2 * l + 1] > 0 ? hl[2 * l] / hl[2 * l + 1] : 0.0;
-    if (!(lmb > 0.0) || !std::isfinite(lmb)) lmb = 1.0;   // empty level: any positive scale
-    s->lambda[l] = lmb;
-    s->ent[l].inv_theta = (float)(1.0 / (0.5 * (kChebHi + kChebLo) * lmb));
-    s->ent[l].inv_delta = (float)(1.0 / (0.5 * (kChebHi - kChebLo) * lmb));
-  }
+  k_mg_start<<<(unsigned)nset, 64, 0, st>>>(S);
+  int from_y = 0;
+  for (int k = 0; k < kPowerSteps; ++k, from_y ^= 1) k_mg_power<<<(unsigned)nset, kRowThreads, 0, st>>>(S, from_y, 0);
+  k_mg_power<<<(unsigned)nset, kRowThreads, 0, st>>>(S, from_y, 1);
+  k_mg_lambda<<<(unsigned)L, kMB, 0, st>>>(S, cheb);
   for (int l = 0; l + 1 < s->tail; ++l) {
     s->ent[l].yc = s->ent[l + 1].y;
     s->ent[l].dc = s->ent[l + 1].d;
     s->ent[l].dinvc = s->ent[l + 1].dinv;
-    s->ent[l].inv_thetac = s->ent[l + 1].inv_theta;
+    s->ent[l].chebc = s->ent[l + 1].cheb;
   }
-  // dense coarsest inverse (masked DoFs: identity in, zero out)
-  {
-    const int n = (int)nc;
-    std::vector<double> A((size_t)n * n, 0.0);
-    const int64_t NL = h->lev[L].N;
-    for (int64_t j = 0; j < NL; ++j)
-      for (int64_t g = h->c_adj_ptr[j]; g < h->c_adj_ptr[j + 1]; ++g) {
-        const int64_t i = h->c_adj[g];
-        for (int c = 0; c < 3; ++c)
-          for (int d = 0; d < 3; ++d)
-            A[(size_t)(3 * j + c) * n + 3 * i + d] = cval[block32_at(h->lev[L].nadj, g, 3 * c + d)];
-      }
-    std::vector<uint8_t> dead(n, 0);
-    for (int i = 0; i < n; ++i) dead[i] = h->c_mask[i] || !(A[(size_t)i * n + i] > 0.0);
-    for (int i = 0; i < n; ++i)
-      if (dead[i]) {
-        for (int k = 0; k < n; ++k) A[(size_t)i * n + k] = A[(size_t)k * n + i] = 0.0;
-        A[(size_t)i * n + i] = 1.0;
-      }
-    if (!invert_dense(n, A)) {
+  s->ent[L].Ainv = Ainv;
+  s->ent[L].nc = (int32_t)nc;
+  if (nc <= kInvMax) {
+    const auto& D = h->lev[L];
+    k_mg_inverse<<<1, kInvT * kInvT, 0, st>>>((int)nc, D.N, D.nadj, D.adj_ptr, D.adj, val[L], D.mask, Ainv, s->status);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) {
       amg_sys_free(ctx, s);
-      return fail(LLFEM_EINVAL, "AMG: singular coarsest operator");
+      return fail(LLFEM_EHIP, std::string("AMG set-up: ") + hipGetErrorString(e));
     }
-    std::vector<float> Af((size_t)n * n);
-    for (int i = 0; i < n; ++i)
-      for (int k = 0; k < n; ++k)
-        Af[(size_t)i * n + k] = (dead[i] || dead[k]) ? 0.f : (float)A[(size_t)i * n + k];
-    LLFEM_HIP(hipMemcpyAsync(Ainv, Af.data(), sizeof(float) * Af.size(), hipMemcpyHostToDevice, st));
-    s->ent[L].Ainv = Ainv;
-    s->ent[L].nc = n;
-    LLFEM_HIP(hipStreamSynchronize(st));
+  } else if ((rc = host_inverse(ctx, h, val[L], Ainv, s->status)) != LLFEM_OK) {
+    amg_sys_free(ctx, s);
+    return rc;
   }
   // restart tables (this system alone, always runs)
   TabBuild T;
   tab_add(T, s, nullptr);
-  rc = tab_upload(ctx, T, &s->solo_tab, &s->solo_bytes, &s->solo);
+  rc = tab_upload(ctx, T, &s->solo_tab, &s->solo_bytes, &s->solo_src, &s->solo);
   if (rc != LLFEM_OK) {
     amg_sys_free(ctx, s);
     return rc;
@@ -1630,18 +1741,19 @@ int amg_sys_create(llfem_ctx* ctx, const AmgHier* h, const float* val32, float* 
 int amg_apply_solo(llfem_ctx* ctx, AmgSys* s) { return run_vcycle(ctx, s->solo, true); }
 
 // Level 0's first Chebyshev step, for the kernel that writes its right-hand
-// side: *y = *d = inv_theta dinv b.  False: the tail kernel does it.
-bool amg_head(const AmgSys* s, float** y, float** d, const float** dinv, float* inv_theta) {
+// side: *y = *d = theta[0] dinv b.  False: the tail kernel does it.
+bool amg_head(const AmgSys* s, float** y, float** d, const float** dinv, const float** theta) {
   if (s->tail == 0) return false;
   const MgEnt& e = s->ent[0];
   *y = e.y;
   *d = e.d;
   *dinv = e.dinv;
-  *inv_theta = e.inv_theta;
+  *theta = e.cheb;
   return true;
 }
 
 struct AmgBatch {
+  std::vector<char> src;
   void* mem = nullptr;
   size_t bytes = 0;
   std::vector<AmgSys::Tab> tab;
@@ -1658,7 +1770,7 @@ int amg_batch_build(llfem_ctx* ctx, const std::vector<AmgSys*>& sys, const std::
     (*b)->tab.clear();
     return LLFEM_OK;
   }
-  return tab_upload(ctx, T, &(*b)->mem, &(*b)->bytes, &(*b)->tab);
+  return tab_upload(ctx, T, &(*b)->mem, &(*b)->bytes, &(*b)->src, &(*b)->tab);
 }
 
 int amg_batch_apply(llfem_ctx* ctx, AmgBatch* b) {
@@ -1674,7 +1786,12 @@ void amg_batch_free(llfem_ctx* ctx, AmgBatch* b) {
   delete b;
 }
 
-const std::vector<double>& amg_lambda(const AmgSys* s) { return s->lambda; }
+const double* amg_status(const AmgSys* s) { return s->status; }
+
+int amg_host_inverse(llfem_ctx* ctx, AmgSys* s) {
+  const MgEnt& e = s->ent.back();
+  return host_inverse(ctx, s->h, e.val, const_cast<float*>(e.Ainv), s->status);
+}
 
 int amg_build(llfem_ctx* ctx, const SysSpec& sp, const double* d_xyz, AmgHier** out) {
   using clk = std::chrono::steady_clock;

@@ -350,7 +350,9 @@ int amg_sys_create(llfem_ctx* ctx, const AmgHier* h, const float* val32, float* 
                    double* rzpart, AmgSys** out);
 void amg_sys_free(llfem_ctx* ctx, AmgSys* s);
 int amg_apply_solo(llfem_ctx* ctx, AmgSys* s);
-bool amg_head(const AmgSys* s, float** y, float** d, const float** dinv, float* inv_theta);
+bool amg_head(const AmgSys* s, float** y, float** d, const float** dinv, const float** theta);
+const double* amg_status(const AmgSys* s);   // device word: not 0 = amg_host_inverse has to finish the set-up
+int amg_host_inverse(llfem_ctx* ctx, AmgSys* s);
 int amg_batch_build(llfem_ctx* ctx, const std::vector<AmgSys*>& sys, const std::vector<const double*>& states,
                     AmgBatch** b);
 int amg_batch_apply(llfem_ctx* ctx, AmgBatch* b);

@@ -72,9 +72,8 @@ struct SysDev {
   double* scal;            // [SC_N]
   double* spart;           // [nsblk] partials of a product, then [kFoldBlocks] sums of them if nsblk > kFoldMax
   double* part;            // [nvblk][2] (r.r, r.z) of a vector kernel
-  float *mgy, *mgd;        // AMG: the V-cycle's first step y = d = mgt mgdinv r goes here (NULL: the tail kernel does it)
-  const float* mgdinv;
-  float mgt;
+  float *mgy, *mgd;        // AMG: the V-cycle's first step y = d = mgt[0] mgdinv r goes here (NULL: the tail kernel does it)
+  const float *mgdinv, *mgt;
   int32_t sblk0, nsblk, vblk0, nvblk;
   int32_t amg;             // 1: z and the r.z partials (in spart) come from the AMG V-cycle
 };
@@ -220,7 +219,7 @@ __global__ __launch_bounds__(kSB) void k_bs_update(const SysDev* __restrict__ sy
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
           const int64_t i = 3 * j + c;
-          const float v = S.mgt * gp(S.mgdinv)[i] * (float)r[c];
+          const float v = gp(S.mgt)[0] * gp(S.mgdinv)[i] * (float)r[c];
           gp(S.mgy)[i] = v;
           gp(S.mgd)[i] = v;
         }
@@ -650,8 +649,14 @@ int BatchSolver::update_many(const std::vector<SolveSys*>& ss, bool init) {
     }
     LLFEM_HIP(hipMemcpyAsync(h + 4 * i, s->scal + SC_N - 1, sizeof(double), hipMemcpyDeviceToHost, st));
     LLFEM_HIP(hipMemcpyAsync(h + 4 * i + 1, s->scal + SC_ITER, sizeof(double), hipMemcpyDeviceToHost, st));
+    h[4 * i + 2] = 0.0;
+    if (init && s->amg)   // the set-up has been enqueued only
+      LLFEM_HIP(hipMemcpyAsync(h + 4 * i + 2, amg_status(s->amg), sizeof(double), hipMemcpyDeviceToHost, st));
   }
   LLFEM_HIP(hipStreamSynchronize(st));
+  if (init)
+    for (size_t i = 0; i < m; ++i)
+      if (h[4 * i + 2] != 0.0) LLFEM_TRY(amg_host_inverse(ctx_, ss[i]->amg));
   // 2. adoption or rollback.  LLFEM_ENGINE_FORCE_ROLLBACK=k treats the k-th
   // update's trial as not finite (a host-side switch for testing the
   // rollback path).
