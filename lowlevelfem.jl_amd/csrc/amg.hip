@@ -168,33 +168,43 @@ __global__ __launch_bounds__(kRowThreads) void k_mg_smooth(const MgEnt* __restri
                                                            float cbt, float cbd, int from_y, int rz) {
   __shared__ float sh[3 * kRowNodes];
   const MgEnt& E = mg_ent(ents, map, nent);
-  const int lb = blockIdx.x - E.sblk0;
-  const RowSpan rs = row_span(E.N, gp(E.adj_ptr), lb);
-  if (mg_skip(E)) return;
-  const auto* __restrict__ u = gp((const float*)(from_y ? E.y : E.x));
+  const int lb = blockIdx.x - pinned(E.sblk0);
+  const int64_t N = pinned(E.N), nadj = pinned(E.nadj);
+  const auto ap = gp(pinned(E.adj_ptr));
+  const auto adj = gp(pinned(E.adj));
+  const auto val = gp(pinned(E.val));
+  const double* const state = pinned(E.state);
+  float *const ex = pinned(E.x), *const ey = pinned(E.y), *const ed = pinned(E.d);
+  const float *const eb = pinned(E.b), *const edinv = pinned(E.dinv), *const echeb = pinned(E.cheb);
+  double* const erz = pinned(E.rzpart);
+  const double st = state ? *gp(state) : 0.0;
+  const RowSpan rs = row_span(N, ap, lb);
+  if (st != 0.0) return;
+  const auto* __restrict__ u = gp((const float*)(from_y ? ey : ex));
   const int64_t i = (int64_t)lb * 3 * kRowNodes + threadIdx.x;
-  const bool own = threadIdx.x < 3 * kRowNodes && i < 3 * E.N;
-  float bi = 0.f, di = 0.f, vi = 0.f, ui = 0.f, cb = 0.f;
+  const bool own = threadIdx.x < 3 * kRowNodes && i < 3 * N;
+  const float c0 = gp(echeb)[0], c1 = gp(echeb)[1];
+  float bi = 0.f, di = 0.f, vi = 0.f, ui = 0.f;
   if (own) {   // loaded now, beside the product's
-    cb = cbt * gp(E.cheb)[0] + cbd * gp(E.cheb)[1];
-    bi = gp(E.b)[i];
-    di = gp(E.d)[i];
-    vi = gp(E.dinv)[i];
+    bi = gp(eb)[i];
+    di = gp(ed)[i];
+    vi = gp(edinv)[i];
     ui = u[i];
   }
-  block_rows<float>(E.nadj, rs, gp(E.adj), gp(E.val), u, sh);
+  block_rows<float>(nadj, rs, adj, val, u, sh);
   if (threadIdx.x >= 64) return;
   double acc = 0.0;
   if (own) {
+    const float cb = cbt * c0 + cbd * c1;
     const float dv = ca * di + cb * vi * (bi - sh[threadIdx.x]);
     const float wv = ui + dv;
-    gp(E.d)[i] = dv;
-    gp(from_y ? E.x : E.y)[i] = wv;
+    gp(ed)[i] = dv;
+    gp(from_y ? ex : ey)[i] = wv;
     acc = (double)bi * (double)wv;
   }
   if (rz) {
     acc = wave_sum(acc);
-    if (threadIdx.x == 0) gp(E.rzpart)[lb] = acc;
+    if (threadIdx.x == 0) gp(erz)[lb] = acc;
   }
 }
 
@@ -203,20 +213,29 @@ __global__ __launch_bounds__(kRowThreads) void k_mg_resid(const MgEnt* __restric
                                                           const int32_t* __restrict__ map, int nent, int from_y) {
   __shared__ float sh[3 * kRowNodes];
   const MgEnt& E = mg_ent(ents, map, nent);
-  const int lb = blockIdx.x - E.sblk0;
-  const RowSpan rs = row_span(E.N, gp(E.adj_ptr), lb);
-  if (mg_skip(E)) return;
-  const auto* __restrict__ u = gp((const float*)(from_y ? E.y : E.x));
+  const int lb = blockIdx.x - pinned(E.sblk0);
+  const int64_t N = pinned(E.N), nadj = pinned(E.nadj);
+  const auto ap = gp(pinned(E.adj_ptr));
+  const auto adj = gp(pinned(E.adj));
+  const auto val = gp(pinned(E.val));
+  const double* const state = pinned(E.state);
+  float *const ex = pinned(E.x), *const ey = pinned(E.y);
+  const float* const eb = pinned(E.b);
+  const uint8_t* const emask = pinned(E.mask);
+  const double st = state ? *gp(state) : 0.0;
+  const RowSpan rs = row_span(N, ap, lb);
+  if (st != 0.0) return;
+  const auto* __restrict__ u = gp((const float*)(from_y ? ey : ex));
   const int64_t i = (int64_t)lb * 3 * kRowNodes + threadIdx.x;
-  const bool own = threadIdx.x < 3 * kRowNodes && i < 3 * E.N;
+  const bool own = threadIdx.x < 3 * kRowNodes && i < 3 * N;
   float bi = 0.f;
   uint8_t mi = 1;
   if (own) {
-    bi = gp(E.b)[i];
-    mi = gp(E.mask)[i];
+    bi = gp(eb)[i];
+    mi = gp(emask)[i];
   }
-  block_rows<float>(E.nadj, rs, gp(E.adj), gp(E.val), u, sh);
-  if (own) gp(from_y ? E.x : E.y)[i] = mi ? 0.f : bi - sh[threadIdx.x];
+  block_rows<float>(nadj, rs, adj, val, u, sh);
+  if (own) gp(from_y ? ex : ey)[i] = mi ? 0.f : bi - sh[threadIdx.x];
 }
 
 // bc = Q^T r, r in y (in_y) or x: kMG lanes per aggregate stride over its

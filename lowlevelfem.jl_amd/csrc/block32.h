@@ -63,14 +63,22 @@ struct RowSpan {
   int R;
 };
 
-// The span is loaded before a kernel checks whether its system runs, so that
-// the two loads, 0.6 us each on an idle chip, go together.
+// Loaded without a branch, so that the load of the system's state can be under
+// way with it (0.6 us each on an idle chip).
 template <typename AdjPtr>
 __device__ __forceinline__ RowSpan row_span(int64_t N, AdjPtr adj_ptr, int64_t lb) {
-  const int64_t j = lb * kRowNodes + threadIdx.x / kRowLanes;
-  if (j >= N) return {0, 0};
-  const int64_t p0 = adj_ptr[j];
-  return {p0, (int)(adj_ptr[j + 1] - p0)};
+  const int64_t j = lb * kRowNodes + threadIdx.x / kRowLanes, i = j < N ? j : N - 1;
+  const int64_t p0 = adj_ptr[i], p1 = adj_ptr[i + 1];
+  return {p0, j < N ? (int)(p1 - p0) : 0};
+}
+
+// A wave-uniform value that has to be in its registers here: the fields of a
+// table entry are fetched together at the kernel's start instead of one by one
+// where they are first used, each a wait of 0.1 us.
+template <typename T>
+__device__ __forceinline__ T pinned(T v) {
+  asm volatile("" : "+s"(v));
+  return v;
 }
 
 // The rows of one block's kRowNodes nodes: y[3 n + c] = sum_t block(t) x, into

@@ -116,28 +116,36 @@ __global__ __launch_bounds__(kRowThreads) void k_bs_spmv(const SysDev* __restric
                                                          const int32_t* __restrict__ bsys, int nsys) {
   __shared__ VT sh[3 * kRowNodes];
   const SysDev& S = sys_of(sys, bsys, nsys);
-  const int lb = blockIdx.x - S.sblk0;
-  const RowSpan rs = row_span(S.N, gp(S.adj_ptr), lb);
-  if (S.scal[SC_STATE] != ST_RUN) return;   // block-uniform
-  const auto* __restrict__ pv = gp(static_cast<const VT*>(S.p));
+  const int lb = blockIdx.x - pinned(S.sblk0);
+  const int64_t N = pinned(S.N), nadj = pinned(S.nadj);
+  const auto ap = gp(pinned(S.adj_ptr));
+  const auto adj = gp(pinned(S.adj));
+  const auto val = gp(pinned(S.val));
+  const auto* __restrict__ pv = gp(static_cast<const VT*>(pinned(S.p)));
+  VT* const q = static_cast<VT*>(pinned(S.q));
+  const uint8_t* const fixed = pinned(S.fixed);
+  double* const spart = pinned(S.spart);
+  const double st = gp(pinned(S.scal))[SC_STATE];
+  const RowSpan rs = row_span(N, ap, lb);
+  if (st != ST_RUN) return;   // block-uniform
   const int64_t i = (int64_t)lb * 3 * kRowNodes + threadIdx.x;
-  const bool own = threadIdx.x < 3 * kRowNodes && i < 3 * S.N;
+  const bool own = threadIdx.x < 3 * kRowNodes && i < 3 * N;
   VT pi = 0;
   uint8_t fi = 1;
   if (own) {   // loaded now, beside the product's
     pi = pv[i];
-    fi = gp(S.fixed)[i];
+    fi = gp(fixed)[i];
   }
-  block_rows<VT>(S.nadj, rs, gp(S.adj), gp(S.val), pv, sh);
+  block_rows<VT>(nadj, rs, adj, val, pv, sh);
   if (threadIdx.x >= 64) return;
   double d = 0.0;
   if (own) {
     const VT v = fi ? (VT)0 : sh[threadIdx.x];
-    gp(static_cast<VT*>(S.q))[i] = v;
+    gp(q)[i] = v;
     d = (double)pi * (double)v;
   }
   d = wave_sum(d);
-  if (threadIdx.x == 0) S.spart[lb] = d;
+  if (threadIdx.x == 0) gp(spart)[lb] = d;
 }
 
 // spart of systems with more than kFoldMax product blocks -> kFoldBlocks sums
