@@ -48,3 +48,23 @@ def test_mass(gpu_ctx, elem, order, cells, perturb, deg):
         _lib.assemble_batch([(dev, _lib.OP_STIFFNESS, tab, {}), (dev, _lib.OP_MASS, tab, dict(rho=2.5, lumped=True))])
         close(dev.values(_lib.OP_MASS, lumped=True), refl)
         close(dev.values(_lib.OP_STIFFNESS), K0)
+
+
+# the lumped sums leave for the host while the panel launches run on one or two
+# side streams: the values written by them are whole for the call that follows
+@pytest.mark.parametrize("streams", ["1", "2", "3"])
+@pytest.mark.parametrize("elem,order,n", [("hex", 1, 1), ("tet", 2, 12), ("hex", 2, 6)])
+def test_lumped_beside_panels(gpu_ctx, monkeypatch, elem, order, n, streams):
+    m = M.structured_box_mesh(n=n, elem=elem, order=order)
+    tab = R.rule_tables(m.etype, 2 * order + 1)
+    dev = _lib.DeviceMesh(gpu_ctx, m.coords, m.etype, m.conn)
+    ref, _ = dev.assemble(_lib.OP_MASS, tab, rho=2.5)
+    monkeypatch.setenv("LLFEM_PANEL_STREAMS", streams)
+    refl = O.mass_legacy(m, tab, rho=2.5, lumped=True).diagonal()
+    for _ in range(3):
+        lum, st = dev.assemble(_lib.OP_MASS, tab, rho=2.5, lumped=True)
+        assert np.abs(lum - refl).max() <= 1e-13 * np.abs(refl).max()
+        assert st.kernel_ms >= st.main_kernel_ms > 0.0
+        twice, _ = dev.assemble(_lib.OP_MASS, tab, rho=2.5, accumulate=True)
+        assert np.array_equal(twice, 2.0 * ref)
+    dev.close()
