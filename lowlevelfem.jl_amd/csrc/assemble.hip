@@ -542,15 +542,25 @@ int assemble_impl(llfem_mesh* m, const llfem_op_desc* d, double* nzval_out, llfe
   const bool rounds_on =
       !std::getenv("LLFEM_PANEL_NO_ROUNDS") && !(tuned != ctx->tune.end() && tuned->second.rounds == 0);
   nstreams = std::min<int>(nstreams, (int)plan.size());
-  const int first_side = lump && nstreams > 0 ? 0 : 1;   // side stream s - first_side stands for stream s; below 0: st
-  if (lump) nstreams = std::min(nstreams, 2);
+  // Values for the host: the launches go in parts and the copy of a part runs
+  // beside the next one's.  The parts cost 70 us of launches and waits, so it
+  // takes long launches: us per call whole and in parts, curved hex27 36 MB
+  // 1068 and 1035, 99 MB 2487 and 2302, hex8 27 MB 712 and 746, 52 MB 1295 and
+  // 1266, tet10 45 MB 1130 and 1157, 80 MB 1854 and 1830; affine tet10 45 MB
+  // 1102 and 1136, 130 MB 2810 and 2800, 253 MB 5248 and 5152, hex8 104 MB 2265
+  // and 2248.
+  const size_t split_bytes = size_t(affine ? 96 : 48) << 20;
+  const bool split = nzval_out && !lump && !plan.empty() && sizeof(double) * (size_t)nnz >= split_bytes;
+  const int parts = split ? kParts : 1;
+  const bool on_side = (lump || split) && nstreams > 0;   // the launches leave st to the copy
+  const int first_side = on_side ? 0 : 1;   // side stream s - first_side stands for stream s; below 0: st
+  if (on_side) nstreams = std::min(nstreams, 2);
   auto stream = [&](int s) { return s < first_side ? st : ctx->side[s - first_side]; };
   // per launch: kernel, waves per block, LDS, grid, and resident waves per CU
   struct Cfg {
     PanelFn fn;
     int wpb;
     size_t lds_bytes;
-    unsigned blocks;
     double cost;   // steps / resident waves per CU: the launch's time alone, in relative units
   };
   std::vector<Cfg> cfg(plan.size());
@@ -585,11 +595,9 @@ int assemble_impl(llfem_mesh* m, const llfem_op_desc* d, double* nzval_out, llfe
     if (const char* env = std::getenv("LLFEM_PANEL_WPB")) want_wpb = std::atoi(env);   // A/B knob
     if (want_wpb > 0 && (size_t)want_wpb <= max_wpb && (size_t)want_wpb * wave_bytes + block_extra <= kLdsPerCU)
       wpb = want_wpb;
-    const int64_t used = (L.waves + wpb - 1) / wpb;
     Cfg& c = cfg[li];
     c.fn = lfn;
     c.wpb = wpb;
-    c.blocks = (unsigned)((used + kXcds - 1) / kXcds * kXcds);   // see k_panel
     c.lds_bytes = wave_bytes * wpb + block_extra;
     const size_t res = std::max<size_t>(1, resident_waves(lfn, wave_bytes, block_extra, wpb));
     c.cost = (double)L.waves * L.rounds * L.cnt / (double)res;
@@ -633,28 +641,48 @@ int assemble_impl(llfem_mesh* m, const llfem_op_desc* d, double* nzval_out, llfe
     LLFEM_HIP(hipEventRecord(ctx->fork_ev, st));   // after the geometry
     for (int k = first_side; k < nstreams; ++k) LLFEM_HIP(hipStreamWaitEvent(stream(k), ctx->fork_ev, 0));
   }
-  for (size_t li : issue) {
-    const PanelLaunch& L = plan[li];
-    const Cfg& c = cfg[li];
-    hipStream_t ls = stream(stream_of[li]);
-    P.rec = static_cast<const uint8_t*>(m->d_rec) + L.rec_base * m->rec_bytes;
-    P.desc = m->d_desc + L.desc_base;
-    P.waves = L.waves;
-    P.rounds = L.rounds;
-    P.cnt = L.cnt;
-    P.max_r = L.max_r;
-    P.lds_per_wave = npw * L.max_r * blkl + 9;   // + dummy block
-    hipLaunchKernelGGL(c.fn, dim3(c.blocks), dim3(64 * c.wpb), c.lds_bytes, ls, P);
-  }
-  LLFEM_HIP(hipGetLastError());
-  for (int k = 1; k < nstreams; ++k) {   // join
-    LLFEM_HIP(hipEventRecord(ctx->join_ev[k - 1], stream(k)));
-    LLFEM_HIP(hipStreamWaitEvent(stream(0), ctx->join_ev[k - 1], 0));
-  }
-  if (!highorder) LLFEM_HIP(hipEventRecord(ctx->ev[2], stream(0)));
-  if (acc) {   // resident += this call's values (group order: the earlier groups first)
-    k_add_into<<<(unsigned)((nnz + 255) / 256), 256, 0, st>>>(nnz, acc_tmp, *outp);
+  CopyGate gate[kParts] = {};
+  for (int part = 0; part < parts; ++part) {
+    for (size_t li : issue) {
+      const PanelLaunch& L = plan[li];
+      const Cfg& c = cfg[li];
+      const int64_t w0 = part == 0 ? 0 : L.cut[part - 1], w1 = part + 1 == parts ? L.waves : L.cut[part];
+      if (w1 <= w0) continue;
+      const int64_t slot0 = w0 * L.rounds * npw;   // node slots of the waves before
+      P.rec = static_cast<const uint8_t*>(m->d_rec) + (L.rec_base + slot0 * L.cnt) * m->rec_bytes;
+      P.desc = m->d_desc + L.desc_base + slot0;
+      P.waves = w1 - w0;
+      P.rounds = L.rounds;
+      P.cnt = L.cnt;
+      P.max_r = L.max_r;
+      P.lds_per_wave = npw * L.max_r * blkl + 9;   // + dummy block
+      const int64_t used = (P.waves + c.wpb - 1) / c.wpb;
+      hipLaunchKernelGGL(c.fn, dim3((unsigned)((used + kXcds - 1) / kXcds * kXcds)), dim3(64 * c.wpb), c.lds_bytes,
+                         stream(stream_of[li]), P);   // whole kXcds: see k_panel
+    }
     LLFEM_HIP(hipGetLastError());
+    const bool last = part + 1 == parts;
+    if (last || acc)
+      for (int k = 1; k < nstreams; ++k) {   // join
+        LLFEM_HIP(hipEventRecord(ctx->join_ev[k - 1], stream(k)));
+        LLFEM_HIP(hipStreamWaitEvent(stream(0), ctx->join_ev[k - 1], 0));
+      }
+    if (last && !highorder) LLFEM_HIP(hipEventRecord(ctx->ev[2], stream(0)));
+    if (acc) {   // resident += this call's values (group order: the earlier groups first)
+      const int64_t i0 = part == 0 ? 0 : blk * m->part_adj[part - 1], i1 = last ? nnz : blk * m->part_adj[part];
+      if (i1 > i0)
+        k_add_into<<<(unsigned)((i1 - i0 + 255) / 256), 256, 0, stream(0)>>>(i1 - i0, acc_tmp + i0, *outp + i0);
+      LLFEM_HIP(hipGetLastError());
+    }
+    if (split) {
+      gate[part].end = last ? (size_t)nnz : (size_t)(blk * m->part_adj[part]);
+      for (int k = 0; k < (acc ? 1 : nstreams); ++k) {
+        hipEvent_t& e = ctx->gate_ev[part][k];
+        if (!e) LLFEM_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+        LLFEM_HIP(hipEventRecord(e, stream(k)));
+        gate[part].ev[k] = e;
+      }
+    }
   }
   LLFEM_HIP(hipEventRecord(ctx->ev[3], stream(0)));
   if (dev_out) {
@@ -683,13 +711,12 @@ int assemble_impl(llfem_mesh* m, const llfem_op_desc* d, double* nzval_out, llfe
       m->have_lumped = complete && d->lumped != 0;
     }
   }
-  if (lump) {
-    const int rc = nzval_out ? copy_to_host(ctx, nzval_out, m->d_lumped, 3 * (size_t)m->N) : LLFEM_OK;
-    LLFEM_HIP(hipStreamWaitEvent(st, ctx->ev[3], 0));   // later work on the stream follows the panels
-    LLFEM_TRY(rc);
-  } else if (nzval_out) {
-      LLFEM_TRY(copy_to_host(ctx, nzval_out, acc ? *outp : target, (size_t)nnz));
-  }
+  int rc = LLFEM_OK;
+  if (nzval_out && lump) rc = copy_to_host(ctx, nzval_out, m->d_lumped, 3 * (size_t)m->N);
+  else if (nzval_out)
+    rc = copy_to_host(ctx, nzval_out, acc ? *outp : target, (size_t)nnz, gate, split ? parts : 0);
+  if (on_side) LLFEM_HIP(hipStreamWaitEvent(st, ctx->ev[3], 0));   // later work on the stream follows the panels
+  LLFEM_TRY(rc);
   LLFEM_HIP(hipEventSynchronize(ctx->ev[3]));
   if (stats) {
     float ms = 0.f, ms_main = 0.f;

@@ -51,6 +51,10 @@ inline int fail(int code, const std::string& msg) {
 // One panel-kernel launch.  Nodes of similar incidence count are grouped
 // (padded with null steps to `cnt`), laid out in processing order as
 // per-step records so a wavefront streams `rounds` nodes per lane group.
+// A large assembly whose values go to the host is issued in kParts parts of the
+// values, so that the first part's copy runs beside the others' launches.
+constexpr int kParts = 3;
+
 struct PanelLaunch {
   int64_t rec_base;     // first record of the launch
   int64_t desc_base;    // first node descriptor of the launch
@@ -59,6 +63,9 @@ struct PanelLaunch {
   int32_t rounds;       // nodes per lane group (per wavefront stream)
   int32_t max_r;        // LDS panel rows per lane group
   int32_t nodes;        // real nodes in the launch
+  // waves [0, cut[k]) write every panel of the launch before the mesh's
+  // part_adj[k] (the last part ends with the launch)
+  int32_t cut[kParts - 1];
 };
 
 // Per-rule geometry state: affine detection is a property of the mesh and
@@ -115,6 +122,7 @@ struct llfem_ctx {
   void* ws = nullptr;
   size_t ws_bytes = 0;
   bool ws_busy = false;
+  hipEvent_t gate_ev[llfem::kParts][2] = {};       // a part's panels are written (one event per side stream)
   double* d_sink = nullptr;                        // 64 doubles: target of padding-lane panel stores
   // pinned staging of device-to-host copies and the threads that empty it
   // (copy_to_host), made on first use
@@ -154,6 +162,7 @@ struct llfem_mesh {
   int2* d_desc = nullptr;         // {adj offset, R} per node slot
   int64_t desc_count = 0;
   std::vector<llfem::PanelLaunch> launches;
+  int64_t part_adj[llfem::kParts - 1] = {};   // adjacency slot where each part but the last ends
   int32_t max_r = 0;
   // host copies kept for pattern export
   std::vector<int64_t> h_adj_ptr;
@@ -205,7 +214,13 @@ namespace llfem {
 int dmalloc(llfem_ctx* ctx, void** p, size_t bytes);
 // n doubles from device memory to pageable host memory, after the work
 // already queued on the context's stream; returns when dst holds them.
-int copy_to_host(llfem_ctx* ctx, double* dst, const double* src, size_t n);
+// src[0 .. end) is valid on ctx->stream once the events have happened.
+struct CopyGate {
+  size_t end;             // elements
+  hipEvent_t ev[2];       // NULL: none
+};
+int copy_to_host(llfem_ctx* ctx, double* dst, const double* src, size_t n, const CopyGate* gates = nullptr,
+                 int ngates = 0);
 void dfree(llfem_ctx* ctx, void* p, size_t bytes);
 
 template <typename T>

@@ -175,7 +175,9 @@ class CopyPool {
 // transfer), small ones last (what is left for the threads after the last has
 // arrived).  PCIe bound, 57 GB/s.  HIP's own pageable path takes 18 GB/s:
 //   64 KB 39 -> 11 us, 4 MB 236 -> 120, 50 MB 2.97 -> 1.06 ms, 124 MB 7.4 -> 2.5.
-int copy_to_host(llfem_ctx* ctx, double* dst_, const double* src_, size_t n) {
+// gates (ascending, the last one covers all): chunks end where a gate does, and
+// the first chunk behind a gate's predecessor waits for the gate.
+int copy_to_host(llfem_ctx* ctx, double* dst_, const double* src_, size_t n, const CopyGate* gates, int ngates) {
   constexpr size_t kOneCopy = size_t(512) << 10, kSmall = size_t(4) << 20, kSlot = size_t(16) << 20;
   constexpr size_t kSlots = CopyPool::kSlots;
   const size_t bytes = n * sizeof(double);
@@ -194,21 +196,32 @@ int copy_to_host(llfem_ctx* ctx, double* dst_, const double* src_, size_t n) {
   };
   LLFEM_TRY(slot(0));
   if (bytes <= kOneCopy) {
+    for (int g = 0; g < ngates; ++g)
+      for (hipEvent_t e : gates[g].ev)
+        if (e) LLFEM_HIP(hipStreamWaitEvent(st, e, 0));
     LLFEM_HIP(hipMemcpyAsync(ctx->h_stage[0], src, bytes, hipMemcpyDeviceToHost, st));
     LLFEM_HIP(hipStreamSynchronize(st));
     std::memcpy(dst, ctx->h_stage[0], bytes);
     return LLFEM_OK;
   }
   std::vector<std::pair<size_t, size_t>> chunk;   // offset, length
+  int g = 0;
   for (size_t off = 0; off < bytes;) {
+    while (g < ngates && gates[g].end * sizeof(double) <= off) ++g;
     const size_t left = bytes - off;
-    const size_t len = std::min(left, std::min(kSlot, std::max(kSmall, left / 4 / kSmall * kSmall)));
+    size_t len = std::min(left, std::min(kSlot, std::max(kSmall, left / 4 / kSmall * kSmall)));
+    if (g < ngates) len = std::min(len, gates[g].end * sizeof(double) - off);
     chunk.push_back({off, len});
     off += len;
   }
+  int opened = 0;   // gates waited for
   auto issue = [&](size_t i) -> int {
     const size_t s = i % kSlots;
     LLFEM_TRY(slot(s));
+    const size_t end = (chunk[i].first + chunk[i].second) / sizeof(double);
+    for (; opened < ngates && (opened == 0 || gates[opened - 1].end < end); ++opened)
+      for (hipEvent_t e : gates[opened].ev)
+        if (e) LLFEM_HIP(hipStreamWaitEvent(st, e, 0));
     LLFEM_HIP(hipMemcpyAsync(ctx->h_stage[s], src + chunk[i].first, chunk[i].second, hipMemcpyDeviceToHost, st));
     LLFEM_HIP(hipEventRecord(ctx->stage_ev[s], st));
     return LLFEM_OK;
@@ -389,6 +402,9 @@ int llfem_ctx_destroy(llfem_ctx* ctx) {
   if (ctx->h_poll) (void)hipHostFree(ctx->h_poll);
   for (auto& e : ctx->poll_ev)
     if (e) (void)hipEventDestroy(e);
+  for (auto& part : ctx->gate_ev)
+    for (auto& e : part)
+      if (e) (void)hipEventDestroy(e);
   delete ctx->pool;
   for (size_t b = 0; b < sizeof(ctx->h_stage) / sizeof(ctx->h_stage[0]); ++b) {
     if (ctx->h_stage[b]) (void)hipHostFree(ctx->h_stage[b]);

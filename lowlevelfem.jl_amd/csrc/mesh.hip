@@ -220,15 +220,26 @@ int build_records(llfem_mesh* m, const std::vector<int32_t>& h_inc_ptr) {
   int64_t rec_total = 0, desc_total = 0;
   std::vector<std::pair<int64_t, int64_t>> ranges;   // order ranges of the launches
   const int64_t ncu = std::max(1, ctx->num_cus);
+  // parts of the values: the first one small, so that its copy starts early;
+  // each copy (57 GB/s) then outlasts the next part's panels (150 GB/s and up)
+  int64_t part_node[kParts - 1];
+  const double kShare[kParts - 1] = {0.125, 0.5};
+  for (int k = 0; k < kParts - 1; ++k) {
+    const auto it = std::lower_bound(m->h_adj_ptr.begin(), m->h_adj_ptr.begin() + N, (int64_t)(kShare[k] * m->nadj));
+    part_node[k] = it - m->h_adj_ptr.begin();
+    m->part_adj[k] = *it;
+  }
   for (int64_t p = 0; p < (int64_t)order.size();) {
     const int32_t cmin = count(order[p]);
     int64_t q = p;
     int32_t cmax = cmin, rmax = 0;
+    std::vector<int64_t> run;   // where the launch's further counts begin
     while (q < (int64_t)order.size()) {
       const int32_t c = count(order[q]);
       // merge while the padded steps stay within 25% of the smallest count,
       // or while the launch is still tiny
       if (c > cmax && c * 4 > cmin * 5 && (q - p) >= 4096) break;
+      if (q > p && c != count(order[q - 1])) run.push_back(q);
       cmax = std::max(cmax, c);
       rmax = std::max(rmax, rows(order[q]));
       ++q;
@@ -256,6 +267,14 @@ int build_records(llfem_mesh* m, const std::vector<int32_t>& h_inc_ptr) {
     L.rounds = (int32_t)G;
     L.max_r = rmax;
     L.nodes = (int32_t)nodes;
+    // ascending nodes within the launch, so that its waves write the values in order
+    run.push_back(q);
+    for (size_t i = 0; i + 1 < run.size(); ++i)
+      std::inplace_merge(order.begin() + p, order.begin() + run[i], order.begin() + run[i + 1]);
+    for (int k = 0; k < kParts - 1; ++k) {
+      const int64_t before = std::lower_bound(order.begin() + p, order.begin() + q, part_node[k]) - (order.begin() + p);
+      L.cut[k] = (int32_t)((before + per_wave - 1) / per_wave);
+    }
     m->launches.push_back(L);
     ranges.push_back({p, q});
     rec_total += slots * cmax;
