@@ -34,7 +34,6 @@ constexpr int kG = 8;   // lanes per row the workspace's partial count is sized 
 constexpr int64_t kFoldMax = 2048;
 constexpr unsigned kFoldBlocks = 64;
 constexpr int64_t kMaxPasses = 8;
-constexpr int64_t kFuseMax = 30000;   // DoFs up to which pcg forms the direction inside the SpMV
 
 // S_RHO0 / S_RHO1: r.z of even / odd iterations (the p-update reads one and
 // writes the other, so no block sees the new value in place of the old).
@@ -76,20 +75,42 @@ __device__ __forceinline__ double2 block_sum2(double a, double b, double* sh) {
   return make_double2(ra, rb);
 }
 
-// Sum of n partials, or of n pairs of them; the same order in every block.
-__device__ __forceinline__ double sum_partials(int64_t n, const double* __restrict__ part, double* sh) {
+// This thread's share of n partials, or of n pairs of them; the same order in
+// every block.  Eight loads under way at a time: one by one, 2,048 partials
+// are a chain of eight loads, 0.6 us each on an idle chip.  Loads only, so a
+// kernel can issue them before it knows whether the solve is done.
+__device__ __forceinline__ double own_partials(int64_t n, const double* __restrict__ part) {
   double s = 0.0;
-  for (int64_t i = threadIdx.x; i < n; i += kBS) s += part[i];
-  return block_sum(s, sh);
+  for (int64_t i0 = threadIdx.x; i0 < n; i0 += 8 * kBS) {
+    double a[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) a[k] = i0 + k * kBS < n ? part[i0 + k * kBS] : 0.0;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) s += a[k];
+  }
+  return s;
+}
+__device__ __forceinline__ double2 own_pairs(int64_t n, const double* __restrict__ part) {
+  const double2* const q = reinterpret_cast<const double2*>(part);
+  double2 s = make_double2(0.0, 0.0);
+  for (int64_t i0 = threadIdx.x; i0 < n; i0 += 8 * kBS) {
+    double2 a[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) a[k] = i0 + k * kBS < n ? q[i0 + k * kBS] : make_double2(0.0, 0.0);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      s.x += a[k].x;
+      s.y += a[k].y;
+    }
+  }
+  return s;
+}
+__device__ __forceinline__ double sum_partials(int64_t n, const double* __restrict__ part, double* sh) {
+  return block_sum(own_partials(n, part), sh);
 }
 __device__ __forceinline__ double2 sum_pairs(int64_t n, const double* __restrict__ part, double* sh) {
-  double a = 0.0, b = 0.0;
-  for (int64_t i = threadIdx.x; i < n; i += kBS) {
-    const double2 v = reinterpret_cast<const double2*>(part)[i];
-    a += v.x;
-    b += v.y;
-  }
-  return block_sum2(a, b, sh);
+  const double2 s = own_pairs(n, part);
+  return block_sum2(s.x, s.y, sh);
 }
 
 // Blocks are dealt round-robin to the 8 XCDs; neighbouring rows share most of
@@ -104,9 +125,12 @@ __device__ __forceinline__ int64_t xcd_block() {
 // What an SpMV multiplies: a vector as it stands, ...
 template <typename VT>
 struct Plain {
+  using Raw = VT;   // what is loaded of an entry, before begin()
   const VT* __restrict__ x;
+  __device__ __forceinline__ void fetch() {}
   __device__ __forceinline__ bool begin(double*) { return true; }
-  __device__ __forceinline__ VT at(int64_t i) const { return x[i]; }
+  __device__ __forceinline__ Raw raw(int64_t i) const { return x[i]; }
+  __device__ __forceinline__ VT value(Raw v) const { return v; }
   __device__ __forceinline__ void keep(int64_t, VT) const {}
 };
 
@@ -125,11 +149,21 @@ struct Direction {
   int64_t np, it, maxiter;
   volatile double* done_host;
   VT beta;
+  double2 own;
+  double rho;
+  struct Raw {
+    VT z, p;
+  };
+  __device__ __forceinline__ void fetch() {   // the loads of begin()
+    if (it == 0) return;
+    own = own_pairs(np, part);
+    rho = scal[S_RHO0 + (int)((it - 1) & 1)];
+  }
   __device__ __forceinline__ bool begin(double* sh) {
     beta = 0;
     if (it == 0) return true;   // p = z, rho from k_init_scal
-    const double2 s = sum_pairs(np, part, sh);
-    beta = (VT)(s.y / scal[S_RHO0 + (int)((it - 1) & 1)]);
+    const double2 s = block_sum2(own.x, own.y, sh);
+    beta = (VT)(s.y / rho);
     const bool done = s.x <= scal[S_TOL2] || it >= maxiter;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
       scal[S_RHO0 + (int)(it & 1)] = s.y;
@@ -142,7 +176,8 @@ struct Direction {
     }
     return !done;
   }
-  __device__ __forceinline__ VT at(int64_t i) const { return it == 0 ? z[i] : z[i] + beta * pold[i]; }
+  __device__ __forceinline__ Raw raw(int64_t i) const { return {z[i], it == 0 ? (VT)0 : pold[i]}; }
+  __device__ __forceinline__ VT value(Raw v) const { return v.z + beta * v.p; }
   __device__ __forceinline__ void keep(int64_t i, VT v) const { pnew[i] = v; }
 };
 
@@ -160,21 +195,30 @@ __global__ __launch_bounds__(kBS) void k_spmv(int64_t N, int passes, const int64
                                              const uint8_t* __restrict__ fixed, VT* __restrict__ y,
                                              double* __restrict__ part, const double* __restrict__ scal) {
   __shared__ double sh[2 * kWaves];
-  if (scal && scal[S_DONE] != 0.0) return;
-  if (!xs.begin(sh)) return;
   const int64_t lb = xcd_block();
   const int l = (int)(threadIdx.x % G);
+  int64_t j = lb * passes * (kBS / G) + threadIdx.x / G;
+  int64_t p0 = 0;
+  int R = 0;
+  auto span = [&]() {
+    const int64_t i = j < N ? j : N - 1;
+    p0 = adj_ptr[i];
+    R = j < N ? (int)(adj_ptr[i + 1] - p0) : 0;
+  };
+  const double done = scal ? scal[S_DONE] : 0.0;
+  xs.fetch();
+  span();
+  if (done != 0.0) return;
+  if (!xs.begin(sh)) return;
   double d = 0.0;
-  for (int ps = 0; ps < passes; ++ps) {
-    const int64_t j = (lb * passes + ps) * (kBS / G) + threadIdx.x / G;
+  for (int ps = 0; ps < passes; ++ps, j += kBS / G, span()) {
     VT a0 = 0, a1 = 0, a2 = 0;
-    if (j < N) {
-      const int64_t p0 = adj_ptr[j];
-      const int R = (int)(adj_ptr[j + 1] - p0);
+    {
       const MT* P = val + 9 * p0;
       for (int s = l; s < R; s += G) {
         const int64_t i = adj[p0 + s];
-        const VT x0 = xs.at(3 * i), x1 = xs.at(3 * i + 1), x2 = xs.at(3 * i + 2);
+        const auto r0 = xs.raw(3 * i), r1 = xs.raw(3 * i + 1), r2 = xs.raw(3 * i + 2);
+        const VT x0 = xs.value(r0), x1 = xs.value(r1), x2 = xs.value(r2);
         a0 += (VT)P[3 * s] * x0 + (VT)P[3 * s + 1] * x1 + (VT)P[3 * s + 2] * x2;
         a1 += (VT)P[3 * R + 3 * s] * x0 + (VT)P[3 * R + 3 * s + 1] * x1 + (VT)P[3 * R + 3 * s + 2] * x2;
         a2 += (VT)P[6 * R + 3 * s] * x0 + (VT)P[6 * R + 3 * s + 1] * x1 + (VT)P[6 * R + 3 * s + 2] * x2;
@@ -190,7 +234,7 @@ __global__ __launch_bounds__(kBS) void k_spmv(int64_t N, int passes, const int64
       const VT r = l == 0 ? a0 : l == 1 ? a1 : a2;
       const int64_t i = 3 * j + l;
       const VT v = (fixed && fixed[i]) ? (VT)0 : r;
-      const VT xv = xs.at(i);
+      const VT xv = xs.value(xs.raw(i));
       y[i] = v;
       xs.keep(i, xv);
       d += (double)xv * (double)v;
@@ -236,15 +280,27 @@ __global__ __launch_bounds__(kBS) void k_update(int64_t n, const double* __restr
                                                const VT* __restrict__ q, const VT* __restrict__ dinv,
                                                VT* __restrict__ z, double* __restrict__ part) {
   __shared__ double sh[2 * kWaves];
-  if (scal[S_DONE] != 0.0) return;
-  const VT alpha = (VT)(scal[S_RHO0 + par] / sum_partials(np, pq, sh));
+  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  VT xi = 0, pi = 0, ri = 0, qi = 0, di = 0;   // of the entry under way; the first one's load beside the partials
+  auto load = [&]() {
+    if (i < n) {
+      xi = x[i];
+      pi = p[i];
+      ri = r[i];
+      qi = q[i];
+      di = dinv[i];
+    }
+  };
+  load();
+  const double done = scal[S_DONE], rho = scal[S_RHO0 + par], own = own_partials(np, pq);
+  if (done != 0.0) return;
+  const VT alpha = (VT)(rho / block_sum(own, sh));
   double rr = 0.0, rz = 0.0;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    x[i] += alpha * p[i];
-    const VT ri = r[i] - alpha * q[i];
+  for (; i < n; i += (int64_t)gridDim.x * blockDim.x, load()) {
+    x[i] = xi + alpha * pi;
+    ri -= alpha * qi;
     r[i] = ri;
-    const VT zi = dinv[i] * ri;
+    const VT zi = di * ri;
     z[i] = zi;
     rr += (double)ri * (double)ri;
     rz += (double)ri * (double)zi;
@@ -263,9 +319,19 @@ __global__ __launch_bounds__(kBS) void k_pupd(int64_t n, double* __restrict__ sc
                                              const VT* __restrict__ z, VT* __restrict__ p,
                                              volatile double* done_host) {
   __shared__ double sh[2 * kWaves];
-  if (scal[S_DONE] != 0.0) return;
-  const double2 s = sum_pairs(np, part, sh);   // r.r, r.z
-  const double rho = scal[S_RHO0 + (int)(it & 1)];
+  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  VT zi = 0, pi = 0;   // of the entry under way; the first one's load beside the partials
+  auto load = [&]() {
+    if (i < n) {
+      zi = z[i];
+      pi = p[i];
+    }
+  };
+  load();
+  const double done = scal[S_DONE], rho = scal[S_RHO0 + (int)(it & 1)];
+  const double2 own = own_pairs(np, part);
+  if (done != 0.0) return;
+  const double2 s = block_sum2(own.x, own.y, sh);   // r.r, r.z
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     scal[S_RHO0 + (int)(~it & 1)] = s.y;
     scal[S_RR] = s.x;
@@ -276,9 +342,7 @@ __global__ __launch_bounds__(kBS) void k_pupd(int64_t n, double* __restrict__ sc
     }
   }
   const VT beta = (VT)(s.y / rho);
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x)
-    p[i] = z[i] + beta * p[i];
+  for (; i < n; i += (int64_t)gridDim.x * blockDim.x, load()) p[i] = zi + beta * pi;
 }
 
 // init: x = 0; r = b; z = dinv r; p = z; partials (r.r, r.z)
@@ -394,24 +458,30 @@ __global__ __launch_bounds__(kBS) void k_spmv_csc(int64_t n, int passes, const i
                                                  double* __restrict__ part,
                                                  const double* __restrict__ scal) {
   __shared__ double sh[2 * kWaves];
-  if (scal && scal[S_DONE] != 0.0) return;
-  if (!xs.begin(sh)) return;
   const int64_t lb = xcd_block();
   const int l = (int)(threadIdx.x % G);
+  int64_t j = lb * passes * (kBS / G) + threadIdx.x / G;
+  int64_t p0 = 0, p1 = 0;
+  auto span = [&]() {
+    const int64_t i = j < n ? j : n - 1;
+    p0 = colptr[i];
+    p1 = j < n ? colptr[i + 1] : 0;
+  };
+  const double done = scal ? scal[S_DONE] : 0.0;
+  xs.fetch();
+  span();
+  if (done != 0.0) return;
+  if (!xs.begin(sh)) return;
   double d = 0.0;
-  for (int ps = 0; ps < passes; ++ps) {
-    const int64_t j = (lb * passes + ps) * (kBS / G) + threadIdx.x / G;
+  for (int ps = 0; ps < passes; ++ps, j += kBS / G, span()) {
     VT acc = 0;
-    if (j < n) {
-      const int64_t p1 = colptr[j + 1];
 #pragma unroll 4
-      for (int64_t p = colptr[j] + l; p < p1; p += G) acc += (VT)val[p] * xs.at(rowval[p]);
-    }
+    for (int64_t p = p0 + l; p < p1; p += G) acc += (VT)val[p] * xs.value(xs.raw(rowval[p]));
 #pragma unroll
     for (int o = G / 2; o > 0; o >>= 1) acc += __shfl_xor(acc, o, G);
     if (j < n && l == 0) {
       const VT v = (fixed && fixed[j]) ? (VT)0 : acc;
-      const VT xv = xs.at(j);
+      const VT xv = xs.value(xs.raw(j));
       y[j] = v;
       xs.keep(j, xv);
       d += (double)xv * (double)v;
@@ -449,6 +519,7 @@ inline int panel_lanes(int64_t N, int64_t nadj) { return nadj >= 20 * N ? 32 : n
 inline int csc_lanes(int64_t n, int64_t nnz) { return nnz >= 48 * n ? 32 : nnz >= 16 * n ? 16 : kG; }
 
 struct PanelOp {
+  static constexpr int64_t kFuseMax = 40000;   // DoFs up to which pcg forms the direction inside the SpMV
   int64_t N;
   const int64_t* adj_ptr;
   const int32_t* adj;
@@ -473,6 +544,7 @@ struct PanelOp {
 };
 
 struct CscOp {
+  static constexpr int64_t kFuseMax = 24000;
   int64_t n;
   const int64_t* colptr;
   const int32_t* rowval;
@@ -535,13 +607,16 @@ struct Scratch {   // partial sums + scalars
 // is overwritten (it is the second direction array once r holds it).
 // The scalars stay on the device and each kernel sums the partials it needs,
 // so an iteration is two launches -- SpMV of the direction formed on the fly,
-// update -- up to kFuseMax DoFs, and three above, where gathering two vectors
-// costs the SpMV more than the p-update's own launch and pass.  Whole solves,
-// three / two launches: panels of 5,400 DoFs 2.18 / 1.85 ms, 28,611 4.50 /
-// 4.19, 139,725 33.3 / 38.1; CSC 5,400 2.10 / 1.85, 28,611 5.10 / 4.98, 35,547
-// 12.3 / 13.8.  With seven launches an iteration (separate reductions and
-// scalars, a host wait every 16) it was 50 ms at 139,725 DoFs (panels) and
-// 4.8 ms at 5,400 (CSC).
+// update -- up to the operator's kFuseMax DoFs, and three above, where gathering
+// two vectors costs the SpMV more than the p-update's own launch and pass.
+// Whole solves in ms, three / two launches: panels of 5,400 DoFs 3.39 / 2.73,
+// 19,575 6.30 / 5.12, 30,345 7.78 / 6.43, 40,071 8.70 / 7.40, 44,403 14.1 /
+// 14.6, 139,725 48.3 / 55.0; CSC 5,400 3.27 / 3.06, 19,575 7.63 / 6.79, 28,611
+// 14.3 / 15.0, 30,345 10.4 / 10.1, 37,281 20.2 / 21.6.  With seven launches an
+// iteration (separate reductions and scalars, a host wait every 16) the 12x11x40
+// tet10 box (139,725 DoFs) to 1e-12 took 50 ms and a 5,400-DoF CSC 4.8 ms, with
+// two or three 35.8 and 2.0; loads issued before the partials are summed and the
+// done flag is seen, and eight partials under way a thread: 33.4 and 1.9.
 // The host keeps two batches queued and looks at the flag after the older one,
 // so the device never waits for it.
 template <typename Op, typename MT, typename VT>
@@ -556,7 +631,7 @@ int pcg(llfem_ctx* ctx, const Op& K, const MT* val, const uint8_t* fixed, const 
   const int passes = need <= kMaxPasses ? (int)need : 1;
   const unsigned gs = (unsigned)((groups + passes - 1) / passes);
   const bool fold = (int64_t)gs > kFoldMax;
-  const bool fuse = n <= kFuseMax;
+  const bool fuse = n <= Op::kFuseMax;
   volatile double* flag = ctx->h_poll;
   *flag = 0.0;
   k_init<VT><<<gv, kBS, 0, st>>>(n, x, b, r, dinv, z, p, S.part);
