@@ -42,7 +42,8 @@ namespace llfem {
 namespace {
 
 constexpr int kSB = 256;                 // threads per block
-constexpr int kSG = 8;                   // lanes per node row in the FP64 product of an update
+constexpr int kSG = 32;                  // lanes per node row in the FP64 product of an update (8: 1,040 us at
+                                        // 2.1 M nodes and 9.8 at 3,887, 32: 987 and 5.9)
 constexpr int kVecNodes = kSB;           // nodes per vector block pass
 // Vector blocks per system are capped (they stride over the system's nodes).
 // The product's are not: 2,048 striding blocks of 8 lanes a row over 36-byte
