@@ -1450,8 +1450,8 @@ void tab_add(TabBuild& T, const AmgSys* s, const double* state) {
 }
 
 // The tables in one copy.  src keeps their host source until the caller has
-// next waited for the stream.
-int tab_upload(llfem_ctx* ctx, const TabBuild& T, void** mem, size_t* bytes, std::vector<char>* src,
+// next waited for the stream.  grow: room for the tables to double.
+int tab_upload(llfem_ctx* ctx, const TabBuild& T, bool grow, void** mem, size_t* bytes, std::vector<char>* src,
                std::vector<AmgSys::Tab>* out) {
   size_t need = 0;
   auto al = [](size_t b) { return (b + 255) / 256 * 256; };
@@ -1464,8 +1464,9 @@ int tab_upload(llfem_ctx* ctx, const TabBuild& T, void** mem, size_t* bytes, std
     if (*mem) dfree(ctx, *mem, *bytes);
     *mem = nullptr;
     *bytes = 0;
-    LLFEM_TRY(dmalloc(ctx, mem, need * 2));
-    *bytes = need * 2;
+    const size_t room = grow ? need * 2 : need;
+    LLFEM_TRY(dmalloc(ctx, mem, room));
+    *bytes = room;
   }
   out->assign(T.ents.size(), AmgSys::Tab{});
   src->resize(need);
@@ -1746,7 +1747,7 @@ int amg_sys_create(llfem_ctx* ctx, const AmgHier* h, const float* val32, float* 
   // restart tables (this system alone, always runs)
   TabBuild T;
   tab_add(T, s, nullptr);
-  rc = tab_upload(ctx, T, &s->solo_tab, &s->solo_bytes, &s->solo_src, &s->solo);
+  rc = tab_upload(ctx, T, false, &s->solo_tab, &s->solo_bytes, &s->solo_src, &s->solo);
   if (rc != LLFEM_OK) {
     amg_sys_free(ctx, s);
     return rc;
@@ -1789,7 +1790,7 @@ int amg_batch_build(llfem_ctx* ctx, const std::vector<AmgSys*>& sys, const std::
     (*b)->tab.clear();
     return LLFEM_OK;
   }
-  return tab_upload(ctx, T, &(*b)->mem, &(*b)->bytes, &(*b)->src, &(*b)->tab);
+  return tab_upload(ctx, T, true, &(*b)->mem, &(*b)->bytes, &(*b)->src, &(*b)->tab);
 }
 
 int amg_batch_apply(llfem_ctx* ctx, AmgBatch* b) {
