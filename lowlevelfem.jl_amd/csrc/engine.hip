@@ -128,7 +128,7 @@ __global__ __launch_bounds__(kRowThreads) void k_bs_spmv(const SysDev* __restric
   double* const spart = pinned(S.spart);
   const double st = gp(pinned(S.scal))[SC_STATE];
   const RowSpan rs = row_span(N, ap, lb);
-  if (st != ST_RUN) return;   // block-uniform
+  if (st != ST_RUN) return;   // no block writes it here
   const int64_t i = (int64_t)lb * 3 * kRowNodes + threadIdx.x;
   const bool own = threadIdx.x < 3 * kRowNodes && i < 3 * N;
   VT pi = 0;
@@ -173,9 +173,12 @@ __device__ __forceinline__ double sum_spart(const SysDev& S, double* sh) {
 // itself, in the same order, instead of reading alpha from a launch of one
 // block per system (4 us each for alpha and beta; eight systems on a server
 // 41.5 -> 38.8 ms); block 0 keeps the words.  A system flagged PENDING at the
-// end of the previous iteration becomes PAUSED here.  Blocks that read the
-// state before or after that, or before or after a breakdown is noted, leave
-// alike.
+// end of the previous iteration becomes PAUSED here, and one that breaks down
+// does so too, while later blocks still read the word.  So a block reads it
+// once: were every wave to read it for itself, some waves of a block could
+// leave and the others sum LDS words that those never wrote.  A block that
+// reads RUN finds the breakdown by its own sum, one that reads PAUSED leaves;
+// neither changes x or r.
 template <typename VT>
 __global__ __launch_bounds__(kSB) void k_bs_update(const SysDev* __restrict__ sys, const int32_t* __restrict__ bsys,
                                                    int nsys) {
@@ -183,8 +186,11 @@ __global__ __launch_bounds__(kSB) void k_bs_update(const SysDev* __restrict__ sy
   const SysDev& S = sys_of(sys, bsys, nsys);
   const int lb = blockIdx.x - S.vblk0;
   const bool keeper = lb == 0 && threadIdx.x == 0;
-  const double st = S.scal[SC_STATE];
-  if (st != ST_RUN) {   // block-uniform
+  __shared__ double state;
+  if (threadIdx.x == 0) state = S.scal[SC_STATE];
+  __syncthreads();
+  const double st = state;
+  if (st != ST_RUN) {
     if (keeper && st == ST_PENDING) S.scal[SC_STATE] = ST_PAUSED;
     return;
   }
@@ -252,14 +258,14 @@ __global__ __launch_bounds__(kSB) void k_bs_update(const SysDev* __restrict__ sy
 // beta = r.z / rho; p = z + beta p; reliable-update / convergence triggers.
 // The sums as in k_bs_update; block 0 writes no word that another block reads
 // but the state, which only turns from RUN to PENDING here, and both finish
-// their iteration.
+// their iteration: waves of a block that read one and the other stay together.
 template <typename VT>
 __global__ __launch_bounds__(kSB) void k_bs_pupd(const SysDev* __restrict__ sys, const int32_t* __restrict__ bsys,
                                                  int nsys) {
   __shared__ double sh[kSB / 64];
   const SysDev& S = sys_of(sys, bsys, nsys);
   const double st = S.scal[SC_STATE];
-  if (st != ST_RUN && st != ST_PENDING) return;   // block-uniform
+  if (st != ST_RUN && st != ST_PENDING) return;   // the same in every wave
   const int lb = blockIdx.x - S.vblk0;
   auto* __restrict__ pv = gp(static_cast<VT*>(S.p));
   const auto* __restrict__ zv = gp(static_cast<const VT*>(S.z));
