@@ -277,13 +277,15 @@ __global__ __launch_bounds__(64 * kBodyWaves) void k_body_any(int64_t E, int npe
 
 // f[node] = sum of the element parts over the node's incidences in ascending
 // element order (the mesh's (node, element)-sorted incidence lists), times
-// the constant force where the parts are scalars.
+// the constant force where the parts are scalars.  There the set (pos, NULL:
+// every element) is asked again: a node that no element of it touches gets 0
+// whatever the force, and an infinite one times 0 is none.
 template <bool GP>
 __global__ __launch_bounds__(256) void k_body_gather(int64_t N, int64_t E, const int32_t* __restrict__ inc_ptr,
                                                      const int32_t* __restrict__ inc_elem,
                                                      const uint8_t* __restrict__ inc_loc,
-                                                     const double* __restrict__ s, double g0, double g1, double g2,
-                                                     double* __restrict__ f) {
+                                                     const int32_t* __restrict__ pos, const double* __restrict__ s,
+                                                     double g0, double g1, double g2, double* __restrict__ f) {
   const int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (v >= N) return;
   const int32_t k1 = inc_ptr[v + 1];
@@ -296,9 +298,12 @@ __global__ __launch_bounds__(256) void k_body_gather(int64_t N, int64_t E, const
     double acc = 0.0;
 #pragma unroll 4
     for (int32_t k = inc_ptr[v]; k < k1; ++k) acc += s[(int64_t)inc_loc[k] * E + inc_elem[k]];
-    f[3 * v] = g0 * acc;
-    f[3 * v + 1] = g1 * acc;
-    f[3 * v + 2] = g2 * acc;
+    bool in = !pos;
+    if (pos)
+      for (int32_t k = inc_ptr[v]; k < k1 && !in; ++k) in = pos[inc_elem[k]] >= 0;
+    f[3 * v] = in ? g0 * acc : 0.0;
+    f[3 * v + 1] = in ? g1 * acc : 0.0;
+    f[3 * v + 2] = in ? g2 * acc : 0.0;
   }
 }
 
@@ -640,7 +645,8 @@ extern "C" int llfem_load_body(llfem_mesh* m, int32_t q, const double* weights, 
   const size_t lds = sizeof(double) * kBodyWaves * (3 * (size_t)npe + 64 * 4);
   if (g_gp) {
     k_body_any<true><<<gw, 64 * kBodyWaves, lds, st>>>(E, npe, q, m->d_xyz4, m->d_conn, d_pos, d_w, d_N, d_dN, d_gp, d_s);
-    k_body_gather<true><<<gn, 256, 0, st>>>(N, E, m->d_inc_ptr, m->d_inc_elem, m->d_inc_loc, d_s, 0.0, 0.0, 0.0, d_f);
+    k_body_gather<true><<<gn, 256, 0, st>>>(N, E, m->d_inc_ptr, m->d_inc_elem, m->d_inc_loc, d_pos, d_s, 0.0, 0.0, 0.0,
+                                            d_f);
   } else {
     // up to 10 nodes an element's coordinates and sums fit one thread's registers
     switch (npe) {
@@ -652,8 +658,8 @@ extern "C" int llfem_load_body(llfem_mesh* m, int32_t q, const double* weights, 
         k_body_any<false><<<gw, 64 * kBodyWaves, lds, st>>>(E, npe, q, m->d_xyz4, m->d_conn, d_pos, d_w, d_N, d_dN,
                                                            nullptr, d_s);
     }
-    k_body_gather<false><<<gn, 256, 0, st>>>(N, E, m->d_inc_ptr, m->d_inc_elem, m->d_inc_loc, d_s, g[0], g[1], g[2],
-                                             d_f);
+    k_body_gather<false><<<gn, 256, 0, st>>>(N, E, m->d_inc_ptr, m->d_inc_elem, m->d_inc_loc, d_pos, d_s, g[0], g[1],
+                                             g[2], d_f);
   }
   return finish_load(ctx, "llfem_load_body", d_f, N, f_out);
 }
