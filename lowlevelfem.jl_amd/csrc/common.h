@@ -304,6 +304,16 @@ struct SysSpec {
 
 struct SolveSys;
 
+// Lanes per node row of the FP64 products with the panels, by the average row:
+// 32 from 20 blocks on, 16 from 9, else 8.  Jacobi-CG, us an iteration with 8, 16
+// and 32 lanes: rows of 6 blocks 9.5, 10.2, 12.3 (12,000 nodes) and 37, 45, 80
+// (240,000); 8 blocks 9.6, 10.3, 12.2 and 41, 45, 80; 12 blocks 9.2, 9.5, 10.9
+// (8,004) and 26.2, 26.6, 30.9 (80,004); 14.7 blocks 281, 271, 349 (753,571
+// nodes); 16.3 blocks 59, 57, 68 (180,009); 20.2 blocks 53.3, 49.5, 49.8
+// (91,125); 25.7 blocks 49, 44.5, 44 (68,921); 26.4 blocks 533, 495, 517
+// (912,673); 27.7 blocks 82, 78, 77 (117,649); 61 blocks 136, 129, 132 (91,125).
+inline int panel_lanes(int64_t N, int64_t nadj) { return nadj >= 20 * N ? 32 : nadj >= 9 * N ? 16 : 8; }
+
 class BatchSolver {
  public:
   static constexpr double kDelta = 0.1;      // reliable-update trigger (residual reduction)

@@ -42,8 +42,6 @@ namespace llfem {
 namespace {
 
 constexpr int kSB = 256;                 // threads per block
-constexpr int kSG = 32;                  // lanes per node row in the FP64 product of an update (8: 1,040 us at
-                                        // 2.1 M nodes and 9.8 at 3,887, 32: 987 and 5.9)
 constexpr int kVecNodes = kSB;           // nodes per vector block pass
 // Vector blocks per system are capped (they stride over the system's nodes).
 // The product's are not: 2,048 striding blocks of 8 lanes a row over 36-byte
@@ -319,20 +317,25 @@ __global__ void k_ru_trial(int64_t n, VT* __restrict__ x, double inv_s, const do
   x[i] = (VT)0;
 }
 
-// y = mask(K64 x) (mask may be NULL)
+// y = mask(K64 x) (mask may be NULL), kG lanes a row (panel_lanes).  us with 8,
+// 16, 32 lanes: tet4 (14 to 15 blocks a row) 42,875 nodes 11.3, 11.3, 13.4 and
+// 753,571 nodes 178, 160, 231; hex8 (26) 68,921 nodes 29.6, 23.4, 24.7 and
+// 912,673 nodes 394, 341, 348; tet10 (28) 4,913 nodes 5.0, 4.5, 4.2 and 117,649
+// nodes 53.8, 42.7, 41.9; hex27 (61) 91,125 nodes 107, 85, 78.
+template <int kG>
 __global__ __launch_bounds__(kSB) void k_spmv64(int64_t N, const int64_t* __restrict__ adj_ptr,
                                                 const int32_t* __restrict__ adj, const double* __restrict__ val,
                                                 const double* __restrict__ x, const uint8_t* __restrict__ fixed,
                                                 double* __restrict__ y) {
   const int64_t gt = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t j = gt / kSG;
-  const int l = (int)(gt % kSG);
+  const int64_t j = gt / kG;
+  const int l = (int)(gt % kG);
   double a0 = 0, a1 = 0, a2 = 0;
   if (j < N) {
     const int64_t p0 = adj_ptr[j];
     const int R = (int)(adj_ptr[j + 1] - p0);
     const double* P = val + 9 * p0;
-    for (int t = l; t < R; t += kSG) {
+    for (int t = l; t < R; t += kG) {
       const int64_t i = adj[p0 + t];
       const double x0 = x[3 * i], x1 = x[3 * i + 1], x2 = x[3 * i + 2];
       a0 += P[3 * t] * x0 + P[3 * t + 1] * x1 + P[3 * t + 2] * x2;
@@ -341,10 +344,10 @@ __global__ __launch_bounds__(kSB) void k_spmv64(int64_t N, const int64_t* __rest
     }
   }
 #pragma unroll
-  for (int o = kSG / 2; o > 0; o >>= 1) {
-    a0 += __shfl_xor(a0, o, kSG);
-    a1 += __shfl_xor(a1, o, kSG);
-    a2 += __shfl_xor(a2, o, kSG);
+  for (int o = kG / 2; o > 0; o >>= 1) {
+    a0 += __shfl_xor(a0, o, kG);
+    a1 += __shfl_xor(a1, o, kG);
+    a2 += __shfl_xor(a2, o, kG);
   }
   if (j < N && l == 0) {
     const double a[3] = {a0, a1, a2};
@@ -563,6 +566,14 @@ inline int64_t vec_blocks(int64_t N) {
   return std::max<int64_t>(1, std::min<int64_t>((N + kVecNodes - 1) / kVecNodes, kMaxVecBlocks));
 }
 
+void spmv64(hipStream_t st, const SysSpec& sp, const double* x, const uint8_t* mask, double* y) {
+  const int lanes = panel_lanes(sp.N, sp.nadj);
+  const unsigned g = blocks(sp.N * lanes);
+  if (lanes == 32) k_spmv64<32><<<g, kSB, 0, st>>>(sp.N, sp.adj_ptr, sp.adj, sp.val64, x, mask, y);
+  else if (lanes == 16) k_spmv64<16><<<g, kSB, 0, st>>>(sp.N, sp.adj_ptr, sp.adj, sp.val64, x, mask, y);
+  else k_spmv64<8><<<g, kSB, 0, st>>>(sp.N, sp.adj_ptr, sp.adj, sp.val64, x, mask, y);
+}
+
 }  // namespace
 
 // ---------------------------------------------------------------------------
@@ -644,7 +655,7 @@ int BatchSolver::update_many(const std::vector<SolveSys*>& ss, bool init) {
     const SysSpec& sp = s->spec;
     const int64_t n = s->n;
     if (x) {
-      k_spmv64<<<blocks(sp.N * kSG), kSB, 0, st>>>(sp.N, sp.adj_ptr, sp.adj, sp.val64, x, sp.fixed, s->y);
+      spmv64(st, sp, x, sp.fixed, s->y);
       k_ru_resid<<<blocks(n), kSB, 0, st>>>(n, s->b, s->y, sp.fixed, s->rh, s->part);
     } else {
       k_ru_resid<<<blocks(n), kSB, 0, st>>>(n, s->b, nullptr, sp.fixed, s->rh, s->part);
@@ -818,7 +829,7 @@ int BatchSolver::add(const SysSpec& spec, SolveSys** out) {
   }
   // b = mask(f - K u_fixed); x = 0; FP32 operator and block-Jacobi inverse
   k_fill_u<<<blocks(n), kSB, 0, st>>>(n, spec.fixed, spec.ufix, nullptr, s->y);
-  k_spmv64<<<blocks(N * kSG), kSB, 0, st>>>(N, spec.adj_ptr, spec.adj, spec.val64, s->y, nullptr, s->rh);
+  spmv64(st, spec, s->y, nullptr, s->rh);
   k_ru_resid<<<blocks(n), kSB, 0, st>>>(n, spec.f, s->rh, spec.fixed, s->b, s->part);
   k_to32_blocks<<<blocks(N, 8), dim3(32, 8), 0, st>>>(N, spec.nadj, spec.adj_ptr, spec.val64, s->val32);
   k_dinv<<<blocks(N), kSB, 0, st>>>(N, spec.adj_ptr, spec.dslot, spec.val64, spec.fixed, s->dinv);
@@ -1022,7 +1033,7 @@ int BatchSolver::finish(SolveSys* s, double* u) {
   const SysSpec& sp = s->spec;
   const int64_t n = s->n;
   k_fill_u<<<blocks(n), kSB, 0, st>>>(n, sp.fixed, sp.ufix, s->xh, u);
-  k_spmv64<<<blocks(sp.N * kSG), kSB, 0, st>>>(sp.N, sp.adj_ptr, sp.adj, sp.val64, u, nullptr, s->y);
+  spmv64(st, sp, u, nullptr, s->y);
   k_ru_resid<<<blocks(n), kSB, 0, st>>>(n, sp.f, s->y, sp.fixed, nullptr, s->part);
   k_sum<<<1, kSB, 0, st>>>(blocks(n), s->part, s->scal + SC_N - 1);
   k_ru_resid<<<blocks(n), kSB, 0, st>>>(n, sp.f, nullptr, sp.fixed, nullptr, s->part);

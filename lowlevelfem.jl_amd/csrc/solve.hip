@@ -512,10 +512,9 @@ __global__ __launch_bounds__(kBS) void k_dinv_csc(int64_t n, const int64_t* __re
   dinv[j] = (fixed[j] || dv == 0.0) ? (VT)0 : (VT)(1.0 / dv);
 }
 
-// Operator views.  Lanes per row by the average row: 32 from 20 blocks (48
-// entries) on, 16 from 9 blocks (16 entries), else kG.
+// Operator views.  Lanes per row of a panel operator: panel_lanes; of a CSC one
+// by the average row, 32 from 48 entries on, 16 from 16, else kG.
 inline unsigned row_blocks(int64_t rows, int lanes) { return (unsigned)((rows * lanes + kBS - 1) / kBS); }
-inline int panel_lanes(int64_t N, int64_t nadj) { return nadj >= 20 * N ? 32 : nadj >= 9 * N ? 16 : kG; }
 inline int csc_lanes(int64_t n, int64_t nnz) { return nnz >= 48 * n ? 32 : nnz >= 16 * n ? 16 : kG; }
 
 struct PanelOp {
