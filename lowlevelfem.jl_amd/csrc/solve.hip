@@ -447,8 +447,8 @@ __global__ void k_axpy(int64_t n, double s, const double* __restrict__ d, double
 }
 
 // Scalar CSC operator (caller-supplied symmetric matrix, used as CSR of K^T),
-// G lanes per row.  A hexahedral or tetrahedral K has 60-90 entries a row:
-// 32 lanes walk it in three steps and give a small system (5,400 rows: 675
+// G lanes per row (csc_lanes).  A hexahedral or tetrahedral K has 60-90 entries a
+// row: 32 lanes walk it in three steps and give a small system (5,400 rows: 675
 // blocks instead of 169) a block on every CU.
 template <typename MT, typename VT, int G, typename X>
 __global__ __launch_bounds__(kBS) void k_spmv_csc(int64_t n, int passes, const int64_t* __restrict__ colptr,
@@ -513,9 +513,28 @@ __global__ __launch_bounds__(kBS) void k_dinv_csc(int64_t n, const int64_t* __re
 }
 
 // Operator views.  Lanes per row of a panel operator: panel_lanes; of a CSC one
-// by the average row, 32 from 48 entries on, 16 from 16, else kG.
+// by the average row and the number of rows.  More lanes shorten a row's chain
+// of loads, which a small system waits for; a large one has waves enough, and
+// what idle lanes and the longer butterfly cost is all that is left.
+// us an iteration with 8, 16 and 32 lanes (one process, in turn):
+//   below 20 entries 8: 17 entries, 5,000 rows 8.3, 8.5, 8.9, 60,000 12.9, 14.4,
+//     16.7, 500,000 47.9, 61.3, 101;
+//   20 to 48: 27-point (24) 4,913 rows 9.3, 8.7, 9.1, (26) 27,000 rows 12.1, 11.1, 12.9,
+//     216,000 33.7, 32.1, 51.3; tet4 (43) 3,993 rows 9.4, 8.2, 8.4, 73,167 18.8, 18.9,
+//     22.9; 16 up to 2^18 rows, then 8: tet4 352,947 rows 57, 64, 85, 680,943 114, 148,
+//     205, 27-point 729,000 103, 114, 171;
+//   48 to 128: tet10 (80) 3,993 rows 12.8, 10.5, 10.0, 46,875 21.0, 21.7, 21.4; band
+//     (61) 5,000 rows 10.1, 10.0, 9.2; 32 up to 2^16 rows, then 16: hex8 (77) 73,167
+//     24.2, 23.9, 27.1, 352,947 108, 106, 137, 823,875 229, 215 to 227, 303, band (61)
+//     500,000 136, 144, 168, tet10 89,373 38.0, 33.6, 32.1, 273,375 89, 95, 112;
+//   from 128: hex27 (148 to 180) 2,187 rows 16.8, 13.4, 11.3, 107,811 64, 67, 60,
+//     206,763 160, 156, 149.
 inline unsigned row_blocks(int64_t rows, int lanes) { return (unsigned)((rows * lanes + kBS - 1) / kBS); }
-inline int csc_lanes(int64_t n, int64_t nnz) { return nnz >= 48 * n ? 32 : nnz >= 16 * n ? 16 : kG; }
+inline int csc_lanes(int64_t n, int64_t nnz) {
+  if (nnz >= 128 * n) return 32;
+  if (nnz >= 48 * n) return n <= (1 << 16) ? 32 : 16;
+  return nnz >= 20 * n && n <= (1 << 18) ? 16 : kG;
+}
 
 struct PanelOp {
   static constexpr int64_t kFuseMax = 40000;   // DoFs up to which pcg forms the direction inside the SpMV
