@@ -680,9 +680,14 @@ int BatchSolver::update_many(const std::vector<SolveSys*>& ss, bool init) {
       LLFEM_HIP(hipMemcpyAsync(h + 4 * i + 2, amg_status(s->amg), sizeof(double), hipMemcpyDeviceToHost, st));
   }
   LLFEM_HIP(hipStreamSynchronize(st));
-  if (init)
+  if (init) {
+    // LLFEM_AMG_HOST_INVERSE=1 takes every coarsest inverse as left to the host
+    // (a host-side switch for testing that path)
+    const char* env = std::getenv("LLFEM_AMG_HOST_INVERSE");
+    const bool host = env && env[0] == '1';
     for (size_t i = 0; i < m; ++i)
-      if (h[4 * i + 2] != 0.0) LLFEM_TRY(amg_host_inverse(ctx_, ss[i]->amg));
+      if (ss[i]->amg && (host || h[4 * i + 2] != 0.0)) LLFEM_TRY(amg_host_inverse(ctx_, ss[i]->amg));
+  }
   // 2. adoption or rollback.  LLFEM_ENGINE_FORCE_ROLLBACK=k treats the k-th
   // update's trial as not finite (a host-side switch for testing the
   // rollback path).
