@@ -300,7 +300,8 @@ LLFEM_API int llfem_mesh_values(llfem_mesh* mesh, int32_t op, int32_t lumped, do
  * Times the panel assembly of `desc` on `sample` over a grid of launch
  * shapes (launch-width multiplier of the record planner x waves per block),
  * then, for the fastest shape, over the number of streams the node-class
- * launches of one assembly are spread over (1-3) x round kernels on/off;
+ * launches of one assembly are spread over (1-3; at most 2 in calls that copy
+ * values to the host beside the launches) x round kernels on/off;
  * keeps the fastest for the sample's element type in the context (meshes
  * created afterwards, and llfem_assemble / llfem_assemble_batch, use it) and
  * re-plans the sample.  Values do not depend on the choice.  No reference
