@@ -523,7 +523,10 @@ int assemble_impl(llfem_mesh* m, const llfem_op_desc* d, double* nzval_out, llfe
   const int blkl = (op == LLFEM_OP_STIFFNESS) ? 9 : 1;
   // Lumped mass: the sums need the geometry only, so they go first and their
   // way to the host (1.0 ms for 6.3 M DoFs) runs beside the panel launches
-  // (0.75 ms), which then keep to the side streams: 1.95 -> 1.25 ms.
+  // (0.75 ms), which then keep to the side streams: 1.95 -> 1.25 ms.  hex8, one
+  // after the other and side by side: 64 nodes 52 and 60 us, 729 61.7 and 60.4,
+  // 15,625 82 and 70, 531,441 532 and 373.  Without a target on the host they
+  // stay on st (64 nodes 39 us, on the side streams 60).
   const bool lump = op == LLFEM_OP_MASS && d->lumped;
   if (lump) {
     if (!m->d_lumped) LLFEM_TRY(dalloc(ctx, &m->d_lumped, 3 * m->N));
@@ -558,7 +561,8 @@ int assemble_impl(llfem_mesh* m, const llfem_op_desc* d, double* nzval_out, llfe
   const size_t split_bytes = size_t(affine ? 96 : 48) << 20;
   const bool split = nzval_out && !lump && !plan.empty() && sizeof(double) * (size_t)nnz >= split_bytes;
   const int parts = split ? kParts : 1;
-  const bool on_side = (lump || split) && nstreams > 0;   // the launches leave st to the copy
+  // the launches leave st to the copy, if there is one
+  const bool on_side = nzval_out && (lump || split) && nstreams > 0;
   const int first_side = on_side ? 0 : 1;   // side stream s - first_side stands for stream s; below 0: st
   // Two streams at most beside a copy, whatever was tuned or asked for: a third is
   // no faster (us with 2 and 3 side streams: tet10 in parts, affine 10,332 and
