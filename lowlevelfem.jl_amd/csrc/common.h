@@ -48,13 +48,13 @@ inline int fail(int code, const std::string& msg) {
   return code;
 }
 
-// One panel-kernel launch.  Nodes of similar incidence count are grouped
-// (padded with null steps to `cnt`), laid out in processing order as
-// per-step records so a wavefront streams `rounds` nodes per lane group.
 // A large assembly whose values go to the host is issued in kParts parts of the
 // values, so that the first part's copy runs beside the others' launches.
 constexpr int kParts = 3;
 
+// One panel-kernel launch.  Nodes of similar incidence count are grouped
+// (padded with null steps to `cnt`), laid out in processing order as
+// per-step records so a wavefront streams `rounds` nodes per lane group.
 struct PanelLaunch {
   int64_t rec_base;     // first record of the launch
   int64_t desc_base;    // first node descriptor of the launch
@@ -234,9 +234,10 @@ void drelease(llfem_ctx* ctx, T*& p, size_t count) {
 }
 
 // The context's workspace for one call: get() hands out `bytes` bytes that
-// hold anything, take() parts of them (256-byte aligned).  All work on it is
-// on the context's stream, so a later call's kernels run after this call's.
-// It is kept for the next call up to kWsKeep bytes (allocating and freeing the
+// hold anything, take() parts of them (256-byte aligned).  Work on it is on the
+// context's stream, or on the side streams of an accumulating assembly, whose
+// end (ev[3]) the stream and the call wait for: a later call's kernels run after
+// this call's.  It is kept for the next call up to kWsKeep bytes (allocating and freeing the
 // few buffers of a load vector cost it 0.8 of 3.1 ms), counts as in use, and
 // is given back when an allocation would not fit otherwise.
 constexpr size_t kWsKeep = size_t(256) << 20;

@@ -832,7 +832,7 @@ int BatchSolver::add(const SysSpec& spec, SolveSys** out) {
     release(s);
     return fail(LLFEM_EINVAL, "engine: workspace layout overflow");
   }
-  // b = mask(f - K u_fixed); x = 0; FP32 operator and block-Jacobi inverse
+  // b = mask(f - K u_fixed); x = 0; FP32 operator and inverse diagonal
   k_fill_u<<<blocks(n), kSB, 0, st>>>(n, spec.fixed, spec.ufix, nullptr, s->y);
   spmv64(st, spec, s->y, nullptr, s->rh);
   k_ru_resid<<<blocks(n), kSB, 0, st>>>(n, spec.f, s->rh, spec.fixed, s->b, s->part);

@@ -139,6 +139,10 @@ struct Plain {
 // Every block sums the previous update's partials (r.r, r.z) itself; block 0
 // keeps the scalars, tests convergence and tells the host.  Each row's owner
 // writes its part of p to a second array (neighbours still read p_old).
+// Block 0 may set S_DONE while waves of later blocks read it, so such a block
+// can lose some of its waves, and what the others then sum and write (p, y and
+// the product's partials) means nothing.  No kernel of this solve reads any of
+// it: all that follow see S_DONE set, and x is not written here.
 template <typename VT>
 struct Direction {
   const VT* __restrict__ z;
@@ -311,8 +315,9 @@ __global__ __launch_bounds__(kBS) void k_update(int64_t n, const double* __restr
 
 // beta = rz / rho, p = z + beta p; block 0 keeps the scalars, tests
 // convergence on ||r|| and tells the host (done_host: pinned memory).  A block
-// that starts after block 0 set S_DONE leaves its part of p as it was: no
-// kernel of this solve reads p any more then.
+// whose waves, some or all, read S_DONE after block 0 set it leaves its part of p
+// as it was or writes anything there: no kernel of this solve reads p any more
+// then.
 template <typename VT>
 __global__ __launch_bounds__(kBS) void k_pupd(int64_t n, double* __restrict__ scal, int64_t it, int64_t np,
                                              const double* __restrict__ part, int64_t maxiter,
