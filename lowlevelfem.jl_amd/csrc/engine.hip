@@ -92,9 +92,9 @@ __device__ __forceinline__ const SysDev& sys_of(const SysDev* sys, const int32_t
   return sys[nsys == 1 ? 0 : bsys[blockIdx.x]];
 }
 
-// Sum of q[i * stride], i < n, over the block, eight loads under way a thread:
-// one at a time, 3,165 partials took 5 us on an idle chip.
-__device__ __forceinline__ double sum_strided(const double* q, int n, int stride, double* sh) {
+// This thread's share of the sum of q[i * stride], i < n, over the block, eight
+// loads under way: one at a time, 3,165 partials took 5 us on an idle chip.
+__device__ __forceinline__ double own_strided(const double* q, int n, int stride) {
   double v = 0.0;
   for (int i0 = threadIdx.x; i0 < n; i0 += 8 * kSB) {
     double a[8];
@@ -106,7 +106,10 @@ __device__ __forceinline__ double sum_strided(const double* q, int n, int stride
 #pragma unroll
     for (int k = 0; k < 8; ++k) v += a[k];
   }
-  return bsum(v, sh);
+  return v;
+}
+__device__ __forceinline__ double sum_strided(const double* q, int n, int stride, double* sh) {
+  return bsum(own_strided(q, n, stride), sh);
 }
 
 // q = mask(K32 p) for RUNNING systems; partial p.q per block.
@@ -161,9 +164,9 @@ __global__ __launch_bounds__(kSB) void k_bs_fold(const SysDev* __restrict__ sys)
   if (threadIdx.x == 0) S.spart[S.nsblk + b] = v;
 }
 
-__device__ __forceinline__ double sum_spart(const SysDev& S, double* sh) {
+__device__ __forceinline__ double own_spart(const SysDev& S) {
   const double* q = S.spart + (S.nsblk > kFoldMax ? S.nsblk : 0);
-  return sum_strided(q, S.nsblk > kFoldMax ? kFoldBlocks : S.nsblk, 1, sh);
+  return own_strided(q, S.nsblk > kFoldMax ? kFoldBlocks : S.nsblk, 1);
 }
 
 // alpha = rho / p.q; x += alpha p; r -= alpha q; z = Dinv r; partials
@@ -172,11 +175,13 @@ __device__ __forceinline__ double sum_spart(const SysDev& S, double* sh) {
 // block per system (4 us each for alpha and beta; eight systems on a server
 // 41.5 -> 38.8 ms); block 0 keeps the words.  A system flagged PENDING at the
 // end of the previous iteration becomes PAUSED here, and one that breaks down
-// does so too, while later blocks still read the word.  So a block reads it
-// once: were every wave to read it for itself, some waves of a block could
-// leave and the others sum LDS words that those never wrote.  A block that
-// reads RUN finds the breakdown by its own sum, one that reads PAUSED leaves;
-// neither changes x or r.
+// does so too, while later blocks still read the word: waves of one block may
+// read RUN and PAUSED.  So none leaves by itself.  A wave that does not read RUN
+// puts NaN into the block's sum in place of its share, and the block leaves as
+// one where that sum is not positive: at a breakdown, which it finds by itself,
+// or because some wave saw the system paused.  (The word read by one thread and
+// handed on through LDS, with a barrier of its own, cost eight systems on a
+// server 0.8 %.)
 template <typename VT>
 __global__ __launch_bounds__(kSB) void k_bs_update(const SysDev* __restrict__ sys, const int32_t* __restrict__ bsys,
                                                    int nsys) {
@@ -184,14 +189,8 @@ __global__ __launch_bounds__(kSB) void k_bs_update(const SysDev* __restrict__ sy
   const SysDev& S = sys_of(sys, bsys, nsys);
   const int lb = blockIdx.x - S.vblk0;
   const bool keeper = lb == 0 && threadIdx.x == 0;
-  __shared__ double state;
-  if (threadIdx.x == 0) state = S.scal[SC_STATE];
-  __syncthreads();
-  const double st = state;
-  if (st != ST_RUN) {
-    if (keeper && st == ST_PENDING) S.scal[SC_STATE] = ST_PAUSED;
-    return;
-  }
+  const double st = S.scal[SC_STATE];
+  const bool run = st == ST_RUN;   // of this wave
   auto* __restrict__ xv = gp(static_cast<VT*>(S.x));
   auto* __restrict__ rv = gp(static_cast<VT*>(S.r));
   auto* __restrict__ zv = gp(static_cast<VT*>(S.z));
@@ -210,10 +209,10 @@ __global__ __launch_bounds__(kSB) void k_bs_update(const SysDev* __restrict__ sy
         q[c] = qv[3 * j + c];
       }
   };
-  load();
-  const double rho = S.scal[SC_RHO], pq = sum_spart(S, sh);
-  if (!(pq > 0.0)) {   // breakdown (p = 0 or K not SPD on the free set): check the true residual
-    if (keeper) S.scal[SC_STATE] = ST_PAUSED;
+  if (run) load();
+  const double rho = S.scal[SC_RHO], pq = bsum(run ? own_spart(S) : (double)NAN, sh);
+  if (!(pq > 0.0)) {   // paused, or a breakdown (p = 0 or K not SPD on the free set): check the true residual
+    if (keeper && (run || st == ST_PENDING)) S.scal[SC_STATE] = ST_PAUSED;
     return;
   }
   if (keeper) S.scal[SC_RHOP] = rho;
@@ -279,7 +278,7 @@ __global__ __launch_bounds__(kSB) void k_bs_pupd(const SysDev* __restrict__ sys,
   };
   load();
   const double rho = S.scal[SC_RHOP];
-  const double rz = S.amg ? sum_spart(S, sh) : sum_strided(S.part + 1, S.nvblk, 2, sh);
+  const double rz = S.amg ? bsum(own_spart(S), sh) : sum_strided(S.part + 1, S.nvblk, 2, sh);
   if (lb == 0) {
     const double rr = sum_strided(S.part, S.nvblk, 2, sh);
     if (threadIdx.x == 0) {
